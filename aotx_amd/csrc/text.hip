@@ -5,15 +5,20 @@
  * right) that holds the merge rank and the merged token (so the merge step never joins
  * strings), the token of each single byte, and the control bits.
  *
- * Encoding is three launches:
- *   - pre-tokens: one thread per text runs the family's split pattern, a state machine
- *     that takes the first alternative matching at a position (cuda/text/pretok.cu:1-45);
- *   - merge: one 64-lane workgroup per pre-token (a work list the pre-token pass appends
- *     to) holds its symbols in LDS as a linked list
- *     with the rank of each symbol's pair; each round a wave minimum over (rank, position)
- *     picks the pair to merge (the lowest rank, the leftmost of equal ranks), and only
- *     the two pairs next to it are looked up again;
- *   - gather: one wave per text copies its pre-tokens' tokens in order.
+ * Encoding is five launches, six with special tokens; each works on many places of a text
+ * at a time:
+ *   - clean: a workgroup per text, four bytes per thread, replaces what is not UTF-8;
+ *   - special tokens (when the vocabulary has any): a wave per text lists their places;
+ *   - pre-tokens: one thread per byte. The family's split pattern is a state machine that
+ *     takes the first alternative matching at a position (cuda/text/pretok.cu:1-45); a
+ *     thread at a place where every match must begin anew (is_sync) runs it up to the next
+ *     such place, so a text is cut in parallel;
+ *   - merge: a wave per 64 bytes, one lane per pre-token that starts there: its symbols and
+ *     the rank of each symbol's pair in LDS, each round the pair of the lowest rank (the
+ *     leftmost of equal ranks), and only the two pairs next to it looked up again;
+ *   - pre-tokens of more than TX_SHORT bytes: a workgroup of 64 lanes each, the same rounds
+ *     with a wave minimum;
+ *   - gather: a workgroup per text, a prefix sum over the tokens of each place.
  * Detokenizing is one wave per text: token lengths, a wave prefix sum, then the bytes.
  */
 #include "aotx_internal.h"
@@ -135,9 +140,7 @@ struct aotx_text_vocab {
     unsigned int slots;                 /* power of two */
     const unsigned int *slot;           /* token of each slot, or AOTX_TEXT_NONE */
     unsigned int pairs;                 /* power of two */
-    const unsigned long long *pair_key; /* left << 32 | right, or all ones */
-    const unsigned int *pair_rank;
-    const unsigned int *pair_result;
+    const uint4 *pair;                  /* right, left (all ones: empty), rank, merged token */
     const unsigned int *control;        /* one bit per token */
     const unsigned int *special;        /* tokens of the control and user types */
     unsigned int specials;
@@ -151,17 +154,38 @@ static aotx_text_vocab g_vocab;
 static int g_ready = 0;
 static unsigned int g_report[4];
 
+/* The merge rank (and merged token) of two symbol pairs, AOTX_TEXT_NONE for no merge. Both
+ * probes are in flight together: a lookup is one 16-byte load unless its place was taken. */
+static __device__ __forceinline__ void find_pairs(const aotx_text_vocab &v, unsigned int l0, unsigned int r0,
+                                                  unsigned int l1, unsigned int r1, unsigned int rank[2],
+                                                  unsigned int res[2])
+{
+    const unsigned int mask = v.pairs - 1u;
+    unsigned int at0 = (unsigned int)pair_mix(((unsigned long long)l0 << 32) | r0) & mask;
+    unsigned int at1 = (unsigned int)pair_mix(((unsigned long long)l1 << 32) | r1) & mask;
+    bool on0 = l0 != AOTX_TEXT_NONE && r0 != AOTX_TEXT_NONE, on1 = l1 != AOTX_TEXT_NONE && r1 != AOTX_TEXT_NONE;
+    rank[0] = rank[1] = AOTX_TEXT_NONE;
+    res[0] = res[1] = 0u;
+    for (unsigned int i = 0u; i <= mask && (on0 || on1); ++i) {
+        const uint4 e0 = v.pair[at0], e1 = v.pair[at1];
+        if (on0 && e0.x == r0 && e0.y == l0) { rank[0] = e0.z; res[0] = e0.w; on0 = false; }
+        if (on1 && e1.x == r1 && e1.y == l1) { rank[1] = e1.z; res[1] = e1.w; on1 = false; }
+        on0 = on0 && !(e0.x == AOTX_TEXT_NONE && e0.y == AOTX_TEXT_NONE);
+        on1 = on1 && !(e1.x == AOTX_TEXT_NONE && e1.y == AOTX_TEXT_NONE);
+        at0 = (at0 + 1u) & mask;
+        at1 = (at1 + 1u) & mask;
+    }
+}
 static __device__ __forceinline__ unsigned int find_pair(const aotx_text_vocab &v, unsigned int l,
                                                          unsigned int r, unsigned int *result)
 {
     if (l == AOTX_TEXT_NONE || r == AOTX_TEXT_NONE) return AOTX_TEXT_NONE;
-    const unsigned long long key = ((unsigned long long)l << 32) | r;
     const unsigned int mask = v.pairs - 1u;
-    unsigned int at = (unsigned int)pair_mix(key) & mask;
+    unsigned int at = (unsigned int)pair_mix(((unsigned long long)l << 32) | r) & mask;
     for (unsigned int i = 0; i <= mask; ++i) {
-        const unsigned long long got = v.pair_key[at];
-        if (got == ~0ull) return AOTX_TEXT_NONE;
-        if (got == key) { *result = v.pair_result[at]; return v.pair_rank[at]; }
+        const uint4 e = v.pair[at];
+        if (e.x == r && e.y == l) { *result = e.w; return e.z; }
+        if (e.x == AOTX_TEXT_NONE && e.y == AOTX_TEXT_NONE) return AOTX_TEXT_NONE;
         at = (at + 1u) & mask;
     }
     return AOTX_TEXT_NONE;
@@ -309,34 +333,99 @@ static __device__ unsigned int match(unsigned int pattern, const unsigned char *
     return spaces(b, end, at, span, 1);
 }
 
-/* one thread per text: the text with every byte that does not start a UTF-8 character
- * (and the bytes of a cut or malformed one) written as U+FFFD, EF BF BD (cuda/text/
- * text.cuh:367-374); text t goes to out + 3 at[t], its length to clean_len[t] */
-__global__ void aotx_text_clean_kernel(const unsigned char *bytes, const unsigned long long *at,
-                                       unsigned int texts, unsigned char *out,
-                                       unsigned long long *at3, unsigned int *clean_len)
+/* The sum of `mine` over the threads before this one of a workgroup of 1024, and over all of
+ * them in *total. `part` is 16 words of LDS; ends with every thread past its reads. */
+static __device__ __forceinline__ unsigned int block_before(unsigned int mine, unsigned int *part,
+                                                            unsigned int *total)
 {
-    const unsigned int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t > texts) return;
-    at3[t] = 3ull * at[t];
-    if (t == texts) return;
+    const unsigned int lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    unsigned int incl = mine;
+#pragma unroll
+    for (unsigned int d = 1u; d < 64u; d <<= 1) {
+        const unsigned int o = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += o;
+    }
+    if (lane == 63u) part[wave] = incl;
+    __syncthreads();
+    unsigned int before = 0u, all = 0u;
+#pragma unroll
+    for (unsigned int w = 0u; w < 16u; ++w) {
+        const unsigned int n = part[w];
+        before += w < wave ? n : 0u;
+        all += n;
+    }
+    __syncthreads();
+    *total = all;
+    return before + incl - mine;
+}
+
+/* Whether a character starts at `at`, reading forward from `from`: every byte but those that
+ * a whole character before it holds. A lead byte is never inside another character, so the
+ * bytes up to the nearest lead decide it. */
+static __device__ bool char_starts(const unsigned char *b, unsigned int from, unsigned int end, unsigned int at)
+{
+    if ((b[at] & 0xC0u) != 0x80u) return true;
+    for (unsigned int j = 1u; j <= 3u && at >= from + j; ++j) {
+        if ((b[at - j] & 0xC0u) == 0x80u) continue;
+        unsigned int p;
+        return utf8_at(b, end, at - j, &p) <= j;
+    }
+    return true;
+}
+
+/* A workgroup per text, four bytes per thread: the text with every byte that does not start a
+ * UTF-8 character (and the bytes of a cut or malformed one) written as U+FFFD, EF BF BD
+ * (cuda/text/text.cuh:367-374); text t goes to out + 3 at[t], its length to clean_len[t], and
+ * the marks of its places (mark, the pre-token pass's) are cleared. Each byte decides by
+ * itself whether it is kept (one byte) or replaced (three), and a prefix sum places it. Bound
+ * by the latency of its byte loads; 64 texts of 4000 bytes 2765 -> 14.5 us against one thread
+ * per text. */
+__global__ __launch_bounds__(1024) void aotx_text_clean_kernel(const unsigned char *bytes,
+                                                               const unsigned long long *at,
+                                                               unsigned char *out, unsigned char *mark,
+                                                               unsigned int *clean_len, unsigned int *longs)
+{
+    __shared__ unsigned int part[16];
+    const unsigned int t = blockIdx.x;
     const unsigned char *b = bytes + at[t];
     const unsigned int end = (unsigned int)(at[t + 1u] - at[t]);
-    unsigned char *o = out + 3ull * at[t];
-    unsigned int w = 0u;
-    for (unsigned int pos = 0u; pos < end;) {
-        unsigned int p;
-        const unsigned int k = utf8_at(b, end, pos, &p);
-        if (p == 0xFFFDu && k == 1u) {        /* no character starts here */
-            o[w] = 0xEFu; o[w + 1u] = 0xBFu; o[w + 2u] = 0xBDu;
-            w += 3u;
-        } else {
-            for (unsigned int i = 0u; i < k; ++i) o[w + i] = b[pos + i];
-            w += k;
+    unsigned char *o = out + 3ull * at[t], *m = mark + 3ull * at[t];
+    if (t == 0u && threadIdx.x == 0u) *longs = 0u;
+    unsigned int done = 0u;
+    for (unsigned int tile = 0u; tile < end; tile += 4096u) {
+        const unsigned int i0 = tile + 4u * threadIdx.x;
+        unsigned int bad = 0u, n = 0u;
+#pragma unroll
+        for (unsigned int j = 0u; j < 4u; ++j) {
+            const unsigned int i = i0 + j;
+            if (i >= end) continue;
+            bool replace = false;
+            if (b[i] >= 0x80u && char_starts(b, 0u, end, i)) {
+                unsigned int p;
+                replace = utf8_at(b, end, i, &p) == 1u;
+            }
+            bad |= replace ? 1u << j : 0u;
+            n += replace ? 3u : 1u;
         }
-        pos += k;
+        unsigned int total;
+        unsigned int w = done + block_before(n, part, &total);
+#pragma unroll
+        for (unsigned int j = 0u; j < 4u; ++j) {
+            const unsigned int i = i0 + j;
+            if (i >= end) continue;
+            if ((bad >> j) & 1u) {
+                o[w] = 0xEFu; o[w + 1u] = 0xBFu; o[w + 2u] = 0xBDu;
+                m[w] = 0u; m[w + 1u] = 0u; m[w + 2u] = 0u;
+                w += 3u;
+            } else {
+                o[w] = b[i];
+                m[w] = 0u;
+                w += 1u;
+            }
+        }
+        done += total;
     }
-    clean_len[t] = w;
+    if (threadIdx.x == 0u) clean_len[t] = done;
 }
 
 /* The longest special token whose bytes start at `at` (cuda/text/pretok.cu:339-372): its
@@ -359,170 +448,356 @@ static __device__ unsigned int special_at(const aotx_text_vocab &v, const unsign
     return best;
 }
 
-/* one thread per text: pre-token p of text t is (start[at[t] + p], len[at[t] + p]), and
- * tok[at[t] + p] its token when it is a special token (else AOTX_TEXT_NONE). A special
- * token is a whole match and the pattern reads no text across it. */
-__global__ void aotx_text_pretok_kernel(aotx_text_vocab v, const unsigned char *bytes,
-                                        const unsigned long long *at, const unsigned int *clean_len,
-                                        unsigned int texts, unsigned int *start, unsigned int *len,
-                                        unsigned int *tok, unsigned int *pieces, unsigned int *work,
-                                        unsigned int *works)
+#define TX_MARK_START   1u     /* a pre-token starts here */
+#define TX_MARK_SPECIAL 2u     /* a special token starts here */
+
+/* One wave per text: the places of its special tokens, in order: the leftmost first, the
+ * longest there, then from its end on. The i-th of text t starts at sat[3 at[t] + i] and ends
+ * at send[3 at[t] + i]; scount[t] counts them. */
+__global__ __launch_bounds__(64) void aotx_text_special_kernel(aotx_text_vocab v, const unsigned char *bytes,
+                                                               const unsigned long long *at,
+                                                               const unsigned int *clean_len, unsigned char *mark,
+                                                               unsigned int *sat, unsigned int *send,
+                                                               unsigned int *scount)
 {
-    const unsigned int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= texts) return;
-    const unsigned long long base = at[t];
+    const unsigned int t = blockIdx.x, lane = threadIdx.x;
+    const unsigned long long base = 3ull * at[t];
     const unsigned char *b = bytes + base;
-    const unsigned int text_end = clean_len[t];
+    const unsigned int end = clean_len[t];
     unsigned int pos = 0u, n = 0u;
-    while (pos < text_end) {
-        unsigned int stop = pos, special = 0u, id = AOTX_TEXT_NONE;
-        while (stop < text_end && v.specials != 0u) {
-            special = special_at(v, b, stop, text_end, &id);
-            if (special != 0u) break;
-            stop += 1u;
+    for (unsigned int tile = 0u; tile < end; tile += 512u) {
+        unsigned int c[8];
+#pragma unroll
+        for (unsigned int j = 0u; j < 8u; ++j) {
+            const unsigned int i = tile + 64u * j + lane;
+            c[j] = b[i < end ? i : tile];
         }
-        if (v.specials == 0u) stop = text_end;
-        const unsigned int end = stop;
-        while (pos < end) {
-        unsigned int m = match(v.pattern, b, pos, end);
-        if (m == 0u) m = 1u;
-        if (m > AOTX_TEXT_CHUNK_BYTES) {          /* cut at a character boundary */
-            unsigned int cut = 0u;
-            while (cut < end - pos) {
-                unsigned int p;
-                const unsigned int k = utf8_at(b, end, pos + cut, &p);
-                if (cut + k > AOTX_TEXT_CHUNK_BYTES) break;
-                cut += k;
+#pragma unroll
+        for (unsigned int j = 0u; j < 8u; ++j) {
+            const unsigned int i = tile + 64u * j + lane;
+            const bool maybe = i < end && ((v.first[c[j] >> 6] >> (c[j] & 63u)) & 1ull) != 0ull;
+            if (!__any(maybe)) continue;
+            unsigned int id = 0u;
+            const unsigned int span = maybe ? special_at(v, b, i, end, &id) : 0u;
+            unsigned long long found = __ballot(span != 0u);
+            while (found != 0ull) {
+                const unsigned int l = (unsigned int)__builtin_ctzll(found);
+                found &= found - 1ull;
+                const unsigned int p = tile + 64u * j + l, k = (unsigned int)__shfl((int)span, (int)l, 64);
+                if (p < pos) continue;                   /* inside the one before */
+                if (lane == 0u) {
+                    mark[base + p] = TX_MARK_SPECIAL;
+                    sat[base + n] = p;
+                    send[base + n] = p + k;
+                }
+                n += 1u;
+                pos = p + k;
             }
-            m = cut;
-        }
-        start[base + n] = pos;
-        len[base + n] = m;
-        tok[base + n] = AOTX_TEXT_NONE;
-        n += 1u;
-        pos += m;
-        }
-        if (special != 0u) {
-            start[base + n] = stop;
-            len[base + n] = special;
-            tok[base + n] = id;
-            n += 1u;
-            pos = stop + special;
         }
     }
-    pieces[t] = n;
-    /* the merge step takes one workgroup per pre-token of the batch, from this list */
-    const unsigned int first = atomicAdd(works, n);
-    for (unsigned int i = 0u; i < n; ++i) work[first + i] = (unsigned int)(base + i);
+    if (lane == 0u) scount[t] = n;
 }
 
-/* ---- merge: one 64-lane workgroup per pre-token slot ----------------------------------- */
+/* Whether every way of cutting the text up to `at` has a cut at `at`, a place where a
+ * character starts in the run [from, end): its start; or a letter (or, with the family's
+ * marks, a mark) or a number before it and no such character at it. A pre-token that holds a
+ * letter is a run of letters or a contraction, and one that holds a number is a run of
+ * numbers; both end where the run ends (one that is cut at AOTX_TEXT_CHUNK_BYTES ends
+ * earlier, and the rest is matched again). */
+static __device__ bool is_sync(unsigned int pattern, const unsigned char *b, unsigned int from,
+                               unsigned int end, unsigned int at)
+{
+    if (at == from) return true;
+    unsigned int before = 0xFFFDu, here, k = at - 1u;
+    while (k > from && at - k < 4u && (b[k] & 0xC0u) == 0x80u) k -= 1u;
+    unsigned int p;
+    if (utf8_at(b, end, k, &p) == at - k) before = p;
+    const int marks = pattern == AOTX_TEXT_PATTERN_QWEN35;
+    const bool letter = is_letter(before) || (marks && is_mark(before));
+    if (!letter && !is_number(before)) return false;
+    utf8_at(b, end, at, &here);
+    return letter ? !(is_letter(here) || (marks && is_mark(here))) : !is_number(here);
+}
+
+/* One thread per byte of the cleaned texts (chunks workgroups of 256 per text, each taking
+ * every chunks-th tile): a thread at a place of is_sync runs the pattern from there to the
+ * next such place, mostly one or two pre-tokens, and marks each start. A text without letters
+ * or numbers is one thread's, as every text was before. Bound by the chain of byte loads of a
+ * word: 64 texts of 4000 bytes 6812 -> 45 us. */
+__global__ __launch_bounds__(256) void aotx_text_pretok_kernel(aotx_text_vocab v, const unsigned char *bytes,
+                                                               const unsigned long long *at,
+                                                               const unsigned int *clean_len, unsigned int chunks,
+                                                               const unsigned int *sat, const unsigned int *send,
+                                                               const unsigned int *scount, unsigned char *mark)
+{
+    const unsigned int t = blockIdx.x / chunks;
+    const unsigned long long base = 3ull * at[t];
+    const unsigned char *b = bytes + base;
+    const unsigned int text_end = clean_len[t];
+    for (unsigned int tile = (blockIdx.x % chunks) * 256u; tile < text_end; tile += chunks * 256u) {
+        unsigned int pos = tile + threadIdx.x;
+        if (pos >= text_end) return;
+        unsigned int from = 0u, end = text_end;
+        if (v.specials != 0u) {
+            /* the run between special tokens that holds pos: after the last one at or before it */
+            unsigned int lo = 0u, hi = scount[t];
+            while (lo < hi) {
+                const unsigned int mid = (lo + hi) >> 1;
+                if (sat[base + mid] <= pos) lo = mid + 1u; else hi = mid;
+            }
+            if (lo > 0u) from = send[base + lo - 1u];
+            if (lo < scount[t]) end = sat[base + lo];
+            if (pos < from) continue;                    /* inside a special token */
+        }
+        if (!char_starts(b, from, end, pos) || !is_sync(v.pattern, b, from, end, pos)) continue;
+        do {
+            unsigned int m = match(v.pattern, b, pos, end);
+            if (m == 0u) m = 1u;
+            if (m > AOTX_TEXT_CHUNK_BYTES) {          /* cut at a character boundary */
+                unsigned int cut = 0u;
+                while (cut < end - pos) {
+                    unsigned int p;
+                    const unsigned int k = utf8_at(b, end, pos + cut, &p);
+                    if (cut + k > AOTX_TEXT_CHUNK_BYTES) break;
+                    cut += k;
+                }
+                m = cut;
+            }
+            mark[base + pos] = TX_MARK_START;
+            pos += m;
+        } while (pos < end && !is_sync(v.pattern, b, from, end, pos));
+    }
+}
+
+/* ---- merge -------------------------------------------------------------------------------- */
 
 #define TX_N AOTX_TEXT_CHUNK_BYTES
+#define TX_SHORT 32u           /* bytes of the pre-tokens that one lane merges */
+#define TX_WAVES 4u
 
-__global__ __launch_bounds__(64) void aotx_text_merge_kernel(aotx_text_vocab v, const unsigned char *bytes,
-                                                             const unsigned long long *at, unsigned int texts,
-                                                             const unsigned int *start, const unsigned int *len,
-                                                             const unsigned int *ptok,
-                                                             const unsigned int *pieces, const unsigned int *work,
-                                                             unsigned int *out, unsigned int *out_count)
+/* A wave per 64 places of a cleaned text. The lane at a pre-token's first byte owns it; the
+ * tokens go where its bytes are (never more than those), their number to count[place], which
+ * is 0 at every other place. The pairs of neighbouring bytes are looked up by all lanes at
+ * once; then every lane merges its own pre-token in its bytes' places of LDS. Most pre-tokens
+ * hold a few bytes, so a wave of lanes with one each is busier than a wave for each, and needs
+ * 6 KB of LDS instead of 64 (64 texts of 4000 bytes 370 -> 37 us, bound by the chain of table
+ * lookups). Longer ones are left to aotx_text_long_kernel, in a list of (text, place,
+ * bytes). */
+__global__ __launch_bounds__(64 * TX_WAVES) void aotx_text_merge_kernel(aotx_text_vocab v, const unsigned char *bytes,
+                                                                        const unsigned long long *at,
+                                                                        const unsigned int *clean_len,
+                                                                        const unsigned char *mark, unsigned int chunks,
+                                                                        unsigned int *out, unsigned short *count,
+                                                                        unsigned int *long_list, unsigned int *longs)
+{
+    __shared__ unsigned int tokl[TX_WAVES][64 + TX_SHORT], rankl[TX_WAVES][64 + TX_SHORT], resl[TX_WAVES][64 + TX_SHORT];
+    __shared__ unsigned char nxtl[TX_WAVES][64 + TX_SHORT], prvl[TX_WAVES][64 + TX_SHORT];
+    const unsigned int lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    unsigned int *tok = tokl[wave], *rank = rankl[wave], *res = resl[wave];
+    unsigned char *nxt = nxtl[wave], *prv = prvl[wave];
+    const unsigned int t = blockIdx.x / chunks;
+    const unsigned long long base = 3ull * at[t];
+    const unsigned char *b = bytes + base;
+    const unsigned int end = clean_len[t];
+    for (unsigned int w = ((blockIdx.x % chunks) * TX_WAVES + wave) * 64u; w < end; w += chunks * TX_WAVES * 64u) {
+        const unsigned int p = w + lane;
+        const unsigned int kind = p < end ? mark[base + p] : 0u;
+        const unsigned long long starts = __ballot(kind != 0u);
+        if (p < end) count[base + p] = 0u;
+        if (starts == 0ull) continue;                    /* inside a longer one */
+        /* the end of the last pre-token that starts here */
+        unsigned int after = w + 64u;
+        for (; after < end; after += 64u) {
+            const unsigned int q = after + lane;
+            const unsigned long long more = __ballot(q < end && mark[base + (q < end ? q : after)] != 0u);
+            if (more != 0ull) {
+                after += (unsigned int)__builtin_ctzll(more);
+                break;
+            }
+        }
+        if (after > end) after = end;
+        const unsigned long long later = lane == 63u ? 0ull : starts >> (lane + 1u);
+        const unsigned int n = later != 0ull ? 1u + (unsigned int)__builtin_ctzll(later) : after - p;
+        unsigned int *dst = out + base + p;
+        bool open = kind != 0u;
+        if (kind == TX_MARK_SPECIAL) {
+            unsigned int id = AOTX_TEXT_NONE;
+            special_at(v, b, p, end, &id);
+            dst[0] = id;
+            count[base + p] = 1u;
+            open = false;
+        } else if (open && v.whole) {
+            const unsigned int whole = find_bytes(v, b + p, n);
+            if (whole != AOTX_TEXT_NONE) {
+                dst[0] = whole;
+                count[base + p] = 1u;
+                open = false;
+            }
+        }
+        if (open && n > TX_SHORT) {
+            unsigned int *item = long_list + 3ull * atomicAdd(longs, 1u);
+            item[0] = t;
+            item[1] = p;
+            item[2] = n;
+            open = false;
+        }
+        const unsigned long long mine = __ballot(open);
+        if (mine == 0ull) continue;
+        /* every byte's token and its pair with the next, the last pre-token's bytes past the
+         * window in a second round */
+#pragma unroll
+        for (unsigned int round = 0u; round < 2u; ++round) {
+            const unsigned int i = round * 64u + lane;
+            const unsigned long long upto = round != 0u ? starts : starts & (~0ull >> (63u - lane));
+            const unsigned int own = upto != 0ull ? 63u - (unsigned int)__builtin_clzll(upto) : 64u;
+            const unsigned int size = (unsigned int)__shfl((int)n, (int)(own & 63u), 64);
+            if (i < 64u + TX_SHORT && own < 64u && ((mine >> own) & 1ull) != 0ull && i < own + size) {
+                const unsigned int x = v.byte_token[b[w + i]];
+                unsigned int r = 0u, k = AOTX_TEXT_NONE;
+                if (i + 1u < own + size) k = find_pair(v, x, v.byte_token[b[w + i + 1u]], &r);
+                tok[i] = x;
+                rank[i] = k;
+                res[i] = r;
+                nxt[i] = (unsigned char)(i + 1u);
+                prv[i] = i == own ? 0xFFu : (unsigned char)(i - 1u);
+            }
+        }
+        /* the wave's writes before its lanes' reads of one another's places */
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (open) {
+            const unsigned int last = lane + n;
+            for (;;) {
+                unsigned int best = AOTX_TEXT_NONE, i = lane;
+                for (unsigned int q = lane; q < last; ++q) {
+                    const unsigned int k = rank[q];
+                    if (k < best) { best = k; i = q; }
+                }
+                if (best == AOTX_TEXT_NONE) break;
+                const unsigned int j = nxt[i], k = nxt[j], f = prv[i], x = res[i];
+                unsigned int ranks[2], made[2];
+                find_pairs(v, x, k < last ? tok[k] : AOTX_TEXT_NONE, f != 0xFFu ? tok[f] : AOTX_TEXT_NONE, x, ranks,
+                           made);
+                tok[i] = x;
+                nxt[i] = (unsigned char)k;
+                if (k < last) prv[k] = (unsigned char)i;
+                rank[j] = AOTX_TEXT_NONE;
+                rank[i] = ranks[0];
+                res[i] = made[0];
+                if (f != 0xFFu) {
+                    rank[f] = ranks[1];
+                    res[f] = made[1];
+                }
+            }
+            unsigned int c = 0u;
+            for (unsigned int i = lane; i < last; i = nxt[i]) dst[c++] = tok[i];
+            count[base + p] = (unsigned short)c;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+/* The pre-tokens of more than TX_SHORT bytes, a workgroup each (a fixed grid goes through the
+ * list that the merge left). */
+__global__ __launch_bounds__(64) void aotx_text_long_kernel(aotx_text_vocab v, const unsigned char *bytes,
+                                                            const unsigned long long *at,
+                                                            const unsigned int *long_list, const unsigned int *longs,
+                                                            unsigned int *out, unsigned short *count)
 {
     __shared__ unsigned int tok[TX_N], rank[TX_N], res[TX_N];
     __shared__ unsigned short nxt[TX_N], prv[TX_N];
     const unsigned int lane = threadIdx.x;
-    const unsigned long long s = work[blockIdx.x];
-    /* the text of slot s: at[t] <= s < at[t + 1] */
-    unsigned int lo = 0u, hi = texts;
-    while (hi - lo > 1u) {
-        const unsigned int mid = (lo + hi) >> 1;
-        if (at[mid] <= s) lo = mid; else hi = mid;
-    }
-    const unsigned int t = lo;
-    if (s - at[t] >= pieces[t]) return;
-    const unsigned char *b = bytes + at[t] + start[s];
-    const unsigned int n = len[s];
-    /* a pre-token's tokens (never more than its bytes) go where its bytes are */
-    unsigned int *dst = out + at[t] + start[s];
-    if (ptok[s] != AOTX_TEXT_NONE) {
-        if (lane == 0u) { dst[0] = ptok[s]; out_count[s] = 1u; }
-        return;
-    }
-    if (v.whole) {
-        const unsigned int w = lane == 0u ? find_bytes(v, b, n) : 0u;
-        const unsigned int whole = __shfl(w, 0, 64);
-        if (whole != AOTX_TEXT_NONE) {
-            if (lane == 0u) { dst[0] = whole; out_count[s] = 1u; }
-            return;
-        }
-    }
-    for (unsigned int i = lane; i < n; i += 64u) {
-        tok[i] = v.byte_token[b[i]];
-        nxt[i] = (unsigned short)(i + 1u);
-        prv[i] = (unsigned short)(i == 0u ? 0xFFFFu : i - 1u);
-    }
-    __syncthreads();
-    for (unsigned int i = lane; i < n; i += 64u) {
-        unsigned int r = 0u;
-        rank[i] = i + 1u < n ? find_pair(v, tok[i], tok[i + 1u], &r) : AOTX_TEXT_NONE;
-        res[i] = r;
-    }
-    __syncthreads();
-    for (;;) {
-        unsigned long long best = ~0ull;
+    const unsigned int items = *longs;
+    for (unsigned int item = blockIdx.x; item < items; item += gridDim.x) {
+        const unsigned long long place = 3ull * at[long_list[3ull * item]] + long_list[3ull * item + 1u];
+        const unsigned int n = long_list[3ull * item + 2u];
+        const unsigned char *b = bytes + place;
+        unsigned int *dst = out + place;
+        __syncthreads();                      /* the item before is read */
         for (unsigned int i = lane; i < n; i += 64u) {
-            const unsigned long long k = ((unsigned long long)rank[i] << 32) | i;
-            best = k < best ? k : best;
-        }
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            const unsigned long long o = __shfl_xor(best, d, 64);
-            best = o < best ? o : best;
-        }
-        if ((unsigned int)(best >> 32) == AOTX_TEXT_NONE) break;
-        if (lane == 0u) {
-            const unsigned int i = (unsigned int)best, j = nxt[i];
-            tok[i] = res[i];
-            const unsigned int k = nxt[j];
-            nxt[i] = (unsigned short)k;
-            if (k < n) prv[k] = (unsigned short)i;
-            rank[j] = AOTX_TEXT_NONE;
-            unsigned int r = 0u;
-            rank[i] = k < n ? find_pair(v, tok[i], tok[k], &r) : AOTX_TEXT_NONE;
-            res[i] = r;
-            const unsigned int p = prv[i];
-            if (p != 0xFFFFu) {
-                unsigned int r2 = 0u;
-                rank[p] = find_pair(v, tok[p], tok[i], &r2);
-                res[p] = r2;
-            }
+            tok[i] = v.byte_token[b[i]];
+            nxt[i] = (unsigned short)(i + 1u);
+            prv[i] = (unsigned short)(i == 0u ? 0xFFFFu : i - 1u);
         }
         __syncthreads();
-    }
-    if (lane == 0u) {
-        unsigned int c = 0u;
-        for (unsigned int i = 0u; i < n; i = nxt[i]) dst[c++] = tok[i];
-        out_count[s] = c;
+        for (unsigned int i = lane; i < n; i += 64u) {
+            unsigned int r = 0u;
+            rank[i] = i + 1u < n ? find_pair(v, tok[i], tok[i + 1u], &r) : AOTX_TEXT_NONE;
+            res[i] = r;
+        }
+        __syncthreads();
+        for (;;) {
+            unsigned long long best = ~0ull;
+            for (unsigned int i = lane; i < n; i += 64u) {
+                const unsigned long long k = ((unsigned long long)rank[i] << 32) | i;
+                best = k < best ? k : best;
+            }
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) {
+                const unsigned long long o = __shfl_xor(best, d, 64);
+                best = o < best ? o : best;
+            }
+            if ((unsigned int)(best >> 32) == AOTX_TEXT_NONE) break;
+            __syncthreads();
+            if (lane == 0u) {
+                const unsigned int i = (unsigned int)best, j = nxt[i], k = nxt[j], f = prv[i], x = res[i];
+                unsigned int ranks[2], made[2];
+                find_pairs(v, x, k < n ? tok[k] : AOTX_TEXT_NONE, f != 0xFFFFu ? tok[f] : AOTX_TEXT_NONE, x, ranks, made);
+                tok[i] = x;
+                nxt[i] = (unsigned short)k;
+                if (k < n) prv[k] = (unsigned short)i;
+                rank[j] = AOTX_TEXT_NONE;
+                rank[i] = ranks[0];
+                res[i] = made[0];
+                if (f != 0xFFFFu) {
+                    rank[f] = ranks[1];
+                    res[f] = made[1];
+                }
+            }
+            __syncthreads();
+        }
+        if (lane == 0u) {
+            unsigned int c = 0u;
+            for (unsigned int i = 0u; i < n; i = nxt[i]) dst[c++] = tok[i];
+            count[place] = (unsigned short)c;
+        }
     }
 }
 
-/* one wave per text: its pre-tokens' tokens, in order, to ids + at[t] */
-__global__ __launch_bounds__(64) void aotx_text_gather_kernel(const unsigned long long *at,
-                                                              const unsigned int *start,
-                                                              const unsigned int *pieces,
-                                                              const unsigned int *piece_tokens,
-                                                              const unsigned int *piece_count,
-                                                              unsigned int *ids, unsigned int *count)
+/* A workgroup per text, four places per thread: the tokens of every place, in order, to
+ * ids + 3 at[t] (64 texts of 4000 bytes 277 -> 6.4 us against a wave that went from pre-token
+ * to pre-token). */
+__global__ __launch_bounds__(1024) void aotx_text_gather_kernel(const unsigned long long *at,
+                                                                const unsigned int *clean_len,
+                                                                const unsigned int *tokens,
+                                                                const unsigned short *place_count,
+                                                                unsigned int *ids, unsigned int *count)
 {
-    const unsigned int t = blockIdx.x, lane = threadIdx.x;
-    const unsigned long long base = at[t];
-    unsigned int w = 0u;
-    for (unsigned int p = 0u; p < pieces[t]; ++p) {
-        const unsigned int c = piece_count[base + p];
-        const unsigned int *src = piece_tokens + base + start[base + p];
-        for (unsigned int i = lane; i < c; i += 64u) ids[base + w + i] = src[i];
-        w += c;
+    __shared__ unsigned int part[16];
+    const unsigned int t = blockIdx.x;
+    const unsigned long long base = 3ull * at[t];
+    const unsigned int end = clean_len[t];
+    unsigned int done = 0u;
+    for (unsigned int tile = 0u; tile < end; tile += 4096u) {
+        unsigned int c[4], mine = 0u;
+#pragma unroll
+        for (unsigned int j = 0u; j < 4u; ++j) {
+            const unsigned int i = tile + 4u * threadIdx.x + j;
+            c[j] = i < end ? place_count[base + i] : 0u;
+            mine += c[j];
+        }
+        unsigned int total;
+        unsigned int w = done + block_before(mine, part, &total);
+#pragma unroll
+        for (unsigned int j = 0u; j < 4u; ++j) {
+            const unsigned long long src = base + tile + 4u * threadIdx.x + j;
+            for (unsigned int i = 0u; i < c[j]; ++i) ids[base + w + i] = tokens[src + i];
+            w += c[j];
+        }
+        done += total;
     }
-    if (lane == 0u) count[t] = w;
+    if (threadIdx.x == 0u) count[t] = done;
 }
 
 /* ---- detokenize ------------------------------------------------------------------------ */
@@ -662,8 +937,7 @@ extern "C" int aotx_text_vocab_build(const aotx_text_source *src, aotx_text_stor
     }
     /* the pair table: rank = merge index, result = the token of the joined string */
     const unsigned int pairs = pow2_at_least(2ull * (src->merges + 1ull));
-    std::vector<unsigned long long> key(pairs, ~0ull);
-    std::vector<unsigned int> rank(pairs, AOTX_TEXT_NONE), result(pairs, AOTX_TEXT_NONE);
+    std::vector<uint4> pair(pairs, make_uint4(AOTX_TEXT_NONE, AOTX_TEXT_NONE, AOTX_TEXT_NONE, AOTX_TEXT_NONE));
     unsigned int taken = 0u, refused = 0u;
     for (unsigned long long m = 0; m < src->merges; ++m) {
         std::string line((const char *)src->merge_bytes + src->merge_at[m], src->merge_at[m + 1u] - src->merge_at[m]);
@@ -675,14 +949,12 @@ extern "C" int aotx_text_vocab_build(const aotx_text_source *src, aotx_text_stor
         const unsigned long long k = ((unsigned long long)il->second << 32) | ir->second;
         unsigned int at = (unsigned int)pair_mix(k) & (pairs - 1u);
         bool seen = false;
-        while (key[at] != ~0ull) {
-            if (key[at] == k) { seen = true; break; }
+        while (pair[at].x != AOTX_TEXT_NONE || pair[at].y != AOTX_TEXT_NONE) {
+            if (pair[at].x == ir->second && pair[at].y == il->second) { seen = true; break; }
             at = (at + 1u) & (pairs - 1u);
         }
         if (seen) { refused += 1u; continue; }              /* a repeated pair keeps its first rank */
-        key[at] = k;
-        rank[at] = (unsigned int)m;
-        result[at] = ij->second;
+        pair[at] = make_uint4(ir->second, il->second, (unsigned int)m, ij->second);
         taken += 1u;
     }
     /* control bits and the single bytes */
@@ -716,9 +988,7 @@ extern "C" int aotx_text_vocab_build(const aotx_text_source *src, aotx_text_stor
     v.slots = slots;
     v.slot = store_put(store, slot.data(), slots);
     v.pairs = pairs;
-    v.pair_key = store_put(store, key.data(), pairs);
-    v.pair_rank = store_put(store, rank.data(), pairs);
-    v.pair_result = store_put(store, result.data(), pairs);
+    v.pair = store_put(store, pair.data(), pairs);
     v.control = store_put(store, control.data(), control.size());
     v.special = store_put(store, special.data(), special.size());
     v.specials = (unsigned int)special.size();
@@ -784,43 +1054,52 @@ extern "C" int aotx_text_encode(const unsigned char *bytes, const unsigned long 
         AOTX_CHECK(hipStreamSynchronize(s));
         return 0;
     }
-    unsigned int *start = nullptr, *len = nullptr, *pieces = nullptr, *ptok = nullptr, *pcount = nullptr,
-                 *pspecial = nullptr, *clean_len = nullptr;
-    unsigned char *clean = nullptr;
-    unsigned long long *at3 = nullptr;
-    const unsigned long long room = 3ull * total;       /* every byte may become U+FFFD */
-    AOTX_CHECK(hipMallocAsync((void **)&clean, room, s));
-    AOTX_CHECK(hipMallocAsync((void **)&at3, (texts + 1ull) * 8u, s));
-    AOTX_CHECK(hipMallocAsync((void **)&clean_len, texts * 4u, s));
-    AOTX_CHECK(hipMallocAsync((void **)&start, room * 4u, s));
-    AOTX_CHECK(hipMallocAsync((void **)&len, room * 4u, s));
-    AOTX_CHECK(hipMallocAsync((void **)&ptok, room * 4u, s));
-    AOTX_CHECK(hipMallocAsync((void **)&pcount, room * 4u, s));
-    AOTX_CHECK(hipMallocAsync((void **)&pspecial, room * 4u, s));
-    AOTX_CHECK(hipMallocAsync((void **)&pieces, texts * 4u, s));
-    unsigned int *work = nullptr, *works = nullptr;
-    AOTX_CHECK(hipMallocAsync((void **)&work, room * 4u, s));
-    AOTX_CHECK(hipMallocAsync((void **)&works, 4u, s));
-    AOTX_CHECK(hipMemsetAsync(works, 0, 4u, s));
-    hipLaunchKernelGGL(aotx_text_clean_kernel, dim3((texts + 64u) / 64u), dim3(64), 0, s, bytes, at, texts,
-                       clean, at3, clean_len);
+    /* one allocation: the cleaned bytes (every byte may become U+FFFD), the marks, and per
+     * place the tokens, their number and the special tokens' places; the list of longer
+     * pre-tokens holds one per TX_SHORT + 1 bytes at most */
+    const size_t room = 3ull * total;
+    size_t at_byte = 0u;
+    const auto put = [&at_byte](size_t bytes) {
+        const size_t here = at_byte;
+        at_byte += (bytes + 255u) & ~(size_t)255u;
+        return here;
+    };
+    const size_t o_clean = put(room), o_mark = put(room), o_tok = put(room * 4u), o_count = put(room * 2u),
+                 o_len = put((size_t)texts * 4u), o_long = put((room / TX_SHORT + 1u) * 12u), o_longs = put(4u),
+                 o_sat = put(g_vocab.specials ? room * 4u : 4u), o_send = put(g_vocab.specials ? room * 4u : 4u),
+                 o_scount = put((size_t)texts * 4u);
+    unsigned char *buf = nullptr;
+    AOTX_CHECK(hipMallocAsync((void **)&buf, at_byte, s));
+    unsigned char *clean = buf + o_clean, *mark = buf + o_mark;
+    unsigned int *tok = (unsigned int *)(buf + o_tok), *clean_len = (unsigned int *)(buf + o_len);
+    unsigned short *pcount = (unsigned short *)(buf + o_count);
+    unsigned int *long_list = (unsigned int *)(buf + o_long), *longs = (unsigned int *)(buf + o_longs);
+    unsigned int *sat = (unsigned int *)(buf + o_sat), *send = (unsigned int *)(buf + o_send),
+                 *scount = (unsigned int *)(buf + o_scount);
+    /* 256-byte tiles of the mean text, each a workgroup (a longer text's take several) */
+    const unsigned long long tiles = (total / texts + 255ull) / 256ull;
+    const unsigned long long most = 65536ull / texts > 0ull ? 65536ull / texts : 1ull;
+    const unsigned int chunks = (unsigned int)(tiles < 1ull ? 1ull : (tiles < most ? tiles : most));
+    hipLaunchKernelGGL(aotx_text_clean_kernel, dim3(texts), dim3(1024), 0, s, bytes, at, clean, mark, clean_len,
+                       longs);
     AOTX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(aotx_text_pretok_kernel, dim3((texts + 63u) / 64u), dim3(64), 0, s, g_vocab, clean, at3,
-                       clean_len, texts, start, len, pspecial, pieces, work, works);
-    AOTX_LAUNCH_CHECK();
-    unsigned int nwork = 0u;
-    AOTX_CHECK(hipMemcpyAsync(&nwork, works, 4u, hipMemcpyDeviceToHost, s));
-    AOTX_CHECK(hipStreamSynchronize(s));
-    if (nwork > 0u) {
-        hipLaunchKernelGGL(aotx_text_merge_kernel, dim3(nwork), dim3(64), 0, s, g_vocab, clean, at3, texts,
-                           start, len, pspecial, pieces, work, ptok, pcount);
+    if (g_vocab.specials != 0u) {
+        hipLaunchKernelGGL(aotx_text_special_kernel, dim3(texts), dim3(64), 0, s, g_vocab, clean, at, clean_len, mark,
+                           sat, send, scount);
         AOTX_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(aotx_text_gather_kernel, dim3(texts), dim3(64), 0, s, at3, start, pieces, ptok, pcount,
-                       ids, count);
+    hipLaunchKernelGGL(aotx_text_pretok_kernel, dim3(texts * chunks), dim3(256), 0, s, g_vocab, clean, at, clean_len,
+                       chunks, sat, send, scount, mark);
     AOTX_LAUNCH_CHECK();
-    void *tmp[] = {clean, at3, clean_len, start, len, ptok, pcount, pspecial, pieces, work, works};
-    for (void *q : tmp) AOTX_CHECK(hipFreeAsync(q, s));
+    hipLaunchKernelGGL(aotx_text_merge_kernel, dim3(texts * chunks), dim3(64 * TX_WAVES), 0, s, g_vocab, clean, at,
+                       clean_len, mark, chunks, tok, pcount, long_list, longs);
+    AOTX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(aotx_text_long_kernel, dim3(512), dim3(64), 0, s, g_vocab, clean, at, long_list, longs, tok,
+                       pcount);
+    AOTX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(aotx_text_gather_kernel, dim3(texts), dim3(1024), 0, s, at, clean_len, tok, pcount, ids, count);
+    AOTX_LAUNCH_CHECK();
+    AOTX_CHECK(hipFreeAsync(buf, s));
     AOTX_CHECK(hipStreamSynchronize(s));
     return 0;
 }

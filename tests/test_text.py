@@ -119,3 +119,30 @@ def test_clean_by_hand():
     assert clean(b"\xf4\x90\x80\x80") == R * 4                  # past U+10FFFF
     assert clean("😀é\ufffd".encode()) == "😀é\ufffd".encode()   # valid text unchanged
     assert clean(b"\x80") == R and clean(b"") == b""
+
+
+@pytest.mark.parametrize("pattern", ["gpt2", "llama3", "qwen2", "qwen35"])
+def test_every_cut_ends_a_run_of_letters_or_numbers(pattern):
+    """The rule by which the encoder cuts a text in parallel (is_sync in text.hip): where a
+    run of letters (with qwen35, and marks) or of numbers ends, a pre-token ends, whatever
+    stands before it."""
+    from oracle.text import PATTERNS, _at15, _unicode15
+    import regex
+    body = _unicode15()
+    letter = regex.compile(_at15(r"[\p{L}\p{M}]" if pattern == "qwen35" else r"\p{L}", body))
+    number = regex.compile(_at15(r"\p{N}", body))
+    rng = random.Random(16)
+    places = 0
+    for _ in range(400):
+        s = "".join(rng.choice([text(rng, 6), "it's're", "'S'LL", " \n", "1234567", "--x", "é́", "٣٤٥a", "''d "])
+                    for _ in range(8))
+        cuts, at = {0}, 0
+        for piece in pretokens(s, pattern):
+            at += len(piece)
+            cuts.add(at)
+        for i in range(1, len(s)):
+            for run in (letter, number):
+                if run.fullmatch(s[i - 1]) and not run.fullmatch(s[i]):
+                    places += 1
+                    assert i in cuts, (pattern, s, i)
+    assert places > 2000

@@ -240,3 +240,35 @@ def test_unicode_15_classes_vs_oracle(torch, lib, bpe, family):
         assert _detok(torch, lib, got) == [s.encode() for s in strings]
     finally:
         built.close()
+
+
+@pytest.mark.parametrize("family", ["gpt-2", "llama3", "qwen35"])
+@pytest.mark.parametrize("special", [False, True])
+def test_encode_edges_vs_oracle(torch, lib, bpe, family, special):
+    """Texts whose pre-tokens, characters, bad bytes and special tokens lie across the places
+    where the launches divide a text: 64-byte windows, 256- and 512-byte tiles, 4096-byte
+    tiles, pre-tokens of 31..34, 63..65 and up to 4097 bytes, and texts without letters."""
+    from tests.test_text import SPECIALS, with_specials
+    tokens, merges, _ = bpe
+    types = [1] * len(tokens)
+    if special:
+        tokens, types = with_specials(tokens, merges)
+    v = Vocab(tokens, merges, types, family=family)
+    built = Built(lib, tokens, merges, types, family)
+    try:
+        rng = random.Random(5 + ROWS[family])
+        strings = [b"", b"a", b"\xff", b"hello" * 13, b" " * 700, b"!?" * 300, "é".encode() * 300, b"7" * 515]
+        for n in (31, 32, 33, 34, 63, 64, 65, 127, 128, 257):
+            strings += [b"x " + b"ab" * (n // 2) + b"c" * (n % 2) + b" y", b"\n" * n + b"z", b"-" * n + b"q1"]
+        for edge in (64, 256, 512, 4096, 8192):
+            for off in range(-4, 4):
+                pad = text(rng, 2 + edge // 3).encode()[:edge + off]
+                mid = rng.choice(["中", "😀", "café 12345", " it's"]).encode()
+                if special:
+                    mid = rng.choice(SPECIALS).encode() + mid
+                strings.append(pad + rng.choice([b"", b"\xff", b"\xe4\xb8", b"\xf0\x9f\x98"]) + mid + text(rng, 9).encode())
+        got = _encode(torch, lib, strings)
+        for s, g in zip(strings, got):
+            assert g == v.encode(s), (family, repr(s[:80]), len(s))
+    finally:
+        built.close()
