@@ -691,7 +691,6 @@ extern "C" int aotx_model_open(unsigned int role, unsigned int max_tokens)
         fprintf(stderr, "aotx: the rank role needs a class head of Q8_0, F16 or F32\n");
         return 1;
     }
-    aotx_gemv_init();
     aotx_state_device();
     /* the token capacity is a power of two, so every bucket of a call fits */
     unsigned int cap = 1u;

@@ -41,7 +41,8 @@ enum {
 };
 
 struct aotx_rgemv_args {
-    const unsigned char *w[3];    /* Q8R tensors stacked along n */
+    const unsigned char *w[3];    /* Q8R tensors stacked along n (file: Q8_0 rows as the model
+                                     file has them, [rows][k/32 blocks of 34 B]) */
     unsigned int seg_end[3];      /* cumulative row ends (multiples of 16 except the last) */
     unsigned int nseg;
     unsigned int n;               /* rows (SWIGLU: rows of one of the pair) */
@@ -51,6 +52,7 @@ struct aotx_rgemv_args {
     unsigned int wide;            /* 1: the tile-split wide-batch kernel (fp16 x only) */
     unsigned int gemm;            /* 1: the GEMM of 33..512 rows (fp16 x, direct rows) */
     unsigned int frag;            /* 1: the fragment-layout product (AOTX_X_FRAG, 5..32 rows) */
+    unsigned int file;            /* 1: the weights are in the file's layout */
     unsigned int pd;              /* quads loaded ahead per wave (narrow kernel) */
     unsigned int nw;              /* waves per workgroup (narrow kernel: 4 or 8) */
     unsigned int groups;          /* workgroups along n */
@@ -83,7 +85,10 @@ struct aotx_rgemv_args {
                                      rsqrt(sum / k + eps) (the RMSNorm scale of x) */
     float row_eps;
     aotx_qkv_epi qkv;
-    /* routed experts (grid.y): as aotx_gemv_args */
+    /* Routed experts (grid.y = expert): the weights of expert e start e * expert_stride bytes
+     * after w[seg]; its batch rows are list[e * list_cap + i] for i < list_count[e] (slot =
+     * token * used + rank); x row = slot / xrow_div; the result row is the slot. Zero
+     * expert_stride = a plain product. */
     unsigned long long expert_stride;
     const unsigned int *list;
     const unsigned int *list_count;
@@ -112,6 +117,9 @@ int aotx_rgemv_plan_routed(aotx_rgemv_args *a, const void *const *w, const unsig
  * refused. */
 int aotx_rgemv_plan_frag(aotx_rgemv_args *a, const void *const *w, const unsigned int *rows,
                          unsigned int nseg, unsigned int k, int epi, unsigned int mt);
+/* Take a planned product's weights in the file's layout (rows of k / 32 blocks of 34 bytes,
+ * any alignment) instead of Q8R: the same plan, kernels, operands and order of sums. */
+static inline void aotx_rgemv_file(aotx_rgemv_args *a) { a->file = 1u; }
 /* Launch one pass (<= 32 rows) and, with splits > 1, the kernel that adds the partials
  * and applies the epilogue. */
 int aotx_rgemv_launch(const aotx_rgemv_args &a, hipStream_t stream);   /* 1 when refused */

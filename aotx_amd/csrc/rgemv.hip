@@ -1,8 +1,11 @@
-/* Streaming Q8 product over repacked (Q8R) weights, for the decode step.
+/* Streaming Q8 product, over repacked (Q8R) weights for the decode step and over the file's
+ * layout (FILE, rg_wsrc) for callers that keep it.
  *
- * Same product and operand values as gemv.hip (A = half(q * scale), B = fp16 activations,
- * fp32 accumulation in v_mfma_f32_16x16x32_f16; reference: cuda/model/gemv.cuh:33-195,
- * cuda/model/gemm.cuh:55-189), arranged so that the weight stream never touches LDS and no
+ * Replaces the memory-bound product aotx_gemv_pass (cuda/model/gemv.cuh:33-195), the
+ * hand-written m == 1 module (ptx/gemv_q8.ptx:18-223) and the tensor-core tile aotx_gemm_tile
+ * (cuda/model/gemm.cuh:55-189) with their operand values (A = half(q * scale), exact int8 ->
+ * fp16 and one correctly rounded multiply as the value reader, cuda/model/matrix.cuh:413-422;
+ * B = fp16 activations; fp32 accumulation in v_mfma_f32_16x16x32_f16), arranged so that the weight stream never touches LDS and no
  * wave waits on another inside the k loop:
  *   - a workgroup owns rt 16-row tiles and a k range; its 4 (or 8) waves take contiguous
  *     shares of the k range, each for all rt tiles, and stream their weights with two 16-byte
@@ -16,7 +19,7 @@
  *     over workgroups the partial tiles go to memory and the last split of the group to
  *     finish (an arrival counter) adds them in split order and applies the epilogue, so
  *     there is no second launch. Results do not depend on timing.
- *   - epilogues as gemv.hip, plus the residual add that also leaves the sums of squares of
+ *   - epilogues (gemv.h), plus the residual add that also leaves the sums of squares of
  *     every 16 rows for the next norm.
  */
 #include "rgemv_dev.h"
@@ -68,12 +71,12 @@ void aotx_q8r_repack(const void *src, unsigned int n, unsigned int k, void *dst,
 
 /* ---- narrow batches ------------------------------------------------------------- */
 
-template <int MT, int RT, int PD, int NW, bool NORM, bool DIRECT>
+template <int MT, int RT, int PD, int NW, bool NORM, bool DIRECT, bool FILE>
 __global__ __launch_bounds__(64 * NW) void aotx_rgemv(aotx_rgemv_args a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     aotx_args_touch(a);
-    rg_narrow<MT, RT, PD, NW, NORM, DIRECT>(a, blockIdx.x, blockIdx.y, lds);
+    rg_narrow<MT, RT, PD, NW, NORM, DIRECT, FILE>(a, blockIdx.x, blockIdx.y, lds);
 }
 
 /* Wide batches (17..32 rows of fp16 x): a workgroup owns T 16-row tiles; its W = T * P
@@ -85,7 +88,7 @@ __global__ __launch_bounds__(64 * NW) void aotx_rgemv(aotx_rgemv_args a)
  * phase order through LDS and the workgroup applies the epilogue (with k split over
  * workgroups, the last split to finish adds the splits first). More phases put more waves
  * on the same tiles (more loads in flight per CU) at the price of more x staging. */
-template <int T, int P, int KC, int PDQ>
+template <int T, int P, int KC, int PDQ, bool FILE>
 __global__ __launch_bounds__(64 * T * P, 4) void aotx_rgemv_wide(aotx_rgemv_args a0)
 {
     /* direct rows: grid.y is the 32-row pass (routed experts: the expert) */
@@ -127,12 +130,13 @@ __global__ __launch_bounds__(64 * T * P, 4) void aotx_rgemv_wide(aotx_rgemv_args
     const unsigned int r = lane & 15u, g = lane >> 4;
     const unsigned int tj = wave / P, ph = wave % P;
 
-    unsigned int dummy = 0u;
-    const unsigned char *qb = rg_tile(a, group, tj, T, expert, dummy) + lane * 16u;
-    const unsigned short *sb = rg_scales(a, group, tj, T, expert) + lane;
+    const rg_wsrc<FILE> wsrc = rg_wopen<FILE>(a, group, tj, T, expert, lane);
+    const unsigned int wend = rg_wend<FILE>(a, lane);
+    const unsigned int wlim = FILE && wend < q1 ? wend : q1;     /* quads past it add nothing */
     rg_f4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
-    rg_u4 wa[2][PDQ][2];             /* two buffers of PDQ quads */
-    unsigned int ws[2][PDQ];         /* one 32-bit register per scale: no packing waits */
+    const unsigned int wshift = rg_wshift<FILE>(wsrc, lane);
+    rg_wreg wr[2][PDQ];              /* two buffers of PDQ quads (one 32-bit register per scale:
+                                        no packing waits) */
 
 /* the wave's n-th quad: chunk n / NQ, its phase's (n % NQ)-th quad of that chunk */
 #define RGW_QUAD(N) (q0 + ((N) / NQ) * KC + ph + P * ((N) % NQ))
@@ -141,10 +145,7 @@ __global__ __launch_bounds__(64 * T * P, 4) void aotx_rgemv_wide(aotx_rgemv_args
         _Pragma("unroll") for (int qi = 0; qi < PDQ; ++qi) {                             \
             unsigned int qq = RGW_QUAD((N) + (unsigned int)qi);                          \
             if (qq >= q1) qq = q1 - 1u;         /* past the range: a cache hit, unused */ \
-            const rg_u4 *src = (const rg_u4 *)(qb + (unsigned long long)qq * 2048ull);   \
-            wa[BUF][qi][0] = __builtin_nontemporal_load(src);                            \
-            wa[BUF][qi][1] = __builtin_nontemporal_load(src + 64);                       \
-            ws[BUF][qi] = __builtin_nontemporal_load(&sb[(unsigned long long)qq * 64ull]); \
+            rg_wload<FILE, true>(a, wsrc, qq, lane, wr[BUF][qi]);                        \
         }                                                                                \
     } while (0)
     /* branch-free: a quad past the range reads a valid x quad and has its scale zeroed */
@@ -158,16 +159,12 @@ __global__ __launch_bounds__(64 * T * P, 4) void aotx_rgemv_wide(aotx_rgemv_args
             _Pragma("unroll") for (int t = 0; t < 2; ++t)                                \
                 _Pragma("unroll") for (int s = 0; s < 4; ++s)                            \
                     B[t][s] = *(const rg_h8 *)(xq + ((unsigned int)t * 16u + r) * XS + 8u * s); \
-            const unsigned int sbits = qq < q1 ? ws[BUF][qi] : 0u;                       \
+            unsigned int qd[8], sbits;                                                   \
+            rg_wquants<FILE>(wr[BUF][qi], wshift, qd, sbits);                            \
+            sbits = qq < wlim ? sbits : 0u;                                              \
             rg_h2 s2 = __builtin_bit_cast(rg_h2, sbits | (sbits << 16));                 \
-            const rg_u4 q0v = wa[BUF][qi][0], q1v = wa[BUF][qi][1];                      \
-            unsigned int qd[8] = {q0v[0], q0v[1], q0v[2], q0v[3], q1v[0], q1v[1], q1v[2], q1v[3]}; \
             _Pragma("unroll") for (int s = 0; s < 4; ++s) {                              \
-                unsigned int d0, d1, d2, d3;                                             \
-                rg_dequant4(qd[2 * s], s2, d0, d1);                                      \
-                rg_dequant4(qd[2 * s + 1], s2, d2, d3);                                  \
-                rg_u4 av = {d0, d1, d2, d3};                                             \
-                rg_h8 A = __builtin_bit_cast(rg_h8, av);                                 \
+                const rg_h8 A = rg_afrag(qd[2 * s], qd[2 * s + 1], s2);            \
                 acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[0][s], acc[0], 0, 0, 0); \
                 acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[1][s], acc[1], 0, 0, 0); \
             }                                                                            \
@@ -564,7 +561,7 @@ __global__ __launch_bounds__(64 * NW) void aotx_rgemv_frag(aotx_rgemv_args a)
  * of at most one workgroup per CU; larger grids run two per CU at 128 registers, where
  * the second workgroup hides the first one's waits (gate/up at 512 rows: 163 against
  * 181 us), and the MFMA loop reads one x fragment at a time. */
-template <int MB, bool WIDE_REGS>
+template <int MB, bool WIDE_REGS, bool FILE, bool TAIL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ? 2 : 4))) void aotx_rgemm(aotx_rgemv_args a0, unsigned int ny)
 {
     aotx_args_touch(a0);
@@ -599,14 +596,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ?
     const unsigned int mrows = total - a.m0 < (unsigned int)MB ? total - a.m0 : (unsigned int)MB;
 
     unsigned short *xl = (unsigned short *)lds;         /* [2][MB][XS] */
-    const unsigned char *qb[2];
-    const unsigned short *sb[2];
+    rg_wsrc<FILE> wsrc[2];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        unsigned int dummy = 0u;
-        qb[t] = rg_tile(a, group, wave * 2u + (unsigned int)t, RT, 0u, dummy) + lane * 16u;
-        sb[t] = rg_scales(a, group, wave * 2u + (unsigned int)t, RT, 0u) + lane;
-    }
+    for (int t = 0; t < 2; ++t) wsrc[t] = rg_wopen<FILE>(a, group, wave * 2u + (unsigned int)t, RT, 0u, lane);
     rg_f4 acc[2][CB];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -621,30 +613,33 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ?
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
         const unsigned int mm = xrow0 + (unsigned int)i * RSTEP;
-        xoff[i] = (a.m0 + (mm < mrows ? mm : 0u)) * a.ldx + xpc * 8u;
+        xoff[i] = (a.m0 + (mm < mrows ? mm : 0u)) * a.ldx + (TAIL ? 0u : xpc * 8u);
     }
 
-    rg_u4 wa[2][2][2];
-    unsigned int ws[2][2];
+    rg_wreg wr[2][2];
+    unsigned int wshift[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) wshift[t] = rg_wshift<FILE>(wsrc[t], lane);
     /* this split's quads [qb0, qn) */
     const unsigned int qb0 = split * a.qps;
     const unsigned int qn = qb0 + a.qps < a.qn ? qb0 + a.qps : a.qn;
+    const unsigned int wend = rg_wend<FILE>(a, lane);
+    const unsigned int wlim = FILE && wend < qn ? wend : qn;     /* quads past it add nothing */
     /* every call issues the same loads (a quad past k repeats the last: never computed) */
 #define RGM_WLOAD(BUF, Q)                                                                \
     do {                                                                                 \
         const unsigned int qq_ = (Q) < qn ? (Q) : qn - 1u;                               \
         _Pragma("unroll") for (int t = 0; t < 2; ++t) {                                  \
-            const rg_u4 *src = (const rg_u4 *)(qb[t] + (unsigned long long)qq_ * 2048ull); \
-            wa[BUF][t][0] = src[0];                                                      \
-            wa[BUF][t][1] = src[64];                                                     \
-            ws[BUF][t] = __builtin_nontemporal_load(&sb[t][(unsigned long long)qq_ * 64ull]); \
+            rg_wload<FILE, false>(a, wsrc[t], qq_, lane, wr[BUF][t]);                    \
         }                                                                                \
     } while (0)
-    /* x pieces of quad Q (k is a whole number of quads: a quad past k repeats the last) */
+    /* x pieces of quad Q (a quad past the split repeats its last). TAIL: k ends inside the
+     * last quad; a piece past it reads the row's first and is stored as zeros */
     rg_u4 xr[2][PPT];                             /* register buffer XB = Q & 1 holds quad Q */
 #define RGM_XLOAD(XB, Q)                                                                 \
     do {                                                                                 \
-        const unsigned int qx_ = ((Q) < qn ? (Q) : qn - 1u) * 128u;                      \
+        unsigned int qx_ = ((Q) < qn ? (Q) : qn - 1u) * 128u;                            \
+        if (TAIL) qx_ = qx_ + xpc * 8u < a.k ? qx_ + xpc * 8u : 0u;                      \
         _Pragma("unroll") for (int i = 0; i < PPT; ++i)                                  \
             xr[XB][i] = *(const rg_u4 *)(a.x + xoff[i] + qx_);                           \
     } while (0)
@@ -657,7 +652,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ?
                             + xrow0 * XS + xpc * 8u;                                     \
         _Pragma("unroll") for (int i = 0; i < PPT; ++i)                                  \
             *(rg_u4 *)(xb_ + (unsigned int)i * RSTEP * XS) =                             \
-                xrow0 + (unsigned int)i * RSTEP < mrows ? xr[XB][i] : (rg_u4){0u, 0u, 0u, 0u}; \
+                xrow0 + (unsigned int)i * RSTEP < mrows                                  \
+                && (!TAIL || (Q) * 128u + xpc * 8u < a.k) ? xr[XB][i] : (rg_u4){0u, 0u, 0u, 0u}; \
     } while (0)
 
     /* Quad q is computed from LDS x buffer q & 1 and weight buffer q & 1. Its step first
@@ -676,21 +672,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ?
     do {                                                                                 \
         const unsigned int qc_ = (QQ);                                                   \
         const unsigned short *xb = xl + RGM_XBUF(qc_) * (unsigned int)(MB * XS) + RGM_XPOS(qc_); \
-        const unsigned int sq_ = qc_ < qn ? 0xffffffffu : 0u;                            \
+        const unsigned int sq_ = qc_ < wlim ? 0xffffffffu : 0u;                          \
         rg_h8 A[2][4];                                                                   \
         _Pragma("unroll") for (int t = 0; t < 2; ++t) {                                  \
-            const unsigned int sbits = ws[BUF][t] & sq_;                                 \
+            unsigned int qd[8], sbits;                                                   \
+            rg_wquants<FILE>(wr[BUF][t], wshift[t], qd, sbits);                          \
+            sbits &= sq_;                                                                \
             rg_h2 s2 = __builtin_bit_cast(rg_h2, sbits | (sbits << 16));                 \
-            const rg_u4 q0v = wa[BUF][t][0], q1v = wa[BUF][t][1];                        \
-            unsigned int qd[8] = {q0v[0], q0v[1], q0v[2], q0v[3],                        \
-                                  q1v[0], q1v[1], q1v[2], q1v[3]};                       \
-            _Pragma("unroll") for (int s = 0; s < 4; ++s) {                              \
-                unsigned int d0, d1, d2, d3;                                             \
-                rg_dequant4(qd[2 * s], s2, d0, d1);                                      \
-                rg_dequant4(qd[2 * s + 1], s2, d2, d3);                                  \
-                rg_u4 av = {d0, d1, d2, d3};                                             \
-                A[t][s] = __builtin_bit_cast(rg_h8, av);                                 \
-            }                                                                            \
+            _Pragma("unroll") for (int s = 0; s < 4; ++s)                                \
+                A[t][s] = rg_afrag(qd[2 * s], qd[2 * s + 1], s2);                  \
         }                                                                                \
         if constexpr (WIDE_REGS) {                                                       \
             /* k step outermost: the step's x fragments are read together and its 8 */  \
@@ -888,12 +878,13 @@ static int aotx_rgemv_plan_n(aotx_rgemv_args *a, const void *const *w, const uns
     unsigned int kmax = 98304u / (mt * 256u);
     if (kmax < 1u) kmax = 1u;
     unsigned int s = (a->qn + kmax - 1u) / kmax;
-    while (a->groups * s < target && (a->qn + s) / (s + 1u) >= minq) s += 1u;
+    /* (routed products: a workgroup row per expert fills the chip, as for the wide kernel) */
+    while (!routed && a->groups * s < target && (a->qn + s) / (s + 1u) >= minq) s += 1u;
     a->qps = (a->qn + s - 1u) / s;
     a->splits = (a->qn + a->qps - 1u) / a->qps;
     /* 8 waves per workgroup while the launch has few workgroups (each wave then has half
      * the quads to dequantise after its data arrives), 4 otherwise */
-    a->nw = a->groups * a->splits <= 256u ? 8u : 4u;
+    a->nw = !routed && a->groups * a->splits <= 256u ? 8u : 4u;
     return 0;
 }
 
@@ -970,21 +961,33 @@ static void aotx_rgemv_go(const aotx_rgemv_args &a, hipStream_t s)
     const bool direct = a.expert_stride == 0ull && a.list == nullptr && a.xrow == nullptr;
 #define RGN_GO(NW, NORM)                                                                   \
     do {                                                                                   \
-        if (direct) hipLaunchKernelGGL((aotx_rgemv<MT, RT, PD, NW, NORM, true>), grid, dim3(64 * NW), lds, s, a); \
-        else hipLaunchKernelGGL((aotx_rgemv<MT, RT, PD, NW, NORM, false>), grid, dim3(64 * NW), lds, s, a); \
+        if (direct) hipLaunchKernelGGL((aotx_rgemv<MT, RT, PD, NW, NORM, true, false>), grid, dim3(64 * NW), lds, s, a); \
+        else hipLaunchKernelGGL((aotx_rgemv<MT, RT, PD, NW, NORM, false, false>), grid, dim3(64 * NW), lds, s, a); \
     } while (0)
-    if (a.nw == 8u) {
+#define RGN_FILE(NW)                                                                       \
+    do {                                                                                   \
+        if (direct) hipLaunchKernelGGL((aotx_rgemv<MT, RT, PD, NW, false, true, true>), grid, dim3(64 * NW), lds, s, a); \
+        else hipLaunchKernelGGL((aotx_rgemv<MT, RT, PD, NW, false, false, true>), grid, dim3(64 * NW), lds, s, a); \
+    } while (0)
+    if (a.file) {
+        if (a.nw == 8u) RGN_FILE(8); else RGN_FILE(4);
+    } else if (a.nw == 8u) {
         if (norm) RGN_GO(8, true); else RGN_GO(8, false);
     } else {
         if (norm) RGN_GO(4, true); else RGN_GO(4, false);
     }
 #undef RGN_GO
+#undef RGN_FILE
     AOTX_LAUNCH_CHECK();
 }
 
 int aotx_rgemv_launch(const aotx_rgemv_args &a0, hipStream_t s)
 {
     aotx_rgemv_args a = a0;
+    if (a.file && (a.frag || a.xmode != AOTX_X_F16)) {
+        fprintf(stderr, "aotx: the product over the file's layout takes fp16 x only\n");
+        return 1;
+    }
     if (a.splits > 1u && a.partial == nullptr) {
         a.partial = (float *)aotx_scratch(AOTX_SCRATCH_GEMV_PARTIAL, aotx_rgemv_partial_bytes(a));
     }
@@ -1001,10 +1004,19 @@ int aotx_rgemv_launch(const aotx_rgemv_args &a0, hipStream_t s)
         const unsigned int ny = (a.m + RGM_MB - 1u) / RGM_MB;
         const dim3 g1(((a.groups + 7u) / 8u) * 8u * ny * a.splits);
         const size_t x2 = 2u * RGM_MB * (256u + 8u) * 2u, res = RGM_RT * 16u * RGM_MB * 4u;
-        if (g1.x <= 256u)
-            hipLaunchKernelGGL((aotx_rgemm<RGM_MB, true>), g1, dim3(512), x2 > res ? x2 : res, s, a, ny);
-        else
-            hipLaunchKernelGGL((aotx_rgemm<RGM_MB, false>), g1, dim3(512), x2 > res ? x2 : res, s, a, ny);
+#define RGM_GO(WIDE, FILE, TAIL)                                                           \
+    hipLaunchKernelGGL((aotx_rgemm<RGM_MB, WIDE, FILE, TAIL>), g1, dim3(512), x2 > res ? x2 : res, s, a, ny)
+        const bool tail = a.k % 128u != 0u;
+        if (g1.x <= 256u) {
+            if (a.file) RGM_GO(true, true, true);
+            else if (tail) RGM_GO(true, false, true);
+            else RGM_GO(true, false, false);
+        } else {
+            if (a.file) RGM_GO(false, true, true);
+            else if (tail) RGM_GO(false, false, true);
+            else RGM_GO(false, false, false);
+        }
+#undef RGM_GO
         AOTX_LAUNCH_CHECK();
         return 0;
     }
@@ -1048,29 +1060,21 @@ int aotx_rgemv_launch(const aotx_rgemv_args &a0, hipStream_t s)
             fprintf(stderr, "aotx: the wide-batch product takes fp16 x only\n");
             return 1;
         }
-        if (a.rt == 2u) {
-            const size_t xb = 2u * 32u * (8u * 128u + 8u) * 2u;
-            hipLaunchKernelGGL((aotx_rgemv_wide<2, 4, 8, 1>), grid, dim3(512), xb, s, a);
-        } else if (a.rt == 4u) {
-            const size_t xb = 2u * 32u * (4u * 128u + 8u) * 2u;
-            hipLaunchKernelGGL((aotx_rgemv_wide<4, 2, 4, 1>), grid, dim3(512), xb, s, a);
-        } else {
-            const size_t xb = 2u * 32u * (4u * 128u + 8u) * 2u;
-            hipLaunchKernelGGL((aotx_rgemv_wide<8, 1, 4, 2>), grid, dim3(512), xb, s, a);
-        }
+#define RGW_GO(T, P, KC, PDQ)                                                              \
+        do {                                                                               \
+            const size_t xb = 2u * 32u * (KC * 128u + 8u) * 2u;                            \
+            if (a.file) hipLaunchKernelGGL((aotx_rgemv_wide<T, P, KC, PDQ, true>), grid, dim3(512), xb, s, a); \
+            else hipLaunchKernelGGL((aotx_rgemv_wide<T, P, KC, PDQ, false>), grid, dim3(512), xb, s, a); \
+        } while (0)
+        if (a.rt == 2u) RGW_GO(2, 4, 8, 1);
+        else if (a.rt == 4u) RGW_GO(4, 2, 4, 1);
+        else RGW_GO(8, 1, 4, 2);
+#undef RGW_GO
         AOTX_LAUNCH_CHECK();
         return 0;
     }
-    if (a.rt == 1u) {
-        if (a.pd >= 8u) aotx_rgemv_go<16, 1, 8>(a, s);
-        else aotx_rgemv_go<16, 1, 4>(a, s);
-    } else if (a.rt == 2u) {
-        if (a.pd >= 4u) aotx_rgemv_go<16, 2, 4>(a, s);
-        else aotx_rgemv_go<16, 2, 2>(a, s);
-    } else {
-        if (a.pd >= 2u) aotx_rgemv_go<16, 4, 2>(a, s);
-        else aotx_rgemv_go<16, 4, 1>(a, s);
-    }
+    if (a.rt == 1u) aotx_rgemv_go<16, 1, 4>(a, s);
+    else aotx_rgemv_go<16, 4, 1>(a, s);
     return 0;
 }
 
@@ -1090,8 +1094,9 @@ extern "C" int aotx_q8_repack(const void *w, unsigned int n, unsigned int k, voi
     return 0;
 }
 
+/* file: wr holds the tensor as the model file has it, not repacked */
 static int aotx_q8r_gemv_any(const void *wr, unsigned int n, unsigned int k, const void *x,
-                             unsigned int m, void *y, int epi, void *stream)
+                             unsigned int m, void *y, int epi, bool file, void *stream)
 {
     if (wr == nullptr || x == nullptr || y == nullptr || n == 0u || m == 0u) return 1;
     if (k == 0u || k % 32u != 0u || k % 8u != 0u) return 1;
@@ -1107,6 +1112,7 @@ static int aotx_q8r_gemv_any(const void *wr, unsigned int n, unsigned int k, con
          * (measured on the four 8B shapes) */
         const unsigned int narrow_max = (n + 15u) / 16u <= 256u && k <= 4096u ? 8u : AOTX_NARROW_ROWS;
         if (aotx_rgemv_plan_n(&a, ws, rows, 1u, k, epi, mt, narrow_max) != 0) return 1;
+        if (file) aotx_rgemv_file(&a);
         a.xmode = AOTX_X_F16;
         a.x = (const unsigned short *)x;
         a.ldx = k;
@@ -1121,11 +1127,23 @@ static int aotx_q8r_gemv_any(const void *wr, unsigned int n, unsigned int k, con
 extern "C" int aotx_q8r_gemv(const void *wr, unsigned int n, unsigned int k, const void *x,
                              unsigned int m, float *y, void *stream)
 {
-    return aotx_q8r_gemv_any(wr, n, k, x, m, y, AOTX_EPI_F32, stream);
+    return aotx_q8r_gemv_any(wr, n, k, x, m, y, AOTX_EPI_F32, false, stream);
 }
 
 extern "C" int aotx_q8r_gemv_f16(const void *wr, unsigned int n, unsigned int k, const void *x,
                                  unsigned int m, void *y, void *stream)
 {
-    return aotx_q8r_gemv_any(wr, n, k, x, m, y, AOTX_EPI_F16, stream);
+    return aotx_q8r_gemv_any(wr, n, k, x, m, y, AOTX_EPI_F16, false, stream);
+}
+
+extern "C" int aotx_q8_gemv(const void *w, unsigned int n, unsigned int k, const void *x,
+                            unsigned int m, float *y, void *stream)
+{
+    return aotx_q8r_gemv_any(w, n, k, x, m, y, AOTX_EPI_F32, true, stream);
+}
+
+extern "C" int aotx_q8_gemv_f16(const void *w, unsigned int n, unsigned int k,
+                                const void *x, unsigned int m, void *y, void *stream)
+{
+    return aotx_q8r_gemv_any(w, n, k, x, m, y, AOTX_EPI_F16, true, stream);
 }

@@ -144,6 +144,115 @@ static __device__ __forceinline__ const unsigned short *rg_scales(const aotx_rge
          + (unsigned long long)tile * a.qn * 64ull;
 }
 
+/* Where a lane (r, g) reads the weights of a 16-row tile: block 4q + g of row r for quad q.
+ * Q8R: 16 + 16 bytes of the tile's quant plane and a word of its scale plane, the wave's
+ * loads contiguous. FILE: the 34-byte block where the model file has it; a wave's load covers
+ * 136 contiguous bytes of each of 16 rows, and the next quad goes on in the same lines, so
+ * these take plain loads (the lines stay cached) while Q8R streams. */
+template <bool FILE>
+struct rg_wsrc {
+    const unsigned char *q;       /* FILE: the row */
+    const unsigned short *s;      /* Q8R only */
+};
+/* The registers of one quad. FILE: a block starts at a multiple of four bytes or two past one.
+ * In the first case w0 and w1 hold its first 32 bytes (the scale, then 30 quants) and sc the
+ * last two quants, in the second w0 and w1 hold the quants and sc the scale: three aligned
+ * loads either way. A lane's loads are in another row than its neighbours', so the address
+ * unit, not the memory, bounds them: two 16-byte loads two bytes past alignment took 29.4 us
+ * at 4096 x 14336 and 8 rows, four aligned loads 21.9, three 19.6. Against a copy of 8 quads
+ * through LDS between two barriers and a launch that added the splits: 33.6 us there, and the
+ * routed layer of 8 experts at 64 tokens (1.5 GB) 800 -> 410 us. */
+struct rg_wreg {
+    rg_u4 w0, w1;
+    unsigned int sc;
+};
+template <bool FILE>
+static __device__ __forceinline__ rg_wsrc<FILE> rg_wopen(const aotx_rgemv_args &a, unsigned int group,
+                                                         unsigned int j, unsigned int rt,
+                                                         unsigned int expert, unsigned int lane)
+{
+    rg_wsrc<FILE> w;
+    if constexpr (FILE) {
+        unsigned int seg, row, rows;
+        if (a.epi == AOTX_EPI_SWIGLU) {
+            const unsigned int half = rt / 2u;
+            seg = j < half ? 0u : 1u;
+            row = (group * half + (j < half ? j : j - half)) * 16u;
+            rows = a.n;
+        } else {
+            unsigned int begin;
+            const unsigned int v0 = (group * rt + j) * 16u;
+            seg = rg_seg(a, v0, begin);
+            row = v0 - begin;
+            rows = rg_seg_end(a, seg) - begin;
+        }
+        row += lane & 15u;
+        if (row >= rows) row = rows - 1u;               /* past the last row: discarded */
+        w.q = rg_seg_w(a, seg) + (unsigned long long)expert * a.expert_stride
+            + (unsigned long long)row * ((unsigned long long)(a.k / 32u) * 34ull);
+        w.s = nullptr;
+    } else {
+        unsigned int dummy = 0u;
+        w.q = rg_tile(a, group, j, rt, expert, dummy) + lane * 16u;
+        w.s = rg_scales(a, group, j, rt, expert) + lane;
+    }
+    return w;
+}
+/* The first of a lane's quads that holds no block of the row (FILE: k may end inside a quad;
+ * Q8R pads it with zeros). */
+template <bool FILE>
+static __device__ __forceinline__ unsigned int rg_wend(const aotx_rgemv_args &a, unsigned int lane)
+{
+    return FILE ? (a.k / 32u + 3u - (lane >> 4)) / 4u : a.qn;
+}
+/* Quad q's quants and scale bits (FILE: of the row's last block past its end). */
+template <bool FILE, bool STREAM>
+static __device__ __forceinline__ void rg_wload(const aotx_rgemv_args &a, const rg_wsrc<FILE> &w,
+                                                unsigned int q, unsigned int lane, rg_wreg &o)
+{
+    if constexpr (FILE) {
+        const unsigned int last = a.k / 32u - 1u, at = 4u * q + (lane >> 4);
+        const unsigned char *b = w.q + (at < last ? at : last) * 34u;
+        const unsigned int odd = (unsigned int)(unsigned long long)b & 2u;     /* the quants are aligned */
+        typedef unsigned int u4d __attribute__((ext_vector_type(4), aligned(4)));
+        o.w0 = *(const u4d *)(b + odd);
+        o.w1 = *(const u4d *)(b + odd + 16u);
+        o.sc = *(const unsigned short *)(b + (odd ? 0u : 32u));
+    } else {
+        const rg_u4 *src = (const rg_u4 *)(w.q + (unsigned long long)q * 2048ull);
+        o.w0 = STREAM ? __builtin_nontemporal_load(src) : src[0];
+        o.w1 = STREAM ? __builtin_nontemporal_load(src + 64) : src[64];
+        o.sc = __builtin_nontemporal_load(&w.s[(unsigned long long)q * 64ull]);
+    }
+}
+/* The quad's 32 quants, four to a word as q + 128, and its scale bits. shift: 16 where a
+ * FILE lane's words start with the scale, 0 where with the quants (rg_wshift). */
+template <bool FILE>
+static __device__ __forceinline__ void rg_wquants(const rg_wreg &o, unsigned int shift, unsigned int *qd,
+                                                  unsigned int &scale)
+{
+    const unsigned int w[9] = {o.w0[0], o.w0[1], o.w0[2], o.w0[3], o.w1[0], o.w1[1], o.w1[2], o.w1[3], o.sc};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qd[i] = FILE ? __builtin_amdgcn_alignbit(w[i + 1], w[i], shift) ^ 0x80808080u : w[i];
+    scale = FILE && shift != 0u ? w[0] & 0xffffu : o.sc;
+}
+template <bool FILE>
+static __device__ __forceinline__ unsigned int rg_wshift(const rg_wsrc<FILE> &w, unsigned int lane)
+{
+    /* 34 bytes a block, 136 a quad: the same for every quad of a lane (and not used for the
+     * last block read in place of one past the row's end, whose scale is zeroed) */
+    return ((unsigned int)(unsigned long long)w.q + 2u * (lane >> 4)) & 2u ? 0u : 16u;
+}
+/* Eight quants (two words of q + 128 bytes) as the A operand. */
+static __device__ __forceinline__ rg_h8 rg_afrag(unsigned int u0, unsigned int u1, rg_h2 s2)
+{
+    unsigned int d0, d1, d2, d3;
+    rg_dequant4(u0, s2, d0, d1);
+    rg_dequant4(u1, s2, d2, d3);
+    const rg_u4 av = {d0, d1, d2, d3};
+    return __builtin_bit_cast(rg_h8, av);
+}
+
 /* The virtual output row of row rr of tile j (SWIGLU: the gate/up row index). */
 static __device__ __forceinline__ unsigned int rg_vrow(const aotx_rgemv_args &a, unsigned int group,
                                                        unsigned int j, unsigned int rr, unsigned int rt)
@@ -754,7 +863,7 @@ static __device__ __forceinline__ bool rg_split_merge(const aotx_rgemv_args &a, 
 /* MT: batch columns of the MFMA (16 or 32); RT: 16-row tiles per workgroup; PD: quads
  * loaded ahead per wave; NW: waves per workgroup, splitting the k range (8 for products of
  * few tiles, so that each wave's share of the dequantisation is short). */
-template <int MT, int RT, int PD, int NW, bool NORM, bool DIRECT>
+template <int MT, int RT, int PD, int NW, bool NORM, bool DIRECT, bool FILE>
 static __device__ __forceinline__ void rg_narrow(const aotx_rgemv_args &a, unsigned int bx,
                                                  unsigned int expert_in, unsigned char *lds)
 {
@@ -791,14 +900,14 @@ static __device__ __forceinline__ void rg_narrow(const aotx_rgemv_args &a, unsig
     const unsigned int wq1 = wq0 + per < q1 ? wq0 + per : q1;
     const unsigned int r = lane & 15u, g = lane >> 4;
 
-    const unsigned char *qb[RT];
-    const unsigned short *sb[RT];
+    rg_wsrc<FILE> wsrc[RT];
 #pragma unroll
-    for (int j = 0; j < RT; ++j) {
-        unsigned int dummy = 0u;
-        qb[j] = rg_tile(a, group, (unsigned int)j, RT, expert, dummy) + lane * 16u;
-        sb[j] = rg_scales(a, group, (unsigned int)j, RT, expert) + lane;
-    }
+    for (int j = 0; j < RT; ++j) wsrc[j] = rg_wopen<FILE>(a, group, (unsigned int)j, RT, expert, lane);
+    unsigned int wshift[RT];
+#pragma unroll
+    for (int j = 0; j < RT; ++j) wshift[j] = rg_wshift<FILE>(wsrc[j], lane);
+    const unsigned int wend = rg_wend<FILE>(a, lane);
+    const unsigned int wlim = FILE && wend < wq1 ? wend : wq1;   /* quads past it add nothing */
 
     rg_f4 acc[RT][MT / 16];
 #pragma unroll
@@ -806,8 +915,7 @@ static __device__ __forceinline__ void rg_narrow(const aotx_rgemv_args &a, unsig
 #pragma unroll
         for (int t = 0; t < MT / 16; ++t) acc[j][t] = (rg_f4){0.0f, 0.0f, 0.0f, 0.0f};
 
-    rg_u4 wa[2][PD][RT][2];
-    unsigned int ws[2][PD][RT];    /* one 32-bit register per scale: no packing waits */
+    rg_wreg wr[2][PD][RT];           /* one 32-bit register per scale: no packing waits */
 
     /* loads past the wave's range repeat its last quad (a cache hit), so every load can be
      * issued unconditionally: no register copies that would wait for them */
@@ -818,10 +926,7 @@ static __device__ __forceinline__ void rg_narrow(const aotx_rgemv_args &a, unsig
             unsigned int qq = (QS) + (unsigned int)qi;                                   \
             if (qq > qlast) qq = qlast;                                                  \
             _Pragma("unroll") for (int j = 0; j < RT; ++j) {                             \
-                const rg_u4 *src = (const rg_u4 *)(qb[j] + (unsigned long long)qq * 2048ull); \
-                wa[BUF][qi][j][0] = __builtin_nontemporal_load(src);                    \
-                wa[BUF][qi][j][1] = __builtin_nontemporal_load(src + 64);                \
-                ws[BUF][qi][j] = __builtin_nontemporal_load(&sb[j][(unsigned long long)qq * 64ull]); \
+                rg_wload<FILE, true>(a, wsrc[j], qq, lane, wr[BUF][qi][j]);             \
             }                                                                            \
         }                                                                                \
     } while (0)
@@ -843,17 +948,12 @@ static __device__ __forceinline__ void rg_narrow(const aotx_rgemv_args &a, unsig
                     B[t][s] = *(const rg_h8 *)(xq + mr * xs + 8u * s);                   \
             }                                                                            \
             _Pragma("unroll") for (int j = 0; j < RT; ++j) {                             \
-                const unsigned int sbits = qq < wq1 ? ws[BUF][qi][j] : 0u;               \
+                unsigned int qd[8], sbits;                                               \
+                rg_wquants<FILE>(wr[BUF][qi][j], wshift[j], qd, sbits);                  \
+                sbits = qq < wlim ? sbits : 0u;                                          \
                 rg_h2 s2 = __builtin_bit_cast(rg_h2, sbits | (sbits << 16));             \
-                const rg_u4 q0v = wa[BUF][qi][j][0], q1v = wa[BUF][qi][j][1];            \
-                unsigned int qd[8] = {q0v[0], q0v[1], q0v[2], q0v[3],                    \
-                                      q1v[0], q1v[1], q1v[2], q1v[3]};                   \
                 _Pragma("unroll") for (int s = 0; s < 4; ++s) {                          \
-                    unsigned int d0, d1, d2, d3;                                         \
-                    rg_dequant4(qd[2 * s], s2, d0, d1);                                  \
-                    rg_dequant4(qd[2 * s + 1], s2, d2, d3);                              \
-                    rg_u4 av = {d0, d1, d2, d3};                                         \
-                    rg_h8 A = __builtin_bit_cast(rg_h8, av);                             \
+                    const rg_h8 A = rg_afrag(qd[2 * s], qd[2 * s + 1], s2);        \
                     _Pragma("unroll") for (int t = 0; t < MT / 16; ++t)                  \
                         acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(               \
                             A, B[t][s], acc[j][t], 0, 0, 0);                             \

@@ -168,3 +168,28 @@ def test_repack_layout(torch, lib):
                     assert scale[t, q, lane] == src[row, blk, :2].view(np.uint16)[0]
                 else:
                     assert (quant[t, q, lane] == 0x80).all() and scale[t, q, lane] == 0
+
+
+@pytest.mark.parametrize("n,k,shift", [(17, 96, 0), (33, 160, 2), (48, 32, 0), (300, 4128, 2), (130, 416, 0), (64, 512, 6)])
+@pytest.mark.parametrize("m", [1, 4, 5, 9, 32, 33, 64, 100])
+def test_product_ends_and_alignment(torch, lib, orc, n, k, shift, m):
+    """Products over the file's layout whose blocks start at odd multiples of two bytes (an odd
+    number of blocks a row, a tensor at any even address), and of both layouts where k ends
+    inside 128 and rows inside 16, by every kernel (1-4, 5-32, 33 rows and more). What lies
+    after x and the weights is never used: it holds NaN and scales of infinity here. The fp32
+    sums agree with the fp64 product to 1e-5 of the result's rms."""
+    w = make(torch, lib, n, k, 3 + n + k)
+    buf = torch.full((shift + w.numel() + 512,), 0x7C, dtype=torch.uint8, device="cuda")
+    buf[shift:shift + w.numel()] = w
+    rng = np.random.default_rng(n + m)
+    x = rng.normal(0, 1, (m, k)).astype(np.float16)
+    xb = torch.full((m * k + 256,), float("nan"), dtype=torch.float16, device="cuda")
+    xb[:m * k] = torch.from_numpy(x).cuda().reshape(-1)
+    want = orc.q8_gemv_f64(w.cpu().numpy(), n, k, x.view(np.uint16))
+    rms = np.sqrt((want ** 2).mean())
+    wr = repack(torch, lib, w, n, k)
+    for fn, at in ((lib.aotx_q8_gemv, buf.data_ptr() + shift), (lib.aotx_q8r_gemv, wr.data_ptr())):
+        y = torch.zeros(m * n, dtype=torch.float32, device="cuda")
+        assert fn(ctypes.c_void_p(at), n, k, p(xb), m, p(y), None) == 0
+        torch.cuda.synchronize()
+        assert np.abs(y.cpu().numpy().reshape(m, n) - want).max() < 1e-5 * max(rms, 1.0) * np.sqrt(k / 32.0)
