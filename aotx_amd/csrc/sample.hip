@@ -28,7 +28,10 @@
 #define PICK_BUCKETS 256u
 #define PICK_PASSES 2u
 #define PICK_CHUNKS 64u   /* workgroups per row of the largest-logit search */
-#define PICK_EXP_WGS 32u  /* workgroups per row of the exponentials and first histogram */
+#define PICK_SUMS 16u     /* of the 256 partial sums of a row, those of one workgroup */
+#define PICK_STEPS 64u    /* tokens of each between two barriers */
+#define PICK_AHEAD 8u     /* such blocks loaded together */
+#define PICK_SLICES 16u   /* workgroups per row of the candidates */
 
 #pragma clang fp contract(off)
 
@@ -91,8 +94,12 @@ struct aotx_pick_args {
     aotx_state *state;
     const aotx_model_run *run;    /* when set, every per-call value comes from here */
     unsigned int *best;           /* [rows][PICK_CHUNKS][2]: each chunk's (value bits, token) */
-    unsigned int *hist;           /* [rows][PICK_BUCKETS] first-pass counts, zero between calls */
-    float *ex;                    /* [rows][vocab] exp(v - top) */
+    unsigned int *hist;           /* [rows][PICK_BUCKETS] first-pass counts */
+    float *sums;                  /* [rows][PICK_THREADS] partial sums of exp(v - top) */
+    float *total;                 /* [rows] their sum */
+    unsigned int *cand;           /* [rows][PICK_SLICES][AOTX_MODEL_PICK_MAX][2] (value bits, token) */
+    unsigned int *found;          /* [rows][PICK_SLICES] candidates of each slice */
+    unsigned int *seen;           /* [rows] slices done */
 };
 
 /* (v, i) ranks ahead of (bv, bi) in the reference's largest-logit search: a larger value;
@@ -152,12 +159,14 @@ __global__ __launch_bounds__(PICK_THREADS) void aotx_argmax_kernel(aotx_pick_arg
     int *token_out = run ? run->token : a.token;
     if (r >= rows || token_out == nullptr) return;
     if (run && run->select != AOTX_MODEL_ROWS_LAST) return;
-    /* the row's histogram starts at zero for the exponential pass that follows (its place
+    /* the row's histogram and counts start at zero for the launches that follow (their place
      * in the sampler's buffer depends on the call's row count, so an earlier call with
      * another count may have left other words there) */
-    if (c == 0u)
+    if (c == 0u) {
         for (unsigned int i = tid; i < PICK_BUCKETS; i += PICK_THREADS)
             a.hist[(unsigned long long)r * PICK_BUCKETS + i] = 0u;
+        if (tid == 0u) a.seen[r] = 0u;
+    }
     const float *row = a.logits + (unsigned long long)r * a.ld;
     const unsigned int span = (a.vocab + PICK_CHUNKS - 1u) / PICK_CHUNKS;
     const unsigned int lo = c * span;
@@ -198,13 +207,20 @@ __global__ __launch_bounds__(PICK_THREADS) void aotx_argmax_kernel(aotx_pick_arg
     }
 }
 
-/* exp(v - top) of every logit of a sampled row (stored for the pick's ordered sums) and
- * the first pass of the cut search: the 256-bucket histogram over [top - 42, top], added
- * into the row's counts (integer counts: their order does not matter). Grid: PICK_EXP_WGS
- * x rows; rows at temperature 0 do nothing. */
+/* The ordered sums of exp(v - top) of a sampled row and the first pass of the cut search.
+ * The reference's thread t adds tokens t, t + 256, ... one after another, so a workgroup
+ * takes PICK_SUMS of the 256 sums over the whole row (grid: 256 / PICK_SUMS x rows): its
+ * threads make the exponentials of PICK_STEPS tokens of each sum in LDS, and one lane per sum
+ * adds them in order while the others make the next block's. Every thread also counts its
+ * values in the 256-bucket histogram over [top - 42, top] (counts: any order; a copy per lane
+ * quarter spreads the bulk of the logits, which falls into few buckets). Rows at temperature
+ * 0 do nothing. Bound by the exponentials and the LDS counts of a workgroup. A launch that
+ * stored every exponential (12.4 us at 32 rows of 128256) and one workgroup per row that added
+ * them and walked the row twice more (86.7 us) became this one (15.7) and the next (24). */
 __global__ __launch_bounds__(PICK_THREADS) void aotx_pick_exp_kernel(aotx_pick_args a)
 {
-    __shared__ unsigned int bucket[PICK_BUCKETS];
+    __shared__ unsigned int bucket[4][PICK_BUCKETS + 1u];
+    __shared__ float block[2][PICK_STEPS][PICK_SUMS + 1u];
     const unsigned int tid = threadIdx.x;
     const unsigned int r = blockIdx.y;
     const aotx_model_run *run = a.run;
@@ -213,46 +229,149 @@ __global__ __launch_bounds__(PICK_THREADS) void aotx_pick_exp_kernel(aotx_pick_a
     if (r >= rows || token_out == nullptr) return;
     if (run && run->select != AOTX_MODEL_ROWS_LAST) return;
     if (aotx_pick_warmth(a, r) <= 0.0f) return;
-    float top;
-    unsigned int at;
-    aotx_pick_top(a, r, top, at);
-    for (unsigned int i = tid; i < PICK_BUCKETS; i += PICK_THREADS) bucket[i] = 0u;
-    __syncthreads();
+    for (unsigned int i = tid; i < 4u * (PICK_BUCKETS + 1u); i += PICK_THREADS) (&bucket[0][0])[i] = 0u;
+    constexpr unsigned int PER = PICK_STEPS * PICK_SUMS / PICK_THREADS;    /* values per thread and block */
+    constexpr unsigned int ROWS = PICK_THREADS / PICK_SUMS;                /* steps of one load */
     const float *row = a.logits + (unsigned long long)r * a.ld;
-    float *ex = a.ex + (unsigned long long)r * a.vocab;
+    const unsigned int c = tid % PICK_SUMS, s0 = tid / PICK_SUMS;
+    const unsigned int col = blockIdx.x * PICK_SUMS + c;
+    const unsigned int steps = (a.vocab + PICK_THREADS - 1u) / PICK_THREADS;
     const float lo = -AOTX_MODEL_PICK_SPAN, hi = 0.0f, band = hi - lo;
-    const unsigned int span = (a.vocab + PICK_EXP_WGS - 1u) / PICK_EXP_WGS;
-    const unsigned int b0 = blockIdx.x * span;
-    const unsigned int b1 = b0 + span < a.vocab ? b0 + span : a.vocab;
-#pragma unroll 8
-    for (unsigned int i = b0 + tid; i < b1; i += PICK_THREADS) {
-        const float scaled = row[i] - top;
-        ex[i] = expf(scaled);
-        if (scaled >= lo && scaled <= hi) {
-            unsigned int b = (unsigned int)((scaled - lo) * (float)PICK_BUCKETS / band);
-            if (b >= PICK_BUCKETS) b = PICK_BUCKETS - 1u;
-            atomicAdd(&bucket[b], 1u);
+    unsigned int *mine = bucket[(tid >> 4) & 3u];
+    float sum = 0.0f, top = 0.0f;
+    for (unsigned int first = 0u; first < steps; first += PICK_AHEAD * PICK_STEPS) {
+        float v[PICK_AHEAD][PER];
+#pragma unroll
+        for (unsigned int k = 0u; k < PICK_AHEAD; ++k)
+#pragma unroll
+            for (unsigned int e = 0u; e < PER; ++e) {
+                const unsigned int i = (first + k * PICK_STEPS + e * ROWS + s0) * PICK_THREADS + col;
+                v[k][e] = row[i < a.vocab ? i : 0u];
+            }
+        if (first == 0u) {           /* the largest logit while the first values are on their way */
+            unsigned int at;
+            aotx_pick_top(a, r, top, at);
+            __syncthreads();
         }
+#pragma unroll
+        for (unsigned int k = 0u; k < PICK_AHEAD; ++k) {
+            const unsigned int base = first + k * PICK_STEPS;
+            if (base < steps) {
+    #pragma unroll
+                for (unsigned int e = 0u; e < PER; ++e) {
+                    const unsigned int step = e * ROWS + s0;
+                    const bool in = (base + step) * PICK_THREADS + col < a.vocab;
+                    const float scaled = v[k][e] - top;
+                    if (in) block[k & 1u][step][c] = expf(scaled);
+                    if (in && scaled >= lo && scaled <= hi) {
+                        unsigned int b = (unsigned int)((scaled - lo) * (float)PICK_BUCKETS / band);
+                        if (b >= PICK_BUCKETS) b = PICK_BUCKETS - 1u;
+                        atomicAdd(&mine[b], 1u);
+                    }
+                }
+                __syncthreads();
+                /* the block's values of a sum in token order; the block before it was read before
+                 * this barrier, so the next one may overwrite that */
+                if (tid < PICK_SUMS) {
+                    const unsigned int left = a.vocab > base * PICK_THREADS + col
+                                            ? (a.vocab - base * PICK_THREADS - col + PICK_THREADS - 1u) / PICK_THREADS : 0u;
+                    if (left >= PICK_STEPS) {
+                        float x[PICK_STEPS];
+    #pragma unroll
+                        for (unsigned int i = 0u; i < PICK_STEPS; ++i) x[i] = block[k & 1u][i][c];
+    #pragma unroll
+                        for (unsigned int i = 0u; i < PICK_STEPS; ++i) sum += x[i];
+                    } else {
+                        for (unsigned int i = 0u; i < left; ++i) sum += block[k & 1u][i][c];
+                    }
+                }
+            }
+        }
+        __syncthreads();
     }
+    if (tid < PICK_SUMS) a.sums[(unsigned long long)r * PICK_THREADS + col] = sum;
     __syncthreads();
     unsigned int *h = a.hist + (unsigned long long)r * PICK_BUCKETS;
-    for (unsigned int i = tid; i < PICK_BUCKETS; i += PICK_THREADS)
-        if (bucket[i] != 0u) atomicAdd(h + i, bucket[i]);
+    for (unsigned int i = tid; i < PICK_BUCKETS; i += PICK_THREADS) {
+        const unsigned int n = bucket[0][i] + bucket[1][i] + bucket[2][i] + bucket[3][i];
+        if (n != 0u) atomicAdd(h + i, n);
+    }
 }
 
+/* The cut over a band's counts, by the first 64 threads of a workgroup: the reference goes
+ * down from the highest bucket and stops at the one with which more than AOTX_MODEL_PICK_MAX
+ * values would be held; the cut is that bucket's upper end, and when nothing is held yet the
+ * band narrows to the bucket. Lane l holds buckets 4l .. 4l + 3. */
+static __device__ __forceinline__ void aotx_pick_cut(const unsigned int *bucket, float lo, float band, float &cut,
+                                                     unsigned int &more, float &lo2)
+{
+    static_assert(PICK_BUCKETS == 256u, "four buckets per lane");
+    const unsigned int lane = threadIdx.x;
+    unsigned int n[4], above = 0u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        n[i] = bucket[4u * lane + (unsigned int)i];
+        above += n[i];
+    }
+    /* the counts of this lane's buckets and all higher ones */
+#pragma unroll
+    for (unsigned int d = 1u; d < 64u; d <<= 1) {
+        const unsigned int o = __shfl_down(above, d, 64);
+        if (lane + d < 64u) above += o;
+    }
+    /* this lane's highest bucket with which more than the most are held, if any */
+    unsigned int held = above - n[0] - n[1] - n[2] - n[3], b = 0u, before = 0u;
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+        if (b == 0u && held + n[i] > AOTX_MODEL_PICK_MAX) {
+            b = 4u * lane + (unsigned int)i + 1u;
+            before = held;
+        }
+        held += n[i];
+    }
+    const unsigned long long any = __ballot(b != 0u);
+    if (any == 0ull) {
+        cut = lo;
+        more = 0u;
+        return;
+    }
+    const int from = 63 - __builtin_clzll(any);
+    b = (unsigned int)__shfl((int)b, from, 64);
+    before = (unsigned int)__shfl((int)before, from, 64);
+    cut = lo + band * (float)b / (float)PICK_BUCKETS;
+    more = before == 0u ? 1u : 0u;
+    lo2 = lo + band * (float)(b - 1u) / (float)PICK_BUCKETS;
+}
+
+/* A word another workgroup (on another XCD, past its L2) wrote or will read. */
+static __device__ __forceinline__ void aotx_pick_put(unsigned int *p, unsigned int v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+static __device__ __forceinline__ unsigned int aotx_pick_get(const unsigned int *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* PICK_SLICES workgroups per row: each finds the cut from the first pass's counts and puts
+ * the candidates of its slice in the row's list; the last one done picks. (The sort orders
+ * candidates by (value, id), a total order, so their places in the list do not matter.) When
+ * one bucket holds too many (logits equal to within 0.16, the reference's second pass) or the
+ * candidates exceed their places, the last one goes through the whole row instead. Bound by
+ * its chain of memory round trips (counts, candidates, arrivals, lists) and the ordered sums. */
 __global__ __launch_bounds__(PICK_THREADS) void aotx_pick_kernel(aotx_pick_args a)
 {
-    __shared__ float part[PICK_THREADS];
     __shared__ unsigned int mark[PICK_THREADS];
     __shared__ unsigned int bucket[PICK_BUCKETS];
-    __shared__ float value[AOTX_MODEL_PICK_MAX];
-    __shared__ unsigned int index[AOTX_MODEL_PICK_MAX];
-    __shared__ float t_min[AOTX_MODEL_PICK_MAX], t_mass[AOTX_MODEL_PICK_MAX], t_heat[AOTX_MODEL_PICK_MAX];
+    __shared__ __attribute__((aligned(16))) float value[AOTX_MODEL_PICK_MAX];
+    __shared__ __attribute__((aligned(16))) unsigned int index[AOTX_MODEL_PICK_MAX];
+    __shared__ __attribute__((aligned(16))) float t_min[AOTX_MODEL_PICK_MAX], t_mass[AOTX_MODEL_PICK_MAX], t_heat[AOTX_MODEL_PICK_MAX];
     __shared__ float s_top, s_sum, s_cut, s_lo, s_hi;
-    __shared__ unsigned int s_more, s_position, s_slot;
+    __shared__ unsigned int s_more, s_position, s_slot, s_last;
 
     const unsigned int tid = threadIdx.x;
-    const unsigned int r = blockIdx.x;
+    const unsigned int r = blockIdx.y;
+    const unsigned int slice = blockIdx.x;
     const aotx_model_run *run = a.run;
     unsigned int rows = run ? run->rows : (a.rows_dev ? *a.rows_dev : a.rows);
     int *token_out = run ? run->token : a.token;
@@ -278,145 +397,155 @@ __global__ __launch_bounds__(PICK_THREADS) void aotx_pick_kernel(aotx_pick_args 
         min_p = how[r].min_p;
     }
 
-    /* largest logit and its place, from the slices of aotx_argmax_kernel */
-    if (tid < 64u) {
+    if (warmth <= 0.0f) {
+        /* the largest logit's place, from the slices of aotx_argmax_kernel */
+        if (slice != 0u || tid >= 64u) return;
         float best;
         unsigned int at;
         aotx_pick_top(a, r, best, at);
         if (tid == 0u) {
+            const unsigned int drawn = atomicAdd(&a.state->draw[agent], 1u);
+            if (draw_out != nullptr) draw_out[r] = drawn;
+            token_out[r] = (int)at;
+        }
+        return;
+    }
+    /* the largest logit, and the cut; the row's sum in thread order by a lane of the last
+     * slice, published like the candidates */
+    bucket[tid] = a.hist[(unsigned long long)r * PICK_BUCKETS + tid];
+    if (slice == PICK_SLICES - 1u) t_mass[tid] = a.sums[(unsigned long long)r * PICK_THREADS + tid];
+    if (tid == 0u) s_slot = 0u;
+    __syncthreads();
+    if (tid < 64u) {
+        float best;
+        unsigned int at;
+        aotx_pick_top(a, r, best, at);
+        float cut = 0.0f, lo2 = 0.0f;
+        unsigned int more = 0u;
+        aotx_pick_cut(bucket, -AOTX_MODEL_PICK_SPAN, AOTX_MODEL_PICK_SPAN, cut, more, lo2);
+        if (tid == 0u) {
             s_top = best;
-            mark[0] = at;
-            s_position = atomicAdd(&a.state->draw[agent], 1u);
-            if (draw_out != nullptr) draw_out[r] = s_position;
+            s_cut = cut;
+            s_more = more;
+            s_lo = lo2;
+            s_hi = cut;
         }
     }
     __syncthreads();
     const float top = s_top;
-    const unsigned int position = s_position;
-    if (warmth <= 0.0f) {
-        if (tid == 0u) token_out[r] = (int)mark[0];
-        return;
-    }
-
-    /* the row sum of exp(v - top) in the reference's order (thread t: tokens t, t + 256,
-     * ...; then thread 0 over the threads), from the stored exponentials */
-    const float *ex = a.ex + (unsigned long long)r * vocab;
-    float row_total = 0.0f;
-#pragma unroll 64
-    for (unsigned int i = tid; i < vocab; i += PICK_THREADS) row_total += ex[i];
-    part[tid] = row_total;
-    /* the first pass's counts, handed back to zero for the next call */
-    unsigned int *h = a.hist + (unsigned long long)r * PICK_BUCKETS;
-    for (unsigned int i = tid; i < PICK_BUCKETS; i += PICK_THREADS) {
-        bucket[i] = h[i];
-        h[i] = 0u;
-    }
-    __syncthreads();
-
-    /* bucket search for the cut: pass 0 counted by aotx_pick_exp_kernel, later passes
-     * here over the narrowed band */
-    float lo = -AOTX_MODEL_PICK_SPAN;
-    float hi = 0.0f;
-    for (unsigned int pass = 0u; pass < PICK_PASSES; ++pass) {
-        float band = hi - lo;
-        if (pass != 0u) {
-            for (unsigned int i = tid; i < PICK_BUCKETS; i += PICK_THREADS) bucket[i] = 0u;
-            __syncthreads();
-            /* counts: any order, so 16-byte loads where the row allows */
-            const bool aligned = ((unsigned long long)row & 15ull) == 0ull;
-            const unsigned int body = aligned ? vocab / 4u * 4u : 0u;
-            if (aligned) {
-                const float4 *row4 = (const float4 *)row;
-#pragma unroll 16
-                for (unsigned int i4 = tid; i4 < vocab / 4u; i4 += PICK_THREADS) {
-                    const float4 f = row4[i4];
-                    const float fs[4] = {f.x, f.y, f.z, f.w};
+    if (slice == PICK_SLICES - 1u && tid == PICK_THREADS - 1u) {
+        float sum = 0.0f;
+#pragma unroll 1
+        for (unsigned int h = 0u; h < PICK_THREADS; h += 64u) {
+            float x[64];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float scaled = fs[e] - top;
-                        if (scaled >= lo && scaled <= hi) {
-                            unsigned int b = (unsigned int)((scaled - lo) * (float)PICK_BUCKETS / band);
-                            if (b >= PICK_BUCKETS) b = PICK_BUCKETS - 1u;
-                            atomicAdd(&bucket[b], 1u);
-                        }
-                    }
-                }
-            }
-            for (unsigned int i = body + tid; i < vocab; i += PICK_THREADS) {
-                float scaled = row[i] - top;
-                if (scaled >= lo && scaled <= hi) {
-                    unsigned int b = (unsigned int)((scaled - lo) * (float)PICK_BUCKETS / band);
-                    if (b >= PICK_BUCKETS) b = PICK_BUCKETS - 1u;
-                    atomicAdd(&bucket[b], 1u);
-                }
-            }
-            __syncthreads();
+            for (int i = 0; i < 64; ++i) x[i] = t_mass[h + (unsigned int)i];
+#pragma unroll
+            for (int i = 0; i < 64; ++i) sum += x[i];
         }
-        if (tid == 0u) {
-            if (pass == 0u) {
-                float sum = 0.0f;
-#pragma unroll 16
-                for (unsigned int i = 0u; i < PICK_THREADS; ++i) sum += part[i];
-                s_sum = sum;
+        aotx_pick_put((unsigned int *)a.total + r, __float_as_uint(sum));
+    }
+    unsigned int *cand = a.cand + (unsigned long long)r * PICK_SLICES * AOTX_MODEL_PICK_MAX * 2u;
+    unsigned int *founds = a.found + r * PICK_SLICES;
+    const bool aligned = ((unsigned long long)row & 15ull) == 0ull;
+    if (s_more == 0u) {
+        /* this slice's candidates, into LDS and then into its list */
+        const float cut = s_cut;
+        const unsigned int span = ((vocab + PICK_SLICES - 1u) / PICK_SLICES + 3u) & ~3u;
+        const unsigned int b0 = slice * span < vocab ? slice * span : vocab;
+        const unsigned int b1 = b0 + span < vocab ? b0 + span : vocab;
+        const unsigned int body = aligned ? b0 + (b1 - b0) / 4u * 4u : b0;
+        const auto take = [&](float v, unsigned int i) {
+            const float scaled = v - top;
+            if (scaled >= cut) {
+                const unsigned int slot = atomicAdd(&s_slot, 1u);
+                if (slot < AOTX_MODEL_PICK_MAX) {
+                    value[slot] = scaled;
+                    index[slot] = i;
+                }
             }
-            unsigned int held = 0u;
-            s_more = 0u;
-            s_cut = lo;
+        };
 #pragma unroll 8
-            for (unsigned int b = PICK_BUCKETS; b != 0u; --b) {
-                if (held + bucket[b - 1u] > AOTX_MODEL_PICK_MAX) {
-                    s_cut = lo + band * (float)b / (float)PICK_BUCKETS;
-                    if (held == 0u) {
-                        s_more = 1u;
-                        s_lo = lo + band * (float)(b - 1u) / (float)PICK_BUCKETS;
-                        s_hi = s_cut;
-                    }
-                    break;
-                }
-                held += bucket[b - 1u];
-            }
+        for (unsigned int i = b0 + 4u * tid; i < body; i += 4u * PICK_THREADS) {
+            const float4 f = *(const float4 *)(row + i);
+            take(f.x, i);
+            take(f.y, i + 1u);
+            take(f.z, i + 2u);
+            take(f.w, i + 3u);
         }
+#pragma unroll 8
+        for (unsigned int i = body + tid; i < b1; i += PICK_THREADS) take(row[i], i);
         __syncthreads();
-        if (s_more == 0u) break;
-        lo = s_lo;
-        hi = s_hi;
-        __syncthreads();
+        const unsigned int n = s_slot < AOTX_MODEL_PICK_MAX ? s_slot : AOTX_MODEL_PICK_MAX;
+        unsigned int *list = cand + slice * AOTX_MODEL_PICK_MAX * 2u;
+        for (unsigned int i = tid; i < n; i += PICK_THREADS) {
+            aotx_pick_put(list + 2u * i, __float_as_uint(value[i]));
+            aotx_pick_put(list + 2u * i + 1u, index[i]);
+        }
+        if (tid == 0u) aotx_pick_put(founds + slice, s_slot);
     }
-
-    /* candidates at or above the cut. The sort below orders them by (value, id), a total
-     * order, so while they fit the 256 places their order of placement does not matter:
-     * one coalesced pass gives each the next free place (an LDS counter). Only when more
-     * pass the cut (logits equal to within the finest band, where the reference keeps
-     * whichever arrive first) are the 256 lowest token ids kept instead: each thread takes
-     * a contiguous run of tokens and a prefix over the threads places them in token order. */
-    const float cut = s_cut;
-    if (tid == 0u) s_slot = 0u;
+    /* what the slice published is out before it counts as done */
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    {
-        /* one coalesced pass: every candidate takes the next place while places remain */
-        const unsigned int v4 = vocab / 4u;
-        const float4 *row4 = (const float4 *)row;
-        const bool aligned = ((unsigned long long)row & 15ull) == 0ull;
-        const unsigned int body = aligned ? v4 * 4u : 0u;
-        if (aligned) {
-#pragma unroll 16
-            for (unsigned int i4 = tid; i4 < v4; i4 += PICK_THREADS) {
-                const float4 f = row4[i4];
-                const float fs[4] = {f.x, f.y, f.z, f.w};
+    if (tid == 0u) s_last = atomicAdd(a.seen + r, 1u) == PICK_SLICES - 1u ? 1u : 0u;
+    __syncthreads();
+    if (s_last == 0u) return;
+    /* the slices' counts; the row's draw and sum with them */
+    if (tid < PICK_SLICES) mark[tid] = s_more == 0u ? aotx_pick_get(founds + tid) : 0u;
+    if (tid == 64u) {
+        s_position = atomicAdd(&a.state->draw[agent], 1u);
+        if (draw_out != nullptr) draw_out[r] = s_position;
+    }
+    if (tid == 128u) {
+        s_sum = __uint_as_float(aotx_pick_get((const unsigned int *)a.total + r));
+        s_slot = 0u;
+    }
+    __syncthreads();
+    unsigned int found = 0u, in = 0u, mine_at = 0u;      /* thread t holds candidate t of the slices' in order */
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float scaled = fs[e] - top;
-                    if (scaled >= cut) {
-                        const unsigned int slot = atomicAdd(&s_slot, 1u);
-                        if (slot < AOTX_MODEL_PICK_MAX) {
-                            value[slot] = scaled;
-                            index[slot] = i4 * 4u + (unsigned int)e;
-                        }
-                    }
-                }
+    for (unsigned int i = 0u; i < PICK_SLICES; ++i) {
+        const unsigned int n = mark[i];
+        if (tid >= found) {
+            in = i;
+            mine_at = tid - found;
+        }
+        found += n;
+    }
+    if (s_more != 0u) {
+        /* the second pass of the cut search, over the band of one bucket */
+        const float lo = s_lo, hi = s_hi, band = hi - lo;
+        for (unsigned int i = tid; i < PICK_BUCKETS; i += PICK_THREADS) bucket[i] = 0u;
+        __syncthreads();
+#pragma unroll 16
+        for (unsigned int i = tid; i < vocab; i += PICK_THREADS) {
+            const float scaled = row[i] - top;
+            if (scaled >= lo && scaled <= hi) {
+                unsigned int b = (unsigned int)((scaled - lo) * (float)PICK_BUCKETS / band);
+                if (b >= PICK_BUCKETS) b = PICK_BUCKETS - 1u;
+                atomicAdd(&bucket[b], 1u);
             }
         }
-        for (unsigned int i = body + tid; i < vocab; i += PICK_THREADS) {
+        __syncthreads();
+        if (tid < 64u) {
+            float cut = 0.0f, lo2 = 0.0f;
+            unsigned int more = 0u;
+            aotx_pick_cut(bucket, lo, band, cut, more, lo2);
+            if (tid == 0u) s_cut = cut;
+        }
+    }
+    __syncthreads();
+    const float cut = s_cut;
+    if (s_more == 0u && found <= AOTX_MODEL_PICK_MAX) {
+        if (tid < found) {
+            const unsigned int *one = cand + (in * AOTX_MODEL_PICK_MAX + mine_at) * 2u;
+            value[tid] = __uint_as_float(aotx_pick_get(one));
+            index[tid] = aotx_pick_get(one + 1u);
+        }
+        if (tid == 0u) s_slot = found;
+    } else {
+        /* the whole row: every candidate takes the next place while places remain */
+#pragma unroll 16
+        for (unsigned int i = tid; i < vocab; i += PICK_THREADS) {
             const float scaled = row[i] - top;
             if (scaled >= cut) {
                 const unsigned int slot = atomicAdd(&s_slot, 1u);
@@ -429,9 +558,10 @@ __global__ __launch_bounds__(PICK_THREADS) void aotx_pick_kernel(aotx_pick_args 
     }
     __syncthreads();
     unsigned int count = s_slot;
-    if (count <= AOTX_MODEL_PICK_MAX) {
-        /* all placed */
-    } else {
+    if (count > AOTX_MODEL_PICK_MAX) {
+        /* more than the places (logits equal to within the finest band, where the reference
+         * keeps whichever arrive first): the lowest token ids are kept. Each thread takes a
+         * contiguous run of tokens and a prefix over the threads places them in order. */
         const unsigned int per = (vocab + PICK_THREADS - 1u) / PICK_THREADS;
         const unsigned int first = tid * per;
         const unsigned int after = first + per < vocab ? first + per : vocab;
@@ -464,89 +594,91 @@ __global__ __launch_bounds__(PICK_THREADS) void aotx_pick_kernel(aotx_pick_args 
         }
         count = AOTX_MODEL_PICK_MAX;
     }
-    for (unsigned int i = tid; i < AOTX_MODEL_PICK_MAX; i += PICK_THREADS) {
-        if (i >= count) {
-            value[i] = -INFINITY;
-            index[i] = 0xFFFFFFFFu;
-        }
+    /* largest first, ties to the lower id: a thread per candidate counts those ahead of it (a
+     * total order, so the counts are the places). The terms of each candidate are the
+     * expressions of the reference's serial loops; the places past the count hold nothing. */
+    static_assert(PICK_THREADS == AOTX_MODEL_PICK_MAX, "a thread per candidate");
+    if (tid >= count) {
+        value[tid] = -INFINITY;
+        index[tid] = 0xFFFFFFFFu;
     }
     __syncthreads();
-
-    /* bitonic sort, largest first, ties to the lower id */
-    for (unsigned int span = 2u; span <= AOTX_MODEL_PICK_MAX; span <<= 1) {
-        for (unsigned int step = span >> 1; step != 0u; step >>= 1) {
-            unsigned int i = tid;
-            unsigned int other = i ^ step;
-            if (other > i && i < AOTX_MODEL_PICK_MAX) {
-                bool down = (i & span) == 0u;
-                float vi = value[i], vo = value[other];
-                unsigned int ii = index[i], io = index[other];
-                bool o_first = vo > vi || (vo == vi && io < ii);  /* other ranks ahead */
-                bool i_first = vi > vo || (vi == vo && ii < io);
-                bool swap = down ? o_first : i_first;
-                if (swap) {
-                    value[i] = vo;
-                    index[i] = io;
-                    value[other] = vi;
-                    index[other] = ii;
-                }
-            }
-            __syncthreads();
+    const float mine = value[tid];
+    const unsigned int my_id = index[tid];
+    unsigned int place = tid;
+    if (tid < count) {
+        place = 0u;
+#pragma unroll 4
+        for (unsigned int j = 0u; j < count; j += 4u) {
+            const float4 v = *(const float4 *)(value + j);
+            const uint4 o = *(const uint4 *)(index + j);
+            place += v.x > mine || (v.x == mine && o.x < my_id) ? 1u : 0u;
+            place += v.y > mine || (v.y == mine && o.y < my_id) ? 1u : 0u;
+            place += v.z > mine || (v.z == mine && o.z < my_id) ? 1u : 0u;
+            place += v.w > mine || (v.w == mine && o.w < my_id) ? 1u : 0u;
         }
+        if (place == 0u) s_lo = mine;
     }
-    /* the per-candidate terms of the serial loops below, each the same expression as
-     * there, computed by all threads; thread 0 then adds them in candidate order */
+    __syncthreads();
+    const float v0 = s_lo;
     const float heat = warmth;
-    {
-        const float v0 = value[0];
-        const float total = s_sum;
-        for (unsigned int i = tid; i < AOTX_MODEL_PICK_MAX; i += PICK_THREADS) {
-            t_min[i] = expf(value[i] - v0);
-            t_mass[i] = expf(value[i]) / total;
-            t_heat[i] = expf((value[i] - v0) / heat);
+    index[place] = my_id;
+    t_min[place] = expf(mine - v0);
+    t_mass[place] = expf(mine) / s_sum;
+    t_heat[place] = expf((mine - v0) / heat);
+    __syncthreads();
+    /* the running sums of the masses and of the tempered terms in candidate order, by a lane
+     * of two waves each: what the serial walks hold after each candidate */
+    if (tid == 0u || tid == 64u) {
+        float *t = tid == 0u ? t_mass : t_heat;
+        float sum = 0.0f;
+#pragma unroll 1
+        for (unsigned int h = 0u; h < count; h += 64u) {
+            float x[64];
+#pragma unroll
+            for (int i = 0; i < 64; ++i) x[i] = t[h + (unsigned int)i];
+#pragma unroll
+            for (int i = 0; i < 64; ++i) {
+                sum += x[i];
+                x[i] = sum;
+            }
+#pragma unroll
+            for (int i = 0; i < 64; ++i) t[h + (unsigned int)i] = x[i];
         }
     }
     __syncthreads();
-    if (tid != 0u) return;
-
+    /* the walks: the first candidate at which each stops, over lane-parallel tests (thread i
+     * tests candidate i) */
+    const auto first = [&](bool stop, unsigned int none) {
+        const unsigned long long at = __ballot(stop);
+        if ((tid & 63u) == 0u) mark[tid >> 6] = at != 0ull ? tid + (unsigned int)__builtin_ctzll(at) : 0xFFFFFFFFu;
+        __syncthreads();
+        unsigned int f = mark[0];
+#pragma unroll
+        for (unsigned int w = 1u; w < PICK_THREADS / 64u; ++w) f = mark[w] < f ? mark[w] : f;
+        __syncthreads();
+        return f < none ? f : none;
+    };
     unsigned int keep = (want_k == 0u || want_k > count) ? count : want_k;
-    if (min_p > 0.0f && min_p <= 1.0f) {
-        unsigned int min_keep = 1u;
-        for (unsigned int i = 1u; i < keep; ++i) {
-            if (t_min[i] < min_p) break;
-            min_keep = i + 1u;
-        }
-        keep = min_keep;
-    }
-    float limit = (want_p <= 0.0f || want_p > 1.0f) ? 1.0f : want_p;
-    float mass = 0.0f;
-    unsigned int taken = 0u;
-#pragma unroll 8
-    for (unsigned int i = 0u; i < keep; ++i) {
-        mass += t_mass[i];
-        taken = i + 1u;
-        if (mass >= limit) break;
-    }
-    float heat_total = 0.0f;
-#pragma unroll 8
-    for (unsigned int i = 0u; i < taken; ++i) heat_total += t_heat[i];
-    aotx_u32x4 word = aotx_philox_dev(position, 0u, 0u, agent, (unsigned int)stream,
-                                      (unsigned int)(stream >> 32));
-    float pick = (float)(word.x >> 8) * (1.0f / 16777216.0f) * heat_total;
-    float walk = 0.0f;
-    unsigned int chosen = index[0];
-    for (unsigned int i = 0u; i < taken; ++i) {
-        walk += t_heat[i];
-        chosen = index[i];
-        if (walk >= pick) break;
-    }
-    token_out[r] = (int)chosen;
+    if (min_p > 0.0f && min_p <= 1.0f)         /* up to the first below it, the largest always */
+        keep = first(tid >= 1u && tid < keep && t_min[tid] < min_p, keep > 1u ? keep : 1u);
+    const float limit = (want_p <= 0.0f || want_p > 1.0f) ? 1.0f : want_p;
+    /* up to and with the first at which the mass reaches the limit */
+    const unsigned int reached = first(tid < keep && t_mass[tid] >= limit, keep);
+    const unsigned int taken = reached < keep ? reached + 1u : keep;
+    const float heat_total = taken != 0u ? t_heat[taken - 1u] : 0.0f;
+    const aotx_u32x4 word = aotx_philox_dev(s_position, 0u, 0u, agent, (unsigned int)stream,
+                                            (unsigned int)(stream >> 32));
+    const float pick = (float)(word.x >> 8) * (1.0f / 16777216.0f) * heat_total;
+    const unsigned int chosen = first(tid < taken && t_heat[tid] >= pick, taken != 0u ? taken - 1u : 0u);
+    if (tid == 0u) token_out[r] = (int)index[chosen];
 }
 
 size_t aotx_pick_scratch(unsigned int rows, unsigned int vocab)
 {
-    return (size_t)rows * (PICK_CHUNKS * 2u + PICK_BUCKETS) * sizeof(unsigned int)
-         + (size_t)rows * vocab * sizeof(float);
+    (void)vocab;
+    return (size_t)rows * (PICK_CHUNKS * 2u + PICK_BUCKETS + PICK_THREADS + PICK_SLICES * (AOTX_MODEL_PICK_MAX * 2u + 1u)
+                           + 2u) * sizeof(unsigned int);
 }
 
 void aotx_launch_pick(const float *logits, unsigned int ld, unsigned int vocab,
@@ -574,12 +706,16 @@ void aotx_launch_pick(const float *logits, unsigned int ld, unsigned int vocab,
     a.run = run;
     a.best = best;
     a.hist = best + (size_t)rows * PICK_CHUNKS * 2u;
-    a.ex = (float *)(a.hist + (size_t)rows * PICK_BUCKETS);
+    a.sums = (float *)(a.hist + (size_t)rows * PICK_BUCKETS);
+    a.cand = (unsigned int *)(a.sums + (size_t)rows * PICK_THREADS);
+    a.found = a.cand + (size_t)rows * PICK_SLICES * AOTX_MODEL_PICK_MAX * 2u;
+    a.seen = a.found + (size_t)rows * PICK_SLICES;
+    a.total = (float *)(a.seen + rows);
     hipLaunchKernelGGL(aotx_argmax_kernel, dim3(PICK_CHUNKS, rows), dim3(PICK_THREADS), 0, s, a);
     AOTX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(aotx_pick_exp_kernel, dim3(PICK_EXP_WGS, rows), dim3(PICK_THREADS), 0, s, a);
+    hipLaunchKernelGGL(aotx_pick_exp_kernel, dim3(PICK_THREADS / PICK_SUMS, rows), dim3(PICK_THREADS), 0, s, a);
     AOTX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(aotx_pick_kernel, dim3(rows), dim3(PICK_THREADS), 0, s, a);
+    hipLaunchKernelGGL(aotx_pick_kernel, dim3(PICK_SLICES, rows), dim3(PICK_THREADS), 0, s, a);
     AOTX_LAUNCH_CHECK();
 }
 

@@ -149,3 +149,32 @@ def test_pick_alternating_row_counts(torch, lib, orc):
             want = orc.pick(logits[i], 40, 0.9, 0.0, 0.8, 77, a, draws.get(a, 0))[0]
             draws[a] = draws.get(a, 0) + 1
             assert got[i] == want, (rows, vocab, i)
+
+
+@pytest.mark.parametrize("vocab", [1, 31, 257, 4095, 32001, 131071, 131073])
+def test_pick_edges_vs_oracle(torch, lib, orc, vocab):
+    """Rows whose ends fall inside the sums' blocks and the candidates' slices (a row is then
+    also off 16-byte alignment), rows of masked logits (the lowest fp32 value, -inf), and rows
+    with 255 to 258 values above the rest, at and past the candidates' 256 places."""
+    rng = np.random.default_rng(vocab)
+    rows = 9
+    logits = rng.normal(0, 2.0, (rows, vocab)).astype(np.float32)
+    logits[1, rng.random(vocab) < 0.9] = -np.inf
+    logits[2, rng.random(vocab) < 0.9] = np.finfo(np.float32).min
+    logits[1:3, vocab // 2] = 3.0
+    for i, n in enumerate((255, 256, 257, 258)):
+        at = rng.permutation(vocab)[:n]
+        logits[3 + i, at] = 20.0 + rng.random(len(at)).astype(np.float32) * 4.0
+    logits[7, :] = np.float32(0.5)                       # all equal
+    logits[8, :] = 0.25 + rng.random(vocab).astype(np.float32) * 0.1   # all inside one bucket
+    agent = np.arange(rows, dtype=np.uint32)
+    tok = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    for top_k, top_p, temp in ((40, 0.9, 0.8), (0, 1.0, 1.0), (0, 1.0, 0.0)):
+        lib.aotx_model_restream()
+        assert lib.aotx_pick(p(dev(logits, torch)), rows, vocab, p(dev(agent, torch)), None, top_k, top_p, temp,
+                             77, p(tok), None, None) == 0
+        torch.cuda.synchronize()
+        got = tok.cpu().numpy()
+        for r in range(rows):
+            want = orc.pick(logits[r], top_k, top_p, 0.0, temp, 77, int(agent[r]), 0)[0]
+            assert got[r] == want, (r, top_k, temp, got[r], want)
