@@ -163,51 +163,6 @@ static __device__ __forceinline__ unsigned int aotx_attn_chunk(unsigned int n, u
         }                                                                                   \
     } while (0)
 
-/* MMA_COMPUTE_SH(KL, VL, B, LIVE, ABS): MMA_COMPUTE over a block its workgroup staged in
- * LDS (keys at KL, values at VL, rows of VS halves); LIVE: the block is in this wave's
- * range; ABS: its page is missing. */
-#define MMA_COMPUTE_SH(KL, VL, B, LIVE, ABS)                                                \
-    do {                                                                                    \
-        aotx_f4a sc = {0.0f, 0.0f, 0.0f, 0.0f};                                             \
-        _Pragma("unroll") for (int kk = 0; kk < KK; ++kk)                                   \
-            sc = __builtin_amdgcn_mfma_f32_16x16x32_f16(                                    \
-                *(const aotx_h8a *)((KL) + r * VS + 32u * (unsigned int)kk + 8u * g), qb[kk], sc, 0, 0, 0); \
-        float pr[4];                                                                        \
-        float mb = -INFINITY;                                                               \
-        _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                     \
-            const unsigned int p = (B) * 16u + 4u * g + (unsigned int)i;                    \
-            const bool ok = (LIVE) && p >= p0 && p < plim && !(ABS);                        \
-            pr[i] = ok ? sc[i] * scale : -INFINITY;                                         \
-            mb = fmaxf(mb, pr[i]);                                                          \
-        }                                                                                   \
-        mb = fmaxf(mb, __shfl_xor(mb, 16, 64));                                             \
-        mb = fmaxf(mb, __shfl_xor(mb, 32, 64));                                             \
-        const float mnew = fmaxf(mrun, mb);                                                 \
-        const float shift = mnew == -INFINITY ? 1.0f : aotx_exp2(mrun - mnew);              \
-        mrun = mnew;                                                                        \
-        aotx_h4a pa;                                                                        \
-        float mass = 0.0f;                                                                  \
-        _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                     \
-            const _Float16 ph = mnew == -INFINITY ? (_Float16)0.0f                          \
-                              : (_Float16)aotx_exp2(pr[i] - mnew);                          \
-            pa[i] = ph;                                                                     \
-            mass += (float)ph;                                                              \
-        }                                                                                   \
-        lrun = lrun * shift + mass;                                                         \
-        if (__any(shift != 1.0f)) {                                                         \
-            float sh[4];                                                                    \
-            _Pragma("unroll") for (int i = 0; i < 4; ++i) sh[i] = __shfl(shift, (int)(4u * g) + i, 64); \
-            _Pragma("unroll") for (int cc = 0; cc < NS; ++cc)                               \
-                _Pragma("unroll") for (int i = 0; i < 4; ++i) o[cc][i] *= sh[i];            \
-        }                                                                                   \
-        _Pragma("unroll") for (int cc = 0; cc < NS; ++cc) {                                 \
-            const aotx_s4a t4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(                    \
-                (__attribute__((address_space(3))) aotx_s4a *)((VL) + vtr + 16u * (unsigned int)cc)); \
-            o[cc] = __builtin_amdgcn_mfma_f32_16x16x16f16(pa, __builtin_bit_cast(aotx_h4a, t4), \
-                                                          o[cc], 0, 0, 0);                  \
-        }                                                                                   \
-    } while (0)
-
 /* One workgroup = W waves = one (token, KV head, context chunk); each wave takes a
  * contiguous run of 16-position layout blocks. Per wave and block, on the matrix cores:
  *   - scores S[pos][head] = K . q^T: one v_mfma_f32_16x16x32_f16 per 32 of d, keys as the A
@@ -442,288 +397,410 @@ static __device__ __forceinline__ void aotx_attend_body(const aotx_attn_args &a,
     }
 }
 
-/* Prompt pieces two waves each: a workgroup of W = 8 waves takes the pieces led inside its
- * range of AOTX_RUN_RANGE tokens (a piece: up to QT = 16 / G consecutive queries of one
- * sequence, led by a token that starts its sequence's run in the batch or sits at a
- * multiple of QT, as in the decode body's prompt pieces), in rounds of 4 in rank order.
- * Wave k < 4 runs one ordered pass of online softmax (the reference's pass per query,
- * cuda/model/attention.cu:22-154) over the first half of the blocks its round's piece sees,
- * wave k + 4 over the second half; the second half's maxima, masses and accumulators pass
- * through LDS and the first wave adds them in block order and writes the outputs. When
- * a round's pieces are all of one sequence, the halves split the blocks of its longest
- * piece instead, and each half's four waves load every block once, into LDS (double
- * buffered, one barrier per block), where all four read their keys and values; otherwise
- * each wave loads its own blocks (the same blocks as its neighbours, from the caches). */
-#define AOTX_RUN_RANGE 16u
-template <int D, int G, int W>
+/* The largest of a value over the four lanes r, r + 16, r + 32 and r + 48. */
+static __device__ __forceinline__ float aotx_attn_max4(float v)
+{
+    typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+    const unsigned int w = __builtin_bit_cast(unsigned int, v);
+    const u2 a = __builtin_bit_cast(u2, __builtin_amdgcn_permlane32_swap(w, w, false, false));
+    const unsigned int a0 = a.x, a1 = a.y;
+    const float m = fmaxf(__builtin_bit_cast(float, a0), __builtin_bit_cast(float, a1));
+    const unsigned int x = __builtin_bit_cast(unsigned int, m);
+    const u2 b = __builtin_bit_cast(u2, __builtin_amdgcn_permlane16_swap(x, x, false, false));
+    const unsigned int b0 = b.x, b1 = b.y;
+    return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
+}
+
+/* Batches with prompt pieces: a workgroup takes 16 NC H score columns of a KV head, the G
+ * query heads of 16 NC H / G consecutive tokens. Its 4 H waves are H halves of the columns (NC
+ * tiles of 16 each) times 4 parts of the positions: part k takes every fourth pair of
+ * 16-position blocks, the parts are added at the end, in part order. Per pair of blocks and
+ * tile:
+ *   - scores: keys as the A operand, 16 positions by 16 columns per MFMA as in the decode body;
+ *   - the largest score over the 32 positions by four lane groups (row swaps, no LDS); the
+ *     weights 2^(score - max) round to fp16 in the A layout of v_mfma_f32_16x16x32_f16, block
+ *     0's positions 4g .. 4g + 3 and then block 1's, and the values come from LDS in that order
+ *     (two transposing reads, shared by the tiles);
+ *   - the mass is the product of the same fp16 weights with ones, on the matrix core, where it
+ *     has the rows of the accumulators.
+ * With one half (H = 1) a wave loads its pairs by itself, keys into registers and values
+ * through its own LDS slot, and waits for no other wave. With two (H = 2) the halves of a part
+ * load a block of the pair each into LDS for both, double-buffered, one barrier per pair: half
+ * the reads from the L2s, which bound many columns otherwise. The next pair is on its way while
+ * one is computed. The columns may be of several sequences: the workgroup goes over the blocks
+ * of one after the other, and a column that does not take part keeps its state.
+ * Bound by the softmax's vector work and the matrix work of a step, about 1600 cycles a wave.
+ * Against a wave per 16 / G queries with one block per pass of softmax, at 32 / 8 heads x 128:
+ * 512 tokens after 2000 cached ones 74.3 -> 42.8 us (H = 2; 55 with H = 1), a 512-token prompt
+ * 21.7 -> 15.6, 256 tokens 14.6 -> 9.6, 128 tokens 10.8 -> 6.9, 200 tokens after 7800
+ * 210 -> 78. Four tiles per wave at one wave per SIMD took 64 us in the first case. */
+template <int D, int G, int NC, int H>
 static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a, unsigned int bx)
 {
-    constexpr int QT = 16 / G;
-    constexpr int KK = D / 32;
-    constexpr int VP = D / 32;
-    constexpr int NS = D / 16;
-    constexpr int VS = D + 8;
-    constexpr unsigned int RANGE = AOTX_RUN_RANGE;
-    constexpr unsigned int WP = 4u;                 /* waves of a round, a piece each */
-    static_assert(W == 2 * (int)WP, "two waves per piece: the halves of its blocks");
-    static_assert(RANGE + QT <= 64u, "one lane per token word");
-    __shared__ __attribute__((aligned(16))) unsigned short vl[W][16 * VS];
-    /* the second half's column maxima, masses, page-fault flag and accumulators (by lane) */
-    __shared__ float hm[WP][16], hl[WP][16];
-    __shared__ int hmiss[WP];
-    __shared__ float ho[WP][NS][4][64];
-    __shared__ unsigned int rag[WP], rn[WP];
+    constexpr int KK = D / 32;                      /* score MFMA steps */
+    constexpr int NS = D / 16;                      /* d slices of the accumulators */
+    constexpr int VP = D / 32;                      /* 16-byte pieces per lane and block */
+    constexpr int VS = D + 8;                       /* LDS row stride (halves) */
+    constexpr unsigned int TW = 16u * NC * H / G;   /* tokens */
+    constexpr unsigned int PARTS = 4u;
+    constexpr unsigned int COLS = 16u * NC;         /* columns of a half */
+    constexpr int NP = NS / (int)PARTS;             /* d slices that a part adds up */
+    static_assert(TW >= 1u && TW <= 64u && NS % (int)PARTS == 0, "a lane per token, a slice per part");
+    /* H = 1: the waves' value slots; H = 2: [buffer][part][keys, values] of a pair; after the
+     * loop the waves' accumulators */
+    constexpr unsigned int ROWS = 32u * VS * 2u, ACC = COLS * D * 4u;
+    constexpr unsigned int STAGE = H == 1 ? PARTS * ROWS : 2u * PARTS * 2u * ROWS;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[STAGE > H * PARTS * ACC ? STAGE : H * PARTS * ACC];
+    __shared__ float pm[H][PARTS][COLS], pl[H][PARTS][COLS];
+    __shared__ unsigned int pmiss[H][PARTS][NC];
 
     const unsigned int lane = threadIdx.x & 63u;
-    const unsigned int wave = threadIdx.x >> 6;
-    const unsigned int wp = wave % WP, half = wave / WP;
+    /* a scalar, so that the wave's blocks, loads and tests are scalar too */
+    const unsigned int wave = (unsigned int)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const unsigned int part = wave % PARTS, half = H == 1 ? 0u : wave / PARTS;
     const unsigned int r = lane & 15u, g = lane >> 4;
     const unsigned int counted = aotx_attn_scalar(a.m_dev != nullptr ? a.m_dev : a.pos);
     unsigned int tokens = a.m_dev != nullptr ? counted : a.tokens;
     if (tokens > a.tokens) tokens = a.tokens;
     const unsigned int kh = bx % a.kv_heads;
-    const unsigned int r0 = (bx / a.kv_heads) * RANGE;
-    if (r0 >= tokens) return;
-    /* one round trip: lane i holds the slot and position of token r0 - 1 + i (a token
-     * before the batch or past it holds no slot: all ones) */
-    const unsigned int ti = r0 + lane - 1u;
-    unsigned int ag = 0xFFFFFFFFu, ps = 0u;
-    if (lane < RANGE + (unsigned int)QT && (lane != 0u || r0 != 0u) && ti < tokens) {
-        ag = a.agent[ti];
-        ps = a.pos[ti];
-    }
-    const unsigned int ag_prev = (unsigned int)__shfl((int)ag, (int)((lane - 1u) & 63u), 64);
-    const bool lead = lane >= 1u && lane <= RANGE && ti < tokens
-                   && (ag != ag_prev || ps % (unsigned int)QT == 0u);
-    const unsigned long long leaders = (unsigned long long)__ballot(lead) >> 1;   /* bit j: token r0 + j */
-    /* the same in every wave (one ballot over the same words), so every wave runs the same
-     * rounds and meets the same barriers */
-    const unsigned int npieces = (unsigned int)__builtin_popcountll(leaders);
+    const unsigned int t0 = (bx / a.kv_heads) * TW;             /* the workgroup's first token */
+    if (t0 >= tokens) return;
+    /* lane i holds the slot and position of token t0 + i */
+    const bool live = lane < TW && t0 + lane < tokens;
+    const unsigned int tl = live ? t0 + lane : t0;
+    const unsigned int ag = a.agent[tl], ps = a.pos[tl];
+    const unsigned long long all = __ballot(live);
+    unsigned long long left = all;
 
+    const unsigned int c0 = half * COLS;                        /* this half's first column */
+    aotx_h8a qb[NC][KK];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const unsigned int col = c0 + 16u * (unsigned int)c + r;
+        const unsigned int tc = col / (unsigned int)G, hh = col % (unsigned int)G;
+        /* a column past the batch reads its last token's query (its results are not written) */
+        const unsigned int tq = t0 + tc < tokens ? t0 + tc : tokens - 1u;
+        const unsigned short *q = a.q + ((unsigned long long)tq * a.heads + kh * G + hh) * D + 8u * g;
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) qb[c][kk] = __builtin_bit_cast(aotx_h8a, co_load4(q + 32 * kk));
+    }
     const aotx_kv_table *kv = &a.state->kv;
     const float scale = 1.4426950408889634f / sqrtf((float)D);
-    const unsigned int kbyte = ((kh * AOTX_KVL_BLOCK + r) * D + 8u * g) * 2u;
-    const unsigned int vbyte = ((a.kv_heads + kh) * AOTX_KVL_BLOCK * D + lane * 8u) * 2u;
-    unsigned short *vw = vl[wave];
-    /* ds_read_tr16_b64: lane j of a 16-lane group gets halves j % 4 of the chunks that
-     * lanes 4e + j / 4 address, e = 0..3; lane (r, g) = 16 g + 4 i + q addresses row 4g + i,
-     * halves 4q..4q+3 of a 16-column slice, so that it gets column r of rows 4g..4g+3 */
+    const unsigned int kbyte = ((kh * AOTX_KVL_BLOCK + r) * D + 8u * g) * 2u;          /* A operand */
+    const unsigned int kbase = (kh * AOTX_KVL_BLOCK * D + lane * 8u) * 2u;             /* whole rows */
+    const unsigned int vbase = ((a.kv_heads + kh) * AOTX_KVL_BLOCK * D + lane * 8u) * 2u;
+    /* the transposing read of a block's slice (see aotx_attend_body) */
     const unsigned int vtr = (4u * g + (lane & 15u) / 4u) * VS + 4u * (lane & 3u);
-    constexpr int CPOL = 0;
 
-    for (unsigned int round = 0; round * WP < npieces; ++round) {
-        /* piece rank (in token order) round * WP + wp, its blocks split in two halves */
-        const unsigned int rank = round * WP + wp;
-        const bool have = rank < npieces;
-        unsigned long long lb = leaders;
-        for (unsigned int k = 0; k < rank && lb != 0ull; ++k) lb &= lb - 1ull;
-        const unsigned int j = have ? (unsigned int)__builtin_ctzll(lb) : 0u;
-        /* the piece led by token t = r0 + j (lane j + 1): the next tokens of its slot off a
-         * multiple of QT, up to QT in all */
-        const unsigned int lead_lane = j + 1u;
-        const unsigned int t = r0 + j;
-        const unsigned int agent = (unsigned int)__shfl((int)ag, (int)lead_lane, 64);
-        const bool cont = lane > lead_lane && lane < lead_lane + (unsigned int)QT && ag == agent
-                       && ps % (unsigned int)QT != 0u;
-        const unsigned long long cm = (unsigned long long)__ballot(cont) >> (lead_lane + 1u);
-        unsigned int nq = 1u + (unsigned int)__builtin_ctzll(~cm);
-        if (nq > (unsigned int)QT) nq = QT;
-        const unsigned int n = (unsigned int)__shfl((int)ps, (int)(lead_lane + nq - 1u), 64) + 1u;
-        /* this lane's column: query r / G; a column with no query sees position 0 only */
-        const unsigned int qpos = (unsigned int)__shfl((int)ps, (int)(lead_lane + r / (unsigned int)G), 64);
-        const unsigned int plim = r / (unsigned int)G < nq ? qpos + 1u : 1u;
-        const unsigned int p0 = 0u;
-        const unsigned int nb = (n + 15u) / 16u;
-        const unsigned int mid = (nb + 1u) / 2u;
-        const unsigned int b0 = half == 0u ? 0u : mid;
-        const unsigned int b1 = !have ? b0 : (half == 0u ? mid : nb);
+    float mrun[NC];                                  /* column 16c + r */
+    aotx_f4a o[NC][NS], mass[NC];                    /* columns 16c + 4g .. + 3 */
+    unsigned int miss[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        mrun[c] = -INFINITY;
+        miss[c] = 0u;
+        mass[c] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int cc = 0; cc < NS; ++cc) o[c][cc] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const _Float16 one = (_Float16)1.0f;
+    const aotx_h8a ones = {one, one, one, one, one, one, one, one};
 
-        float mrun = -INFINITY, lrun = 0.0f;
-        aotx_f4a o[NS];
+    while (left != 0ull) {
+        /* the tokens of one sequence, in any order of positions */
+        const unsigned int agent = (unsigned int)__builtin_amdgcn_readlane((int)ag, __builtin_ctzll(left));
+        const unsigned long long group = __ballot(ag == agent) & left;
+        const bool whole = group == all;                 /* the workgroup's only sequence */
+        left &= ~group;
+        /* the positions attended: by any token (n) and by every one (nmin) */
+        const bool in = (group >> lane) & 1ull;
+        unsigned int n = in ? ps + 1u : 0u, nmin = in ? ps + 1u : 0xFFFFFFFFu;
 #pragma unroll
-        for (int cc = 0; cc < NS; ++cc) o[cc] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
-        int missing = 0;
-        /* the round's sequences and lengths: when its pieces are of one sequence (every
-         * range of a prompt but those holding a sequence boundary), each half's four waves
-         * stage every block once in LDS and all read it there */
-        if (half == 0u && lane == 0u) {
-            rag[wp] = have ? agent : 0xFFFFFFFFu;
-            rn[wp] = have ? n : 0u;
+        for (int d = 32; d >= 1; d >>= 1) {
+            const unsigned int on = (unsigned int)__shfl_xor((int)n, d, 64), om = (unsigned int)__shfl_xor((int)nmin, d, 64);
+            n = on > n ? on : n;
+            nmin = om < nmin ? om : nmin;
         }
-        __syncthreads();
-        unsigned int sag = 0xFFFFFFFFu, nmax = 0u;
-        bool one = true;
+        n = (unsigned int)__builtin_amdgcn_readfirstlane((int)n);
+        nmin = (unsigned int)__builtin_amdgcn_readfirstlane((int)nmin);
+        unsigned int plim[NC];
 #pragma unroll
-        for (unsigned int i = 0; i < WP; ++i) {
-            const unsigned int ai = rag[i];
-            if (ai == 0xFFFFFFFFu) continue;
-            one = one && (sag == 0xFFFFFFFFu || sag == ai);
-            sag = ai;
-            nmax = rn[i] > nmax ? rn[i] : nmax;
+        for (int c = 0; c < NC; ++c) {
+            const unsigned int tc = (c0 + 16u * (unsigned int)c + r) / (unsigned int)G;
+            const unsigned int pt = (unsigned int)__shfl((int)ps, (int)tc, 64) + 1u;
+            plim[c] = (group >> tc) & 1ull ? pt : 0u;
         }
-        if (one && sag != 0xFFFFFFFFu) {
-            aotx_h8a qb[KK];
+        const unsigned int nblk = (n + 15u) / 16u, pairs = (nblk + 1u) / 2u;
+        unsigned long long pages = 0ull;
+        unsigned int wbase = 0u;
+        bool window = false;
+        /* the scalar resource of block BI (zero-size: loads return zeros) and whether it is
+         * missing; the window holds the addresses of 64 blocks, one per lane */
+        const auto block = [&](unsigned int bi, bool &gone) {
+            const unsigned int at = (bi - wbase) & 63u;
+            const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)(pages >> 32), (int)at);
+            const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)pages, (int)at);
+            const unsigned long long pb = ((unsigned long long)hi << 32) | lo;
+            gone = pb == 0ull && bi < nblk;
+            return __builtin_amdgcn_make_buffer_rsrc((void *)pb, (short)0, pb == 0ull ? 0 : (int)a.shape.block_bytes,
+                                                     0x00020000);
+        };
+        const auto look = [&](unsigned int pair) {
+            const unsigned int b0 = 2u * pair;
+            if (window && b0 + 1u - wbase < 64u) return;
+            window = true;
+            wbase = (unsigned int)__builtin_amdgcn_readfirstlane((int)b0);
+            const unsigned int bl = wbase + lane;
+            pages = bl < nblk ? (unsigned long long)aotx_kvl_block(a.shape, kv, agent, a.layer, bl * 16u) : 0ull;
+        };
+        /* scores of a pair's blocks to weights, mass and the shifted accumulators; then the
+         * values at vw */
+        const auto weigh = [&](aotx_f4a (&scs)[NC][2], const unsigned int p, const bool gone0, const bool gone1,
+                               const unsigned short *vw) {
+            const bool masked = !whole || 32u * p + 32u > nmin || gone0 || gone1;
+            /* two halves: the first half of the values is read before the softmax, the second
+             * before the first products (with one half it costs registers that spill) */
+            constexpr int EARLY = H == 2 ? NS / 2 : 0;
+            aotx_h8a vv[NS];
+            const auto values = [&](int cc) {
+                const aotx_s4a v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) aotx_s4a *)(vw + vtr + 16u * (unsigned int)cc));
+                const aotx_s4a v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) aotx_s4a *)(vw + 16u * VS + vtr + 16u * (unsigned int)cc));
+                vv[cc] = __builtin_bit_cast(aotx_h8a, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+            };
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                aotx_u4a w = {0u, 0u, 0u, 0u};
-                const unsigned int qi = r / (unsigned int)G, hh = r % (unsigned int)G;
-                if (have && qi < nq)
-                    w = co_load4(a.q + ((unsigned long long)(t + qi) * a.heads + kh * G + hh) * D
-                                     + 32 * kk + 8 * g);
-                qb[kk] = __builtin_bit_cast(aotx_h8a, w);
-            }
-            /* blocks [0, smid) to the first half, [smid, nbm) to the second; both halves
-             * run smid steps (the second's last one, when nbm is odd, adds nothing) */
-            const unsigned int nbm = (nmax + 15u) / 16u;
-            const unsigned int smid = (nbm + 1u) / 2u;
-            const unsigned int sb0 = half == 0u ? 0u : smid;
-            const unsigned int sb1 = half == 0u ? smid : nbm;
-            const unsigned int hid = wp * 64u + lane;          /* loader lane of the half */
-            constexpr unsigned int LP = (unsigned int)D / 64u;  /* 16-byte pieces per lane */
-            const unsigned int kbase = kh * AOTX_KVL_BLOCK * D * 2u;
-            const unsigned int vbase = (a.kv_heads + kh) * AOTX_KVL_BLOCK * D * 2u;
-            unsigned short *const sl = &vl[half * 4u][0];       /* [buf][K, V][16][VS] */
-            unsigned long long spages = 0ull;
-            unsigned int swbase = 0xFFFFFFFFu;
-            aotx_u4a ld[LP];
-            bool sabs[2] = {false, false};
-            bool labs = false;
-            /* block SB's keys and values into the registers ld (a block past the
-             * sequence's last reads the last one) */
-#define SH_LOAD(SB)                                                                         \
-            do {                                                                            \
-                const unsigned int bb_ = (SB) < nbm ? (SB) : nbm - 1u;                      \
-                if (swbase == 0xFFFFFFFFu || bb_ - swbase >= 64u) {                         \
-                    swbase = bb_;                                                           \
-                    const unsigned int bl_ = swbase + lane;                                 \
-                    spages = bl_ < nbm ? (unsigned long long)aotx_kvl_block(a.shape, kv, sag, a.layer, bl_ * 16u) \
-                                       : 0ull;                                              \
-                }                                                                           \
-                unsigned long long pb_ = __shfl(spages, (int)(bb_ - swbase), 64);           \
-                pb_ = ((unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((unsigned int)(pb_ >> 32)) << 32) \
-                    | (unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((unsigned int)pb_); \
-                labs = pb_ == 0ull;                                                         \
-                const __amdgpu_buffer_rsrc_t rs_ = __builtin_amdgcn_make_buffer_rsrc(       \
-                    (void *)pb_, (short)0, labs ? 0 : (int)a.shape.block_bytes, 0x00020000); \
-                _Pragma("unroll") for (unsigned int u = 0; u < LP; ++u) {                   \
-                    const unsigned int pc = hid + u * 256u;                                 \
-                    const unsigned int off = pc < 2u * D ? kbase + pc * 16u : vbase + (pc - 2u * D) * 16u; \
-                    ld[u] = __builtin_amdgcn_raw_buffer_load_b128(rs_, (int)off, 0, CPOL);  \
-                }                                                                           \
-            } while (0)
-            /* the registers into LDS buffer BUF (rows padded to VS halves) */
-#define SH_STORE(BUF)                                                                       \
-            do {                                                                            \
-                _Pragma("unroll") for (unsigned int u = 0; u < LP; ++u) {                   \
-                    const unsigned int pc = hid + u * 256u;                                 \
-                    const unsigned int isv = pc < 2u * D ? 0u : 1u;                         \
-                    const unsigned int e = pc - isv * 2u * D;                               \
-                    *(aotx_u4a *)(sl + ((BUF) * 2u + isv) * (16u * VS) + (e / (D / 8u)) * VS \
-                                  + (e % (D / 8u)) * 8u) = ld[u];                           \
-                }                                                                           \
-                sabs[BUF] = labs;                                                           \
-            } while (0)
-            SH_LOAD(sb0);
-            SH_STORE(0u);
-            __syncthreads();
-            for (unsigned int i = 0; i < smid; ++i) {
-                const unsigned int bcur = sb0 + i;
-                SH_LOAD(bcur + 1u);
-                const unsigned int cb = i & 1u;
-                const bool live = bcur < sb1;
-                if (have && live && sabs[cb] && bcur * 16u < n) missing = 1;
-                MMA_COMPUTE_SH(sl + (cb * 2u) * (16u * VS), sl + (cb * 2u + 1u) * (16u * VS), bcur,
-                               live, sabs[cb]);
-                if ((i & 1u) == 0u) SH_STORE(1u); else SH_STORE(0u);
-                __syncthreads();
-            }
-#undef SH_LOAD
-#undef SH_STORE
-        } else if (b0 < b1) {
-            aotx_h8a qb[KK];
+            for (int cc = 0; cc < EARLY; ++cc) values(cc);
+            if (H == 2) __builtin_amdgcn_sched_barrier(0);
+            aotx_h8a pa[NC];
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                aotx_u4a w = {0u, 0u, 0u, 0u};
-                const unsigned int qi = r / (unsigned int)G, hh = r % (unsigned int)G;
-                if (qi < nq)
-                    w = co_load4(a.q + ((unsigned long long)(t + qi) * a.heads + kh * G + hh) * D
-                                     + 32 * kk + 8 * g);
-                qb[kk] = __builtin_bit_cast(aotx_h8a, w);
+            for (int c = 0; c < NC; ++c) {
+                aotx_f4a *const sc = scs[c];
+                if (masked) {
+                    if (gone0 && 32u * p < plim[c]) miss[c] = 1u;
+                    if (gone1 && 32u * p + 16u < plim[c]) miss[c] = 1u;
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const unsigned int at = 32u * p + 16u * (unsigned int)e + 4u * g + (unsigned int)i;
+                            if (at >= plim[c] || (e == 0 ? gone0 : gone1)) sc[e][i] = -INFINITY;
+                        }
+                }
+                float mb = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])),
+                                 fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
+                mb = aotx_attn_max4(mb) * scale;
+                const float mnew = fmaxf(mrun[c], mb);
+                /* a column with no position yet: weights and shift of 0 from -inf */
+                const float msafe = mnew == -INFINITY ? 0.0f : mnew;
+                const bool moved = mnew != mrun[c];
+                const float shift = moved ? aotx_exp2(mrun[c] - msafe) : 1.0f;
+                mrun[c] = mnew;
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        pa[c][4 * e + i] = (_Float16)aotx_exp2(__builtin_fmaf(sc[e][i], scale, -msafe));
+                if (__any(moved)) {
+                    float sh[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) sh[i] = __shfl(shift, (int)(4u * g) + i, 64);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        mass[c][i] *= sh[i];
+#pragma unroll
+                        for (int cc = 0; cc < NS; ++cc) o[c][cc][i] *= sh[i];
+                    }
+                }
+                mass[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[c], ones, mass[c], 0, 0, 0);
             }
-            aotx_u4a kr[2][KK], vr[2][VP];
-            bool absent[2];
-            unsigned long long pages = 0ull;
-            unsigned int wbase = b0;
-            unsigned int b = b0;
-            MMA_WINDOW(b0);
-            MMA_LOAD(0, b);
-            for (;;) {
-                MMA_LOAD(1, b + 1u);
-                MMA_COMPUTE(0, b);
-                b += 1u;
-                if (b >= b1) break;
-                MMA_LOAD(0, b + 1u);
-                MMA_COMPUTE(1, b);
-                b += 1u;
-                if (b >= b1) break;
-            }
-        }
-        /* a head's mass over its 4 lane groups; column c's max and mass sit in lane c */
-        lrun += __shfl_xor(lrun, 16, 64);
-        lrun += __shfl_xor(lrun, 32, 64);
-        missing = __any(missing);
-        if (missing && lane == 0u) atomicAdd(&a.state->faults, 1u);
-        if (half == 1u) {
-            if (lane < 16u) {
-                hm[wp][lane] = mrun;
-                hl[wp][lane] = lrun;
-            }
-            if (lane == 0u) hmiss[wp] = missing;
+#pragma unroll
+            for (int cc = EARLY; cc < NS; ++cc) values(cc);
+            if (H == 2) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int cc = 0; cc < NS; ++cc)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) ho[wp][cc][i][lane] = o[cc][i];
-        }
-        __syncthreads();
-        if (have && half == 0u) {
-            /* the halves in block order: M = max(m0, m1), o = o0 2^(m0 - M) + o1 2^(m1 - M),
-             * the masses likewise (a half with no position yet has m = -inf: factor 0) */
-            const float m1 = hm[wp][r], l1 = hl[wp][r];
-            const float top = fmaxf(mrun, m1);
-            const float f0 = mrun == -INFINITY ? 0.0f : aotx_exp2(mrun - top);
-            const float f1 = m1 == -INFINITY ? 0.0f : aotx_exp2(m1 - top);
-            lrun = lrun * f0 + l1 * f1;
-            missing = missing || hmiss[wp] != 0;
+                for (int c = 0; c < NC; ++c)
+                    o[c][cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[c], vv[cc], o[c][cc], 0, 0, 0);
+        };
+        if constexpr (H == 1) {
+            unsigned short *const vw = (unsigned short *)(lds + part * ROWS);
+            aotx_u4a kr[2][KK], vr[2][VP];
+            bool gone[2] = {false, false};
+            const auto load = [&](unsigned int p) {
+                look(p);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned int col = 4u * g + (unsigned int)i;
-                const float c0 = __shfl(f0, (int)col, 64), c1 = __shfl(f1, (int)col, 64);
+                for (int e = 0; e < 2; ++e) {
+                    const __amdgpu_buffer_rsrc_t rs = block(2u * p + (unsigned int)e, gone[e]);
 #pragma unroll
-                for (int cc = 0; cc < NS; ++cc) o[cc][i] = o[cc][i] * c0 + ho[wp][cc][i][lane] * c1;
-            }
+                    for (int kk = 0; kk < KK; ++kk) kr[e][kk] = __builtin_amdgcn_raw_buffer_load_b128(rs, kbyte + kk * 64, 0, 0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned int col = 4u * g + (unsigned int)i;
-                const float l = __shfl(lrun, (int)col, 64);
-                const float back = !missing && l > 0.0f ? 1.0f / l : 0.0f;
-                const unsigned int qc = col / (unsigned int)G, hc = col % (unsigned int)G;
-#pragma unroll
-                for (int cc = 0; cc < NS; ++cc) {
-                    const float v = o[cc][i] * back;
-                    const float v1 = __shfl_down(v, 1, 64);
-                    if (qc < nq && (r & 1u) == 0u)
-                        co_store2h(a.out + aotx_attn_out_at(a, t + qc, kh * G + hc, 16u * cc + r, D),
-                                   aotx_f2h(v), aotx_f2h(v1));
+                    for (int u = 0; u < VP; ++u) vr[e][u] = __builtin_amdgcn_raw_buffer_load_b128(rs, vbase + u * 1024, 0, 0);
                 }
+            };
+            if (part < pairs) load(part);
+            for (unsigned int p = part; p < pairs; p += PARTS) {
+                aotx_f4a scs[NC][2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int u = 0; u < VP; ++u) {
+                        const unsigned int piece = (unsigned int)u * 64u + lane;
+                        *(aotx_u4a *)(vw + ((unsigned int)e * 16u + piece / (D / 8)) * VS + (piece % (D / 8)) * 8u) = vr[e][u];
+                    }
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) {
+                        scs[c][e] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int kk = 0; kk < KK; ++kk)
+                            scs[c][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(aotx_h8a, kr[e][kk]),
+                                                                               qb[c][kk], scs[c][e], 0, 0, 0);
+                    }
+                const bool gone0 = gone[0], gone1 = gone[1];
+                /* the registers are used: the next pair's loads run under the rest of this
+                 * step (unconditional: no copies where paths join) */
+                __builtin_amdgcn_sched_barrier(0);
+                load(p + PARTS);
+                __builtin_amdgcn_sched_barrier(0);
+                weigh(scs, p, gone0, gone1, vw);
+            }
+        } else {
+            /* a wave brings block `half` of its part's pair; every wave meets every barrier */
+            const auto slot = [&](unsigned int buf, unsigned int what) {
+                return (unsigned short *)(lds + ((buf * PARTS + part) * 2u + what) * ROWS);
+            };
+            aotx_u4a kl[VP], vr[VP];
+            bool gone[2] = {false, false};
+            const auto load = [&](unsigned int p) {
+                look(p);
+                bool g0, g1;
+                const __amdgpu_buffer_rsrc_t r0 = block(2u * p, g0), r1 = block(2u * p + 1u, g1);
+                gone[0] = g0;
+                gone[1] = g1;
+                const __amdgpu_buffer_rsrc_t rs = half == 0u ? r0 : r1;
+#pragma unroll
+                for (int u = 0; u < VP; ++u) kl[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, kbase + u * 1024, 0, 0);
+#pragma unroll
+                for (int u = 0; u < VP; ++u) vr[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, vbase + u * 1024, 0, 0);
+            };
+            const auto store = [&](unsigned int buf) {
+#pragma unroll
+                for (int u = 0; u < VP; ++u) {
+                    const unsigned int piece = (unsigned int)u * 64u + lane;
+                    const unsigned int at = (half * 16u + piece / (D / 8)) * VS + (piece % (D / 8)) * 8u;
+                    *(aotx_u4a *)(slot(buf, 0u) + at) = kl[u];
+                    *(aotx_u4a *)(slot(buf, 1u) + at) = vr[u];
+                }
+            };
+            const bool mine = group >> (c0 / G) << (64u - (COLS + G - 1u) / G) != 0ull;   /* any column here */
+            load(part);
+            __syncthreads();          /* the sequence before is read */
+            store(0u);
+            __syncthreads();
+            const unsigned int steps = (pairs + PARTS - 1u) / PARTS;
+            for (unsigned int st = 0; st < steps; ++st) {
+                const unsigned int p = part + st * PARTS;
+                const bool gone0 = gone[0], gone1 = gone[1];
+                load(p + PARTS);
+                __builtin_amdgcn_sched_barrier(0);
+                if (p < pairs && mine) {
+                    const unsigned short *kw = slot(st & 1u, 0u);
+                    aotx_f4a scs[NC][2];
+                    aotx_h8a k8[2][KK];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int kk = 0; kk < KK; ++kk)
+                            k8[e][kk] = *(const aotx_h8a *)(kw + ((unsigned int)e * 16u + r) * VS + 32u * (unsigned int)kk + 8u * g);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) scs[c][e] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+                        for (int e = 0; e < 2; ++e)
+#pragma unroll
+                            for (int c = 0; c < NC; ++c)
+                                scs[c][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8[e][kk], qb[c][kk], scs[c][e], 0, 0, 0);
+                    weigh(scs, p, gone0, gone1, slot(st & 1u, 1u));
+                }
+                store((st + 1u) & 1u);
+                __syncthreads();
             }
         }
-        __syncthreads();        /* the second halves' slots are free for the next round */
     }
+    if (H == 2) __syncthreads();
+    /* the parts: maxima by column, masses by accumulator row, and which columns met a missing
+     * page (each lane group of a column saw all of its blocks) */
+    unsigned long long missed = 0ull;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const unsigned long long mc = __ballot(miss[c] != 0u);
+        missed |= mc;
+        if (lane == 0u) pmiss[half][part][c] = (unsigned int)mc & 0xffffu;
+        if (g == 0u) pm[half][part][16u * (unsigned int)c + r] = mrun[c];
+        if (r == 0u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pl[half][part][16u * (unsigned int)c + 4u * g + (unsigned int)i] = mass[c][i];
+    }
+    if (missed != 0ull && lane == 0u) atomicAdd(&a.state->faults, 1u);
+    __syncthreads();
+    /* without branches: a part with no position has m = -inf, mass 0 and weight 2^-inf = 0 */
+    float *const acc = (float *)lds + (half * PARTS) * (ACC / 4u);
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned int col = 16u * (unsigned int)c + 4u * g + (unsigned int)i;
+            float m[PARTS], top = -INFINITY, sum = 0.0f;
+            unsigned int absent = 0u;
+#pragma unroll
+            for (unsigned int k = 0; k < PARTS; ++k) {
+                m[k] = pm[half][k][col];
+                top = fmaxf(top, m[k]);
+                absent |= pmiss[half][k][c] >> (col & 15u);
+            }
+            top = top == -INFINITY ? 0.0f : top;
+#pragma unroll
+            for (unsigned int k = 0; k < PARTS; ++k) sum += pl[half][k][col] * aotx_exp2(m[k] - top);
+            const float whole = 1.0f / (sum > 0.0f ? sum : 1.0f);
+            const float f = (absent & 1u) != 0u ? 0.0f : aotx_exp2(pm[half][part][col] - top) * whole;
+#pragma unroll
+            for (int cc = 0; cc < NS; ++cc)
+                acc[part * (ACC / 4u) + ((c * NS + cc) * 4 + i) * 64 + lane] = o[c][cc][i] * f;
+        }
+    __syncthreads();
+    /* part k adds the slices [k NP, (k + 1) NP) of all parts in part order */
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned int col = c0 + 16u * (unsigned int)c + 4u * g + (unsigned int)i;
+            const unsigned int tc = col / (unsigned int)G, hc = col % (unsigned int)G;
+            float v[NP];
+#pragma unroll
+            for (int s = 0; s < NP; ++s) {
+                const unsigned int cc = part * (unsigned int)NP + (unsigned int)s;
+                v[s] = 0.0f;
+#pragma unroll
+                for (unsigned int k = 0; k < PARTS; ++k)
+                    v[s] += acc[k * (ACC / 4u) + (((unsigned int)c * NS + cc) * 4u + (unsigned int)i) * 64u + lane];
+            }
+            if (t0 + tc < tokens)
+#pragma unroll
+                for (int s = 0; s < NP; ++s) {
+                    const unsigned int cc = part * (unsigned int)NP + (unsigned int)s;
+                    a.out[aotx_attn_out_at(a, t0 + tc, kh * G + hc, 16u * cc + r, D)] = aotx_f2h(v[s]);
+                }
+        }
 }
 
 #undef MMA_WINDOW
 #undef MMA_LOAD
 #undef MMA_COMPUTE
-#undef MMA_COMPUTE_SH
 
 #endif

@@ -236,3 +236,51 @@ def test_attend_prompt_pieces_vs_oracle(torch, lib, orc, heads, kvh, d, layout):
         assert lib.aotx_model_faulted() == 0
     finally:
         lib.aotx_kv_close(ctypes.byref(m))
+
+
+@pytest.mark.parametrize("heads,kvh,d", [(16, 8, 128), (8, 8, 128), (16, 2, 128), (8, 2, 64)])
+def test_attend_prompt_edges_vs_oracle(torch, lib, orc, heads, kvh, d):
+    """The batch kernel's edges: contexts around the pairs of blocks that a wave takes in turn
+    (1, 16, 17, 32, 33, 127..129 positions), past the 1024 positions of a window of page
+    addresses, positions of one sequence out of order, tokens that end inside a wave's 32
+    columns; and a slot without pages, whose rows are zero while its neighbours' are right and
+    the fault count grows."""
+    layers, layer = 2, 1
+    rng = np.random.default_rng(heads * 3 + d)
+    pieces = [(1, 0, 1), (2, 15, 1), (3, 14, 3), (4, 30, 2), (5, 30, 3), (6, 120, 9), (7, 2050, 70), (8, 0, 45)]
+    contexts = [c + n for _, c, n in pieces]
+    slots = [s for s, _, _ in pieces]
+    m = _open_pool(lib, 256)
+    try:
+        for s, n in zip(slots, contexts):
+            assert lib.aotx_kv_request(s, layout_pages(n, layers, kvh, d)) == 1
+        lib.aotx_kv_serve(ctypes.byref(m), None)
+        keys, vals = _fill(torch, lib, slots, contexts, layers, layer, kvh, d, rng)
+        pos = np.concatenate([np.arange(c, c + n) for _, c, n in pieces]).astype(np.uint32)
+        ag = np.concatenate([np.full(n, s) for s, _, n in pieces]).astype(np.uint32)
+        pos[-45:] = rng.permutation(45)
+        # a slot that holds no page, inside a run of another
+        pos = np.insert(pos, 40, 100).astype(np.uint32)
+        ag = np.insert(ag, 40, 33).astype(np.uint32)
+        tokens = len(pos)
+        assert tokens >= 128 and tokens % 4 != 0
+        q = rng.normal(0, 1, (tokens, heads, d)).astype(np.float16)
+        out = torch.full((tokens * heads * d,), 7.0, dtype=torch.float16, device="cuda")
+        lib.aotx_model_forget()
+        assert lib.aotx_attend_paged(p(dev(q, torch)), p(dev(pos, torch)), p(dev(ag, torch)),
+                                     tokens, heads, kvh, d, layer, layers, p(out), None) == 0
+        torch.cuda.synchronize()
+        assert lib.aotx_model_faulted() > 0
+        got = out.cpu().numpy().reshape(tokens, heads, d).astype(np.float32)
+        g = heads // kvh
+        for i in range(tokens):
+            if ag[i] == 33:
+                assert (got[i] == 0).all()
+                continue
+            for hh in range(0, heads, 3):
+                kk = keys[int(ag[i])][:, hh // g, :].astype(np.float32)
+                vv = vals[int(ag[i])][:, hh // g, :].astype(np.float32)
+                want = orc.attend_one(q[i, hh].astype(np.float32), kk, vv, int(pos[i]))
+                assert np.abs(got[i, hh] - want).max() < 4e-3, (i, int(ag[i]), int(pos[i]), hh)
+    finally:
+        lib.aotx_kv_close(ctypes.byref(m))
