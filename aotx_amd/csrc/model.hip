@@ -251,11 +251,11 @@ static void aotx_rproduct(aotx_hold *h, const void *const *w, const unsigned int
                           unsigned int nseg, unsigned int k, int epi, unsigned int cap,
                           const unsigned int *m_dev, const aotx_rgemv_args &tmpl)
 {
-    /* 128 rows or more of a dense product: one GEMM pass (up to 512 rows; 128-token prompt
-     * 10.15 -> 8.49 ms against passes of 32 rows, while at 64 rows its few workgroups are
-     * slower than re-reading the weights per 32 rows: the Mixtral-shape step 17.2 -> 19.3
-     * ms); routed experts keep passes of 32 rows through their row lists */
-    const bool gemm = cap >= 128u && tmpl.expert_stride == 0ull && tmpl.list == nullptr
+    /* 64 rows or more of a dense product: passes of up to 512 rows, each as its plan has it
+     * (128-token prompt 10.15 -> 8.49 ms against passes of 32 rows, 64 slots' decode step of
+     * the 8B shape 5.5 -> 4.9 ms); routed experts keep passes of 32 rows through their row
+     * lists */
+    const bool gemm = cap >= 64u && tmpl.expert_stride == 0ull && tmpl.list == nullptr
                    && tmpl.xrow == nullptr && tmpl.xmode == AOTX_X_F16;
     for (unsigned int m0 = 0, mt = 0; m0 < cap; m0 += mt) {
         mt = gemm ? (cap - m0 < AOTX_RGEMM_ROWS ? cap - m0 : AOTX_RGEMM_ROWS)
@@ -280,6 +280,7 @@ static void aotx_rproduct(aotx_hold *h, const void *const *w, const unsigned int
             a.passes = (cap - m0) / 32u;
             if (a.passes > AOTX_WIDE_PASSES) a.passes = AOTX_WIDE_PASSES;
             mt = 32u * a.passes;
+            a.m = mt;
         }
         if (a.splits > 1u) {
             size_t need = aotx_rgemv_partial_bytes(a);
@@ -801,7 +802,8 @@ extern "C" int aotx_model_open(unsigned int role, unsigned int max_tokens)
             if (aotx_rgemv_plan_frag(&a, w1, rv, 1u, d->hidden, AOTX_EPI_F32, mt) == 0)
                 gp = gp > aotx_rgemv_partial_bytes(a) ? gp : aotx_rgemv_partial_bytes(a);
         }
-        /* the GEMM passes (256 rows and more) of the dense products */
+        gp *= AOTX_WIDE_PASSES;                              /* passes in one launch */
+        /* the passes of 64 rows and more of the dense products */
         for (unsigned int mt = 64u; mt <= AOTX_RGEMM_ROWS && mt <= cap; mt += 64u) {
             aotx_rgemv_args a;
             unsigned int r3[3] = {(unsigned int)wide, (unsigned int)narrow, (unsigned int)narrow};
@@ -815,9 +817,12 @@ extern "C" int aotx_model_open(unsigned int role, unsigned int max_tokens)
                 gp = gp > aotx_rgemv_partial_bytes(a) ? gp : aotx_rgemv_partial_bytes(a);
             if (aotx_rgemv_plan(&a, w2, r2, 2u, d->hidden, AOTX_EPI_SWIGLU, mt) == 0)
                 gp = gp > aotx_rgemv_partial_bytes(a) ? gp : aotx_rgemv_partial_bytes(a);
+            unsigned int rv[1] = {d->vocab};
+            if (aotx_rgemv_plan(&a, w1, rv, 1u, d->hidden, AOTX_EPI_F32, mt) == 0)
+                gp = gp > aotx_rgemv_partial_bytes(a) ? gp : aotx_rgemv_partial_bytes(a);
         }
     }
-    h->gemv_partial_bytes = gp * AOTX_WIDE_PASSES + 4096u;   /* passes in one launch */
+    h->gemv_partial_bytes = gp + 4096u;
     h->gemv_partial = (float *)aotx_take(h, h->gemv_partial_bytes);
     h->gemv_count = (unsigned int *)aotx_take(h, AOTX_GEMV_COUNTS * sizeof(unsigned int));
     size_t ap = 0u;

@@ -49,7 +49,8 @@ struct aotx_rgemv_args {
     unsigned int k;
     unsigned int qn;              /* quads of k */
     unsigned int rt;              /* 16-row tiles per workgroup */
-    unsigned int wide;            /* 1: the tile-split wide-batch kernel (fp16 x only) */
+    unsigned int wide;            /* 1: the tile-split wide-batch kernel (fp16 x only), 2: its
+                                     64-row form */
     unsigned int gemm;            /* 1: the GEMM of 33..512 rows (fp16 x, direct rows) */
     unsigned int frag;            /* 1: the fragment-layout product (AOTX_X_FRAG, 5..32 rows) */
     unsigned int file;            /* 1: the weights are in the file's layout */
@@ -96,13 +97,14 @@ struct aotx_rgemv_args {
     unsigned int xrow_div;
     unsigned int experts;
     /* wide products of direct rows: consecutive 32-row passes in one launch (grid.y is the
-     * pass, rows m0 + 32 * pass on); 0 or 1 is one pass */
+     * pass, rows m0 + 32 * pass on); 0 or 1 is one pass; m counts the rows of all of them */
     unsigned int passes;
 };
 
 /* Plan a product over Q8R tensors; rows per segment; returns 1 when refused. mt is the
  * pass capacity: up to AOTX_NARROW_ROWS rows take the streaming kernel (which can stage x
- * as the RMSNorm of the residual stream), up to 32 the wide kernel, and up to
+ * as the RMSNorm of the residual stream), up to 32 the wide kernel (small matrices: more rows in
+ * passes of it), up to 64 its 64-row form where that is the faster one, and up to
  * AOTX_RGEMM_ROWS the GEMM. */
 #define AOTX_NARROW_ROWS 4u
 #define AOTX_RGEMM_ROWS 512u
@@ -120,7 +122,7 @@ int aotx_rgemv_plan_frag(aotx_rgemv_args *a, const void *const *w, const unsigne
 /* Take a planned product's weights in the file's layout (rows of k / 32 blocks of 34 bytes,
  * any alignment) instead of Q8R: the same plan, kernels, operands and order of sums. */
 static inline void aotx_rgemv_file(aotx_rgemv_args *a) { a->file = 1u; }
-/* Launch one pass (<= 32 rows) and, with splits > 1, the kernel that adds the partials
+/* Launch one pass (the plan's rows at most) and, with splits > 1, the kernel that adds the partials
  * and applies the epilogue. */
 int aotx_rgemv_launch(const aotx_rgemv_args &a, hipStream_t stream);   /* 1 when refused */
 size_t aotx_rgemv_partial_bytes(const aotx_rgemv_args &a);

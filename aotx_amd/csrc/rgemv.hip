@@ -79,7 +79,7 @@ __global__ __launch_bounds__(64 * NW) void aotx_rgemv(aotx_rgemv_args a)
     rg_narrow<MT, RT, PD, NW, NORM, DIRECT, FILE>(a, blockIdx.x, blockIdx.y, lds);
 }
 
-/* Wide batches (17..32 rows of fp16 x): a workgroup owns T 16-row tiles; its W = T * P
+/* Wide batches (MT rows of fp16 x at most, 32 or 64): a workgroup owns T 16-row tiles; its W = T * P
  * waves are T tile owners times P phases. x passes through LDS in chunks of KC quads,
  * double-buffered (the next chunk is loaded into registers while the current one feeds
  * the MFMAs); the P waves of a tile take its quads of each chunk in turn (phase p: chunk
@@ -88,13 +88,14 @@ __global__ __launch_bounds__(64 * NW) void aotx_rgemv(aotx_rgemv_args a)
  * phase order through LDS and the workgroup applies the epilogue (with k split over
  * workgroups, the last split to finish adds the splits first). More phases put more waves
  * on the same tiles (more loads in flight per CU) at the price of more x staging. */
-template <int T, int P, int KC, int PDQ, bool FILE>
-__global__ __launch_bounds__(64 * T * P, 4) void aotx_rgemv_wide(aotx_rgemv_args a0)
+template <int T, int P, int KC, int PDQ, bool FILE, int MT>
+__global__ __launch_bounds__(64 * T * P, MT == 64 ? 2 : 4) void aotx_rgemv_wide(aotx_rgemv_args a0)
 {
-    /* direct rows: grid.y is the 32-row pass (routed experts: the expert) */
+    /* direct rows: grid.y is the pass of MT rows (routed experts: the expert) */
     aotx_rgemv_args a = a0;
-    if (a0.expert_stride == 0ull) a.m0 = a0.m0 + 32u * blockIdx.y;
-    constexpr int MT = 32;
+    const unsigned int before = a0.expert_stride == 0ull ? (unsigned int)MT * blockIdx.y : 0u;
+    a.m0 = a0.m0 + before;
+    constexpr int CB = MT / 16;                              /* column blocks */
     constexpr int W = T * P;
     constexpr int NT = 64 * W;
     constexpr int NQ = KC / P;                               /* a wave's quads per chunk */
@@ -110,8 +111,8 @@ __global__ __launch_bounds__(64 * T * P, 4) void aotx_rgemv_wide(aotx_rgemv_args
     const unsigned int wave = tid >> 6;
     const unsigned int expert = blockIdx.y;
     const unsigned int *list = nullptr;
-    unsigned int mrows = a.m;
-    const unsigned int cap = a.m < (unsigned int)MT ? a.m : (unsigned int)MT;
+    const unsigned int cap = a0.m - before < (unsigned int)MT ? a0.m - before : (unsigned int)MT;
+    unsigned int mrows = cap;
     if (a.expert_stride != 0ull) {
         /* an expert no row chose streams nothing: its row count comes first */
         unsigned int total = rg_scalar(a.list_count + expert);
@@ -133,7 +134,9 @@ __global__ __launch_bounds__(64 * T * P, 4) void aotx_rgemv_wide(aotx_rgemv_args
     const rg_wsrc<FILE> wsrc = rg_wopen<FILE>(a, group, tj, T, expert, lane);
     const unsigned int wend = rg_wend<FILE>(a, lane);
     const unsigned int wlim = FILE && wend < q1 ? wend : q1;     /* quads past it add nothing */
-    rg_f4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+    rg_f4 acc[CB];
+#pragma unroll
+    for (int t = 0; t < CB; ++t) acc[t] = (rg_f4){0.0f, 0.0f, 0.0f, 0.0f};
     const unsigned int wshift = rg_wshift<FILE>(wsrc, lane);
     rg_wreg wr[2][PDQ];              /* two buffers of PDQ quads (one 32-bit register per scale:
                                         no packing waits) */
@@ -155,18 +158,22 @@ __global__ __launch_bounds__(64 * T * P, 4) void aotx_rgemv_wide(aotx_rgemv_args
             const unsigned int qq = RGW_QUAD((N) + (unsigned int)qi);                    \
             const unsigned int qx = qq < q1 ? qq : q1 - 1u;                              \
             const unsigned short *xq = (XB) + ((qx - q0) % KC) * 128u + 32u * g;         \
-            rg_h8 B[2][4];                                                               \
-            _Pragma("unroll") for (int t = 0; t < 2; ++t)                                \
-                _Pragma("unroll") for (int s = 0; s < 4; ++s)                            \
-                    B[t][s] = *(const rg_h8 *)(xq + ((unsigned int)t * 16u + r) * XS + 8u * s); \
+            rg_h8 B[CB][4];                                                              \
+            if (MT == 32)                                                                \
+                _Pragma("unroll") for (int t = 0; t < CB; ++t)                           \
+                    _Pragma("unroll") for (int s = 0; s < 4; ++s)                        \
+                        B[t][s] = *(const rg_h8 *)(xq + ((unsigned int)t * 16u + r) * XS + 8u * s); \
             unsigned int qd[8], sbits;                                                   \
             rg_wquants<FILE>(wr[BUF][qi], wshift, qd, sbits);                            \
             sbits = qq < wlim ? sbits : 0u;                                              \
             rg_h2 s2 = __builtin_bit_cast(rg_h2, sbits | (sbits << 16));                 \
             _Pragma("unroll") for (int s = 0; s < 4; ++s) {                              \
-                const rg_h8 A = rg_afrag(qd[2 * s], qd[2 * s + 1], s2);            \
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[0][s], acc[0], 0, 0, 0); \
-                acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[1][s], acc[1], 0, 0, 0); \
+                if (MT != 32)       /* a step's operands at a time */                    \
+                    _Pragma("unroll") for (int t = 0; t < CB; ++t)                       \
+                        B[t][s] = *(const rg_h8 *)(xq + ((unsigned int)t * 16u + r) * XS + 8u * s); \
+                const rg_h8 A = rg_afrag(qd[2 * s], qd[2 * s + 1], s2);                  \
+                _Pragma("unroll") for (int t = 0; t < CB; ++t)                           \
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, B[t][s], acc[t], 0, 0, 0); \
             }                                                                            \
         }                                                                                \
     } while (0)
@@ -299,7 +306,7 @@ __global__ __launch_bounds__(64 * T * P, 4) void aotx_rgemv_wide(aotx_rgemv_args
     float *part = (float *)lds;
     const unsigned int gr = T * 16u;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < CB; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             part[P == 1 ? rg_o<MT>(wave * 16u + 4u * g + (unsigned int)i, (unsigned int)t * 16u + r)
@@ -807,6 +814,30 @@ static int aotx_rgemv_plan_n(aotx_rgemv_args *a, const void *const *w, const uns
         a->n = total;
         tiles = (total + 15u) / 16u;
     }
+    if (mt > 32u && !routed) {
+        /* More than 32 rows of a small matrix: whole-k passes of the wide kernel in one launch,
+         * while that takes one round of a workgroup per CU (two for a short k against the GEMM).
+         * The larger forms below fill the chip with such a matrix only by splitting k, and their
+         * merge alone costs as much as a pass: 128 rows of 2048 square take 7.2 us against 19.0
+         * by the GEMM, 512 of 512 x 1024 6.9 against 16.1, 400 of 100 x 14336 29.0 against 42.5,
+         * 128 of 4096 x 3072 in two rounds 15.8 against 23.4; 64 rows of 4096 x 2048 7.7 against
+         * 11.3 by the 64-row form, of 1024 x 8064 16.2 against 16.2, in two rounds (6144 x 3072)
+         * 15.7 against 13.8. */
+        const unsigned int passes = (mt + 31u) / 32u;
+        const unsigned int groups = epi == AOTX_EPI_SWIGLU ? (unsigned int)aotx_q8r_tiles(rows[0])
+                                                           : (tiles + 1u) / 2u;
+        if (groups * passes <= 256u ? a->qn <= (mt <= 64u ? 48u : 128u)
+                                    : mt > 64u && groups * passes <= 512u && a->qn <= 32u) {
+            a->wide = 1u;
+            a->rt = 2u;
+            a->pd = 4u;
+            a->groups = groups;
+            a->splits = 1u;
+            a->qps = a->qn;
+            a->passes = passes;
+            return 0;
+        }
+    }
     if (mt > 32u) {
         /* 256 weight rows (16 tiles; SWIGLU: 8 gate/up pairs) by 64 batch rows per workgroup */
         a->gemm = 1u;
@@ -823,6 +854,31 @@ static int aotx_rgemv_plan_n(aotx_rgemv_args *a, const void *const *w, const uns
             sp *= 2u;
         a->qps = (a->qn + sp - 1u) / sp;
         a->splits = (a->qn + a->qps - 1u) / a->qps;
+        /* 33 to 64 rows: the wide kernel's 64-row form, 4 tiles a workgroup and k split up to one
+         * workgroup per CU (within the partials of the GEMM's plan, so that no call needs more
+         * scratch), while a workgroup then walks at most 32 quads: 64 rows of 14336 x 4096 take
+         * 22.5 us against 25.2 by the GEMM, of 4096 x 14336 24.7 against 30.1, of 2048 square
+         * 10.5 against 18.8. Past either line the GEMM, whose 16 tiles read x less often, wins:
+         * 20480 x 4096 41.7 against 29.3 us (a second workgroup on some CUs), 8192 x 28672 78
+         * against 62. */
+        if (mt <= 64u && !routed) {
+            const unsigned int groups = epi == AOTX_EPI_SWIGLU
+                ? ((unsigned int)aotx_q8r_tiles(rows[0]) + 1u) / 2u : (tiles + 3u) / 4u;
+            unsigned int s = 1u;
+            while (groups * (s + 1u) <= 256u && groups * (s + 1u) <= 4u * a->groups * a->splits
+                   && a->splits > 1u && a->qn / (s + 1u) >= 4u)
+                s += 1u;
+            const unsigned int qps = (a->qn + s - 1u) / s;
+            if (groups <= 256u && qps <= 32u) {
+                a->gemm = 0u;
+                a->wide = 2u;
+                a->rt = 4u;
+                a->pd = 2u;
+                a->groups = groups;
+                a->qps = qps;
+                a->splits = (a->qn + qps - 1u) / qps;
+            }
+        }
         return 0;
     }
     /* 5 to 32 rows: the wide kernel. With 32 batch columns per MFMA it wastes matrix-core
@@ -942,7 +998,8 @@ size_t aotx_rgemv_partial_bytes(const aotx_rgemv_args &a)
     if (a.splits <= 1u) return 0u;
     if (a.gemm) return (size_t)aotx_rgemv_count_words(a) * a.splits * RGM_RT * 16u * RGM_MB * sizeof(float);
     size_t e = aotx_rgemv_rows_y(a);
-    return e * a.groups * a.splits * a.rt * 16u * 33u * sizeof(float);   /* rows of 33 (rg_os) */
+    /* rows of 33 or 64 (rg_os) */
+    return e * a.groups * a.splits * a.rt * 16u * (a.wide == 2u ? 64u : 33u) * sizeof(float);
 }
 
 unsigned int aotx_rgemv_count_words(const aotx_rgemv_args &a)
@@ -992,8 +1049,9 @@ int aotx_rgemv_launch(const aotx_rgemv_args &a0, hipStream_t s)
         a.partial = (float *)aotx_scratch(AOTX_SCRATCH_GEMV_PARTIAL, aotx_rgemv_partial_bytes(a));
     }
     if (a.splits > 1u && a.count == nullptr) {
-        a.count = (unsigned int *)aotx_scratch(AOTX_SCRATCH_GEMV_COUNT,
-                                               (size_t)aotx_rgemv_count_words(a) * sizeof(unsigned int));
+        /* at least one counter per CU: a plan of more, smaller tile groups finds them there */
+        const size_t words = aotx_rgemv_count_words(a) < 256u ? 256u : aotx_rgemv_count_words(a);
+        a.count = (unsigned int *)aotx_scratch(AOTX_SCRATCH_GEMV_COUNT, words * sizeof(unsigned int));
     }
     if (a.gemm) {
         if (a.xmode != AOTX_X_F16 || a.expert_stride != 0ull || a.list != nullptr
@@ -1060,15 +1118,16 @@ int aotx_rgemv_launch(const aotx_rgemv_args &a0, hipStream_t s)
             fprintf(stderr, "aotx: the wide-batch product takes fp16 x only\n");
             return 1;
         }
-#define RGW_GO(T, P, KC, PDQ)                                                              \
+#define RGW_GO(T, P, KC, PDQ, MT)                                                            \
         do {                                                                               \
-            const size_t xb = 2u * 32u * (KC * 128u + 8u) * 2u;                            \
-            if (a.file) hipLaunchKernelGGL((aotx_rgemv_wide<T, P, KC, PDQ, true>), grid, dim3(512), xb, s, a); \
-            else hipLaunchKernelGGL((aotx_rgemv_wide<T, P, KC, PDQ, false>), grid, dim3(512), xb, s, a); \
+            const size_t xb = 2u * MT * (KC * 128u + 8u) * 2u;                             \
+            if (a.file) hipLaunchKernelGGL((aotx_rgemv_wide<T, P, KC, PDQ, true, MT>), grid, dim3(512), xb, s, a); \
+            else hipLaunchKernelGGL((aotx_rgemv_wide<T, P, KC, PDQ, false, MT>), grid, dim3(512), xb, s, a); \
         } while (0)
-        if (a.rt == 2u) RGW_GO(2, 4, 8, 1);
-        else if (a.rt == 4u) RGW_GO(4, 2, 4, 1);
-        else RGW_GO(8, 1, 4, 2);
+        if (a.wide == 2u) RGW_GO(4, 2, 4, 1, 64);
+        else if (a.rt == 2u) RGW_GO(2, 4, 8, 1, 32);
+        else if (a.rt == 4u) RGW_GO(4, 2, 4, 1, 32);
+        else RGW_GO(8, 1, 4, 2, 32);
 #undef RGW_GO
         AOTX_LAUNCH_CHECK();
         return 0;

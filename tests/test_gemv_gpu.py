@@ -170,7 +170,8 @@ def test_repack_layout(torch, lib):
                     assert (quant[t, q, lane] == 0x80).all() and scale[t, q, lane] == 0
 
 
-@pytest.mark.parametrize("n,k,shift", [(17, 96, 0), (33, 160, 2), (48, 32, 0), (300, 4128, 2), (130, 416, 0), (64, 512, 6)])
+@pytest.mark.parametrize("n,k,shift", [(17, 96, 0), (33, 160, 2), (48, 32, 0), (300, 4128, 2), (130, 416, 0), (64, 512, 6),
+                                       (200, 6304, 2), (2100, 416, 2), (8200, 416, 0)])
 @pytest.mark.parametrize("m", [1, 4, 5, 9, 32, 33, 64, 100])
 def test_product_ends_and_alignment(torch, lib, orc, n, k, shift, m):
     """Products over the file's layout whose blocks start at odd multiples of two bytes (an odd
