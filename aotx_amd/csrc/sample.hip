@@ -1,7 +1,7 @@
 /* Sampler and Philox stream.
  *
  * Reference: aotx_model_pick (cuda/model/sample.cu:456-765) and the Philox4x32-10 stream
- * (cuda/rng/rng.cuh:29-94). One block of 256 threads takes one row of logits. The steps,
+ * (cuda/rng/rng.cuh:29-94). Several workgroups of 256 threads take one row of logits. The steps,
  * their order and every float expression follow the reference so that the same logits
  * give the same token: the largest logit (ties to the lowest thread = token mod 256, then
  * the lowest token), a temperature of zero returns it; otherwise the row sum of

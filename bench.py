@@ -528,7 +528,7 @@ def text_run(args):
                       "bytes": nbytes, "tokens": ntok, "encode_ms": round(e * 1e3, 3),
                       "decode_ms": round(d * 1e3, 3),
                       "decode_mb_s": round(nbytes / d / 1e6, 2),
-                      "note": "wall clock of the synchronous library calls on inputs in HBM (encode includes its scratch allocations and one 4-byte read-back)",
+                      "note": "wall clock of the synchronous library calls on inputs in HBM (encode includes its scratch allocation and one 8-byte read-back)",
                       "cpu_baseline": cpu}))
 
 

@@ -70,9 +70,10 @@ int aotx_text_vocab_report(unsigned int report[4]);
  * byte that starts no UTF-8 character is read as U+FFFD, three bytes, as
  * cuda/text/text.cuh:367-374 cleans text, and a text never has more tokens than cleaned
  * bytes) and their count to count[t]. The pipeline of cuda/text/pretok.cu:393 and
- * bpe.cu:44-223: one thread per text cuts the pre-tokens (a pre-token longer than
+ * bpe.cu:44-223, a text in parallel throughout: a workgroup per text cleans it, a thread per
+ * end of a run of letters or numbers cuts the pre-tokens from there (a pre-token longer than
  * AOTX_TEXT_CHUNK_BYTES is cut at a character boundary and the rest is matched again),
- * one wave per pre-token merges it (the lowest pair rank first, the leftmost of equal
+ * a lane per pre-token, a wave for a long one, merges it (the lowest pair rank first, the leftmost of equal
  * ranks; with the family's whole rule a pre-token that is a token stays whole). Tokens
  * of the control and user types are whole matches found first, the longest at the
  * leftmost place (cuda/text/pretok.cu:339-372, :404-431); the pattern reads no text across
