@@ -814,30 +814,6 @@ static int aotx_rgemv_plan_n(aotx_rgemv_args *a, const void *const *w, const uns
         a->n = total;
         tiles = (total + 15u) / 16u;
     }
-    if (mt > 32u && !routed) {
-        /* More than 32 rows of a small matrix: whole-k passes of the wide kernel in one launch,
-         * while that takes one round of a workgroup per CU (two for a short k against the GEMM).
-         * The larger forms below fill the chip with such a matrix only by splitting k, and their
-         * merge alone costs as much as a pass: 128 rows of 2048 square take 7.2 us against 19.0
-         * by the GEMM, 512 of 512 x 1024 6.9 against 16.1, 400 of 100 x 14336 29.0 against 42.5,
-         * 128 of 4096 x 3072 in two rounds 15.8 against 23.4; 64 rows of 4096 x 2048 7.7 against
-         * 11.3 by the 64-row form, of 1024 x 8064 16.2 against 16.2, in two rounds (6144 x 3072)
-         * 15.7 against 13.8. */
-        const unsigned int passes = (mt + 31u) / 32u;
-        const unsigned int groups = epi == AOTX_EPI_SWIGLU ? (unsigned int)aotx_q8r_tiles(rows[0])
-                                                           : (tiles + 1u) / 2u;
-        if (groups * passes <= 256u ? a->qn <= (mt <= 64u ? 48u : 128u)
-                                    : mt > 64u && groups * passes <= 512u && a->qn <= 32u) {
-            a->wide = 1u;
-            a->rt = 2u;
-            a->pd = 4u;
-            a->groups = groups;
-            a->splits = 1u;
-            a->qps = a->qn;
-            a->passes = passes;
-            return 0;
-        }
-    }
     if (mt > 32u) {
         /* 256 weight rows (16 tiles; SWIGLU: 8 gate/up pairs) by 64 batch rows per workgroup */
         a->gemm = 1u;
@@ -854,6 +830,39 @@ static int aotx_rgemv_plan_n(aotx_rgemv_args *a, const void *const *w, const uns
             sp *= 2u;
         a->qps = (a->qn + sp - 1u) / sp;
         a->splits = (a->qn + a->qps - 1u) / a->qps;
+        /* More than 32 rows of a small matrix: passes of the wide kernel in one launch, k split up
+         * to a workgroup per CU (within the partials of the GEMM's plan, so that no call needs
+         * more scratch; a split keeps 8 quads), while that takes one round of workgroups (two for
+         * a short k against the GEMM). The larger forms fill the chip with such a matrix only by
+         * cutting k into many short splits: 128 rows of 2048 square take 7.0 us against 19.0 by
+         * the GEMM, 512 of 512 x 1024 6.9 against 16.1, 400 of 100 x 14336 13.5 against 42.5 (28.9
+         * unsplit), 128 of 4096 x 3072 in two rounds 15.8 against 23.4; 64 rows of 4096 x 2048 7.7
+         * against 11.3 by the 64-row form, of 1024 x 8064 10.7 against 16.2, but in two rounds
+         * (6144 x 3072) 15.7 against 13.8. */
+        const unsigned int passes = (mt + 31u) / 32u;
+        const unsigned int pairs = epi == AOTX_EPI_SWIGLU ? (unsigned int)aotx_q8r_tiles(rows[0])
+                                                          : (tiles + 1u) / 2u;
+        if (!routed) {
+            const unsigned int wgs = pairs * passes;
+            unsigned int s = 1u;
+            /* a workgroup's partials are 32 rows of 33, the GEMM's 256 of 64 */
+            while (a->splits > 1u && wgs * (s + 1u) <= 256u && a->qn / (s + 1u) >= 8u
+                   && wgs * (s + 1u) * 32u * 33u <= a->groups * ny * a->splits * RGM_RT * 16u * RGM_MB)
+                s += 1u;
+            const unsigned int qps = (a->qn + s - 1u) / s;
+            if (wgs <= 256u ? qps <= (mt <= 64u ? 48u : 128u)
+                            : mt > 64u && wgs <= 512u && a->qn <= 32u) {
+                a->gemm = 0u;
+                a->wide = 1u;
+                a->rt = 2u;
+                a->pd = 4u;
+                a->groups = pairs;
+                a->qps = qps;
+                a->splits = (a->qn + qps - 1u) / qps;
+                a->passes = passes;
+                return 0;
+            }
+        }
         /* 33 to 64 rows: the wide kernel's 64-row form, 4 tiles a workgroup and k split up to one
          * workgroup per CU (within the partials of the GEMM's plan, so that no call needs more
          * scratch), while a workgroup then walks at most 32 quads: 64 rows of 14336 x 4096 take
@@ -890,8 +899,9 @@ static int aotx_rgemv_plan_n(aotx_rgemv_args *a, const void *const *w, const uns
          * tiles (gate/up pair, head), 4 x 2 for a 14336-row matrix, 2 x 4 for few (QKV, O,
          * down), measured best at the 8B shapes. Products run unsplit (no partials,
          * no second launch) unless they have fewer than 192 workgroups and k of 32 quads or more (down, a 4096-row O):
-         * those split k towards 256 workgroups while a split keeps a whole chunk, and the
-         * last split of a group to finish adds the partials. */
+         * those split k up to 256 workgroups (one round: their LDS holds one to a CU; 6000 x 4096 at
+         * 32 rows unsplit 10.9 us, in two splits of 188 groups 16.1) while a split keeps a whole
+         * chunk, and the last split of a group to finish adds the partials. */
         a->wide = 1u;
         a->rt = tiles >= 1536u ? 8u : (tiles >= 768u ? 4u : 2u);
         /* routed experts' single products (down): the launch has a workgroup row per
@@ -910,7 +920,7 @@ static int aotx_rgemv_plan_n(aotx_rgemv_args *a, const void *const *w, const uns
          * step 16.75 -> 16.15 ms) */
         unsigned int s = 1u;
         if (!routed && a->groups < 192u && a->qn >= 32u)
-            while (a->groups * s < 256u && a->qn / (s + 1u) >= kc) s += 1u;
+            while (a->groups * (s + 1u) <= 256u && a->qn / (s + 1u) >= kc) s += 1u;
         a->qps = (a->qn + s - 1u) / s;
         a->splits = (a->qn + a->qps - 1u) / a->qps;
         return 0;
