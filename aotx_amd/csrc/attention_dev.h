@@ -411,6 +411,69 @@ static __device__ __forceinline__ float aotx_attn_max4(float v)
     return fmaxf(__builtin_bit_cast(float, b0), __builtin_bit_cast(float, b1));
 }
 
+/* One query row by one wave, the values of the positions it attends and no others: the rows
+ * that the products left NaN. There a position that a row does not attend has weight 0, and 0
+ * times a value of Inf or NaN (another sequence's, a later token's, or one past the sequence's
+ * last position) is NaN. Rare and not fast: lanes over 64 positions for the scores, then over
+ * the dimensions for the values, 32-bit weights. */
+template <int D>
+static __device__ void aotx_attend_row(const aotx_attn_args &a, unsigned int t, unsigned int kh, unsigned int h)
+{
+    constexpr int E = D / 64;                        /* dimensions per lane */
+    const unsigned int lane = threadIdx.x & 63u;
+    const unsigned int agent = a.agent[t], n = a.pos[t] + 1u;
+    const aotx_kv_table *kv = &a.state->kv;
+    const float scale = 1.4426950408889634f / sqrtf((float)D);
+    const unsigned short *q = a.q + ((unsigned long long)t * a.heads + h) * D;
+    float m = -INFINITY, l = 0.0f, o[E];
+    bool missing = false;
+#pragma unroll
+    for (int e = 0; e < E; ++e) o[e] = 0.0f;
+    for (unsigned int p0 = 0u; p0 < n; p0 += 64u) {
+        const unsigned int p = p0 + lane;
+        const unsigned char *blk = p < n
+            ? (const unsigned char *)aotx_kvl_block(a.shape, kv, agent, a.layer, p / 16u * 16u) : nullptr;
+        missing = missing || __any(p < n && blk == nullptr);
+        float s = -INFINITY;
+        if (blk != nullptr) {
+            const unsigned char *k = blk + (unsigned long long)(kh * AOTX_KVL_BLOCK + p % 16u) * D * 2u;
+            s = 0.0f;
+            for (int e = 0; e < D; e += 8) {
+                const aotx_h8a kk = *(const aotx_h8a *)(k + 2 * e), qq = __builtin_bit_cast(aotx_h8a, co_load4(q + e));
+#pragma unroll
+                for (int i = 0; i < 8; ++i) s += (float)kk[i] * (float)qq[i];
+            }
+            s *= scale;
+        }
+        float mb = s;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) mb = fmaxf(mb, __shfl_xor(mb, d, 64));
+        const float mnew = fmaxf(m, mb), msafe = mnew == -INFINITY ? 0.0f : mnew;
+        const float shift = aotx_exp2(m - msafe), w = blk != nullptr ? aotx_exp2(s - msafe) : 0.0f;
+        m = mnew;
+        float mass = w;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) mass += __shfl_xor(mass, d, 64);
+        l = l * shift + mass;
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[e] *= shift;
+        const unsigned int here = n - p0 < 64u ? n - p0 : 64u;
+        for (unsigned int j = 0; j < here; ++j) {
+            const unsigned long long at = __shfl((unsigned long long)blk, (int)j, 64);
+            const float wj = __shfl(w, (int)j, 64);
+            if (at == 0ull) continue;
+            const unsigned short *v = (const unsigned short *)at
+                                    + (unsigned long long)((a.kv_heads + kh) * AOTX_KVL_BLOCK + (p0 + j) % 16u) * D;
+#pragma unroll
+            for (int e = 0; e < E; ++e) o[e] += wj * aotx_h2f(v[(unsigned int)e * 64u + lane]);
+        }
+    }
+    const float back = 1.0f / (l > 0.0f ? l : 1.0f);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        a.out[aotx_attn_out_at(a, t, h, (unsigned int)e * 64u + lane, D)] = aotx_f2h(missing ? 0.0f : o[e] * back);
+}
+
 /* Batches with prompt pieces: a workgroup takes 16 NC H score columns of a KV head, the G
  * query heads of 16 NC H / G consecutive tokens. Its 4 H waves are H halves of the columns (NC
  * tiles of 16 each) times 4 parts of the positions: part k takes every fourth pair of
@@ -428,7 +491,8 @@ static __device__ __forceinline__ float aotx_attn_max4(float v)
  * load a block of the pair each into LDS for both, double-buffered, one barrier per pair: half
  * the reads from the L2s, which bound many columns otherwise. The next pair is on its way while
  * one is computed. The columns may be of several sequences: the workgroup goes over the blocks
- * of one after the other, and a column that does not take part keeps its state.
+ * of one after the other, and a column that does not take part keeps its state (but for values
+ * that are not finite: aotx_attend_row).
  * Bound by the softmax's vector work and the matrix work of a step, about 1600 cycles a wave.
  * Against a wave per 16 / G queries with one block per pass of softmax, at 32 / 8 heads x 128:
  * 512 tokens after 2000 cached ones 74.3 -> 42.8 us (H = 2; 55 with H = 1), a 512-token prompt
@@ -453,6 +517,7 @@ static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a,
     __shared__ __attribute__((aligned(16))) unsigned char lds[STAGE > H * PARTS * ACC ? STAGE : H * PARTS * ACC];
     __shared__ float pm[H][PARTS][COLS], pl[H][PARTS][COLS];
     __shared__ unsigned int pmiss[H][PARTS][NC];
+    __shared__ unsigned int nan[H * NC];             /* each tile's columns that came out NaN */
 
     const unsigned int lane = threadIdx.x & 63u;
     /* a scalar, so that the wave's blocks, loads and tests are scalar too */
@@ -471,6 +536,7 @@ static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a,
     const unsigned int ag = a.agent[tl], ps = a.pos[tl];
     const unsigned long long all = __ballot(live);
     unsigned long long left = all;
+    if (threadIdx.x < (unsigned int)(H * NC)) nan[threadIdx.x] = 0u;
 
     const unsigned int c0 = half * COLS;                        /* this half's first column */
     aotx_h8a qb[NC][KK];
@@ -775,6 +841,7 @@ static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a,
         }
     __syncthreads();
     /* part k adds the slices [k NP, (k + 1) NP) of all parts in part order */
+    bool odd = false;
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -782,6 +849,7 @@ static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a,
             const unsigned int col = c0 + 16u * (unsigned int)c + 4u * g + (unsigned int)i;
             const unsigned int tc = col / (unsigned int)G, hc = col % (unsigned int)G;
             float v[NP];
+            bool bad = false;
 #pragma unroll
             for (int s = 0; s < NP; ++s) {
                 const unsigned int cc = part * (unsigned int)NP + (unsigned int)s;
@@ -789,14 +857,22 @@ static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a,
 #pragma unroll
                 for (unsigned int k = 0; k < PARTS; ++k)
                     v[s] += acc[k * (ACC / 4u) + (((unsigned int)c * NS + cc) * 4u + (unsigned int)i) * 64u + lane];
+                bad = bad || v[s] != v[s];
             }
-            if (t0 + tc < tokens)
+            if (t0 + tc < tokens) {
 #pragma unroll
                 for (int s = 0; s < NP; ++s) {
                     const unsigned int cc = part * (unsigned int)NP + (unsigned int)s;
                     a.out[aotx_attn_out_at(a, t0 + tc, kh * G + hc, 16u * cc + r, D)] = aotx_f2h(v[s]);
                 }
+                if (bad) atomicOr(nan + col / 16u, 1u << (col % 16u));
+                odd = odd || bad;
+            }
         }
+    if (!__syncthreads_or(odd)) return;
+    for (unsigned int col = wave; col < 16u * NC * H; col += PARTS * H)
+        if ((nan[col / 16u] >> (col % 16u)) & 1u)
+            aotx_attend_row<D>(a, t0 + col / (unsigned int)G, kh, kh * G + col % (unsigned int)G);
 }
 
 #undef MMA_WINDOW

@@ -284,3 +284,65 @@ def test_attend_prompt_edges_vs_oracle(torch, lib, orc, heads, kvh, d):
                 assert np.abs(got[i, hh] - want).max() < 4e-3, (i, int(ag[i]), int(pos[i]), hh)
     finally:
         lib.aotx_kv_close(ctypes.byref(m))
+
+
+# the three forms of a launch with prompt pieces, by its score columns (tokens x heads)
+_FORMS = {"16": (0, 6144), "32": (6144, 12288), "64": (12288, 1 << 30)}
+
+
+@pytest.mark.parametrize("form,tokens,heads,kvh,d", [("16", 150, 32, 8, 128), ("32", 200, 32, 8, 128), ("64", 390, 32, 8, 128),
+                                                     ("16", 300, 8, 8, 64), ("32", 400, 16, 16, 128), ("64", 400, 32, 16, 64),
+                                                     ("64", 1000, 16, 2, 64)])
+def test_attend_prompt_nonfinite_values(torch, lib, orc, form, tokens, heads, kvh, d):
+    """Values of Inf and NaN reach the rows that attend their positions and no others: not the
+    rows of sequences in the same workgroup (single rows, short pieces), not a sequence's own
+    earlier rows; nor do the halves that lie past a sequence's last position."""
+    lo, hi = _FORMS[form]
+    assert lo <= tokens * heads < hi
+    layers, layer = 2, 1
+    rng = np.random.default_rng(tokens + heads)
+    pieces = [(1, 60, 1), (2, 0, 9), (3, 37, 1), (4, 90, 1), (5, 20, 7), (6, 45, 1), (7, 0, 33)]
+    pieces.append((8, 13, tokens - sum(n for _, _, n in pieces)))
+    bad = {2: 3, 4: 30, 7: 21, 8: 95}                 # slot: the position of a value that is not finite
+    contexts = [c + n for _, c, n in pieces]
+    m = _open_pool(lib, 256)
+    try:
+        for (s, _, _), n in zip(pieces, contexts):
+            assert lib.aotx_kv_request(s, layout_pages(n + 5, layers, kvh, d)) == 1
+        lib.aotx_kv_serve(ctypes.byref(m), None)
+        keys, vals = _fill(torch, lib, [s for s, _, _ in pieces], [n + 5 for n in contexts], layers, layer, kvh, d, rng)
+        for (s, _, _), n in zip(pieces, contexts):
+            odd = [(n + i, x) for i, x in enumerate((np.inf, np.nan, -np.inf))]       # never attended
+            if s in bad:
+                odd.append((bad[s], np.inf))
+            at = np.array([i for i, _ in odd], dtype=np.uint32)
+            for i, x in odd:
+                vals[s][i, :, ::5] = x
+            assert lib.aotx_kv_write(p(dev(keys[s][at], torch)), p(dev(vals[s][at], torch)), p(dev(at, torch)),
+                                     p(dev(np.full(len(at), s, np.uint32), torch)), len(at), kvh, d, layer, layers, None) == 0
+        pos = np.concatenate([np.arange(c, c + n) for _, c, n in pieces]).astype(np.uint32)
+        ag = np.concatenate([np.full(n, s) for s, _, n in pieces]).astype(np.uint32)
+        q = rng.normal(0, 1, (tokens, heads, d)).astype(np.float16)
+        out = torch.zeros(tokens * heads * d, dtype=torch.float16, device="cuda")
+        lib.aotx_model_forget()
+        assert lib.aotx_attend_paged(p(dev(q, torch)), p(dev(pos, torch)), p(dev(ag, torch)),
+                                     tokens, heads, kvh, d, layer, layers, p(out), None) == 0
+        torch.cuda.synchronize()
+        got = out.cpu().numpy().reshape(tokens, heads, d).astype(np.float32)
+        g = heads // kvh
+        for i in range(tokens):
+            s, last = int(ag[i]), int(pos[i])
+            sees = s in bad and last >= bad[s]
+            hit = np.zeros(d, bool)
+            hit[::5] = sees
+            assert not np.isfinite(got[i][:, hit]).any(), (i, s, last)
+            if i > 80 and i % 7 and abs(last - 95) > 4:
+                assert np.isfinite(got[i][:, ~hit]).all(), (i, s, last)
+                continue
+            for hh in range(0, heads, 3):
+                v = np.where(np.isfinite(vals[s]), vals[s], 0)[:, hh // g, :].astype(np.float32)
+                want = orc.attend_one(q[i, hh].astype(np.float32), keys[s][:, hh // g, :].astype(np.float32), v, last)
+                assert np.abs(got[i, hh] - want)[~hit].max() < 4e-3, (i, s, last, hh)
+        assert lib.aotx_model_faulted() == 0
+    finally:
+        lib.aotx_kv_close(ctypes.byref(m))
