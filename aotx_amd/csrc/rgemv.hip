@@ -616,11 +616,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ?
      * valid row and are stored as zeros) */
     constexpr unsigned int RSTEP = NT / PIECES;
     const unsigned int xrow0 = tid / PIECES, xpc = tid % PIECES;
-    unsigned int xoff[PPT];                       /* element offsets from a.x */
+    const unsigned short *x0 = a.x + (unsigned long long)a.m0 * a.ldx;
+    unsigned int xoff[PPT];                       /* element offsets from x0 */
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
         const unsigned int mm = xrow0 + (unsigned int)i * RSTEP;
-        xoff[i] = (a.m0 + (mm < mrows ? mm : 0u)) * a.ldx + (TAIL ? 0u : xpc * 8u);
+        xoff[i] = (mm < mrows ? mm : 0u) * a.ldx + (TAIL ? 0u : xpc * 8u);
     }
 
     rg_wreg wr[2][2];
@@ -648,7 +649,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ?
         unsigned int qx_ = ((Q) < qn ? (Q) : qn - 1u) * 128u;                            \
         if (TAIL) qx_ = qx_ + xpc * 8u < a.k ? qx_ + xpc * 8u : 0u;                      \
         _Pragma("unroll") for (int i = 0; i < PPT; ++i)                                  \
-            xr[XB][i] = *(const rg_u4 *)(a.x + xoff[i] + qx_);                           \
+            xr[XB][i] = *(const rg_u4 *)(x0 + xoff[i] + qx_);                            \
     } while (0)
 /* the LDS place of quad Q: buffer and offset within a row */
 #define RGM_XBUF(Q) ((((Q) - qb0) >> 1) & 1u)

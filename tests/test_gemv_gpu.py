@@ -194,3 +194,28 @@ def test_product_ends_and_alignment(torch, lib, orc, n, k, shift, m):
         assert fn(ctypes.c_void_p(at), n, k, p(xb), m, p(y), None) == 0
         torch.cuda.synchronize()
         assert np.abs(y.cpu().numpy().reshape(m, n) - want).max() < 1e-5 * max(rms, 1.0) * np.sqrt(k / 32.0)
+
+
+def test_product_rows_past_32_bit_offsets(torch, lib, orc):
+    """x of more than 2^32 values: the rows past them are read where they are (both layouts, by
+    the GEMM: 544 rows of 14336 are too many workgroups for passes of the 32-row kernel)."""
+    n, k = 544, 14336
+    m = (1 << 32) // k + 50
+    w = make(torch, lib, n, k, 77)
+    wr = repack(torch, lib, w, n, k)
+    rng = np.random.default_rng(77)
+    last = rng.normal(0, 1, (8, k)).astype(np.float16)
+    x = torch.zeros(m, k, dtype=torch.float16, device="cuda")
+    x[:64] = 1.0
+    x[m - 8:] = torch.from_numpy(last).cuda()
+    want = orc.q8_gemv_f64(w.cpu().numpy(), n, k, last.view(np.uint16))
+    rms = np.sqrt((want ** 2).mean())
+    y = torch.zeros(m, n, dtype=torch.float32, device="cuda")
+    for fn, at in ((lib.aotx_q8_gemv, w), (lib.aotx_q8r_gemv, wr)):
+        y.fill_(7.0)
+        assert fn(p(at), n, k, p(x), m, p(y), None) == 0
+        torch.cuda.synchronize()
+        assert np.abs(y[m - 8:].cpu().numpy() - want).max() < 1e-5 * max(rms, 1.0) * np.sqrt(k / 32.0)
+        assert float(y[64:m - 8].abs().max()) == 0.0
+    del x, y
+    torch.cuda.empty_cache()
