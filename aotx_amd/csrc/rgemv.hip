@@ -594,7 +594,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ?
 
     aotx_rgemv_args a = a0;
     a.m0 = a0.m0 + yb * (unsigned int)MB;
-    unsigned int total = a0.m;
+    unsigned int total = a0.m0 + a0.m;                      /* m counts the rows from m0 on */
     if (a0.m_dev != nullptr) {
         const unsigned int live = rg_scalar(a0.m_dev);
         total = live < total ? live : total;

@@ -200,7 +200,8 @@ def test_product_rows_past_32_bit_offsets(torch, lib, orc):
     """x of more than 2^32 values: the rows past them are read where they are (both layouts, by
     the GEMM: 544 rows of 14336 are too many workgroups for passes of the 32-row kernel)."""
     n, k = 544, 14336
-    m = (1 << 32) // k + 50
+    m = 586 * 512                          # the last pass is a whole one
+    assert (m - 100) * k > 1 << 32
     w = make(torch, lib, n, k, 77)
     wr = repack(torch, lib, w, n, k)
     rng = np.random.default_rng(77)
@@ -219,3 +220,25 @@ def test_product_rows_past_32_bit_offsets(torch, lib, orc):
         assert float(y[64:m - 8].abs().max()) == 0.0
     del x, y
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n,k", [(544, 4128), (2064, 512), (100, 96)])
+@pytest.mark.parametrize("m", [512, 513, 580, 1024, 1100])
+def test_product_of_more_rows_than_a_pass(torch, lib, orc, n, k, m):
+    """Products run in passes of 512 rows: every row of the later ones is written, by the GEMM and
+    by passes of the 32-row kernel, in both layouts."""
+    w = make(torch, lib, n, k, m)
+    wr = repack(torch, lib, w, n, k)
+    rng = np.random.default_rng(n + m)
+    x = rng.normal(0, 1, (m, k)).astype(np.float16)
+    rows = w.cpu().numpy().reshape(n, k // 32, 34)
+    scale = rows[:, :, :2].copy().view(np.float16).astype(np.float32)
+    wide = (scale * rows[:, :, 2:].view(np.int8)).astype(np.float16).astype(np.float64).reshape(n, k)
+    want = x.astype(np.float64) @ wide.T                 # the oracle's product, on many rows at once
+    assert np.abs(want[-2:] - orc.q8_gemv_f64(w.cpu().numpy(), n, k, x[-2:].view(np.uint16))).max() < 1e-9
+    rms = np.sqrt((want ** 2).mean())
+    for fn, at in ((lib.aotx_q8_gemv, w), (lib.aotx_q8r_gemv, wr)):
+        y = torch.full((m, n), 7.0, dtype=torch.float32, device="cuda")
+        assert fn(p(at), n, k, p(dev(x, torch)), m, p(y), None) == 0
+        torch.cuda.synchronize()
+        assert np.abs(y.cpu().numpy() - want).max() < 1e-5 * max(rms, 1.0) * np.sqrt(k / 32.0)
