@@ -151,13 +151,13 @@ __global__ __launch_bounds__(64 * T * P, MT == 64 ? 2 : 4) void aotx_rgemv_wide(
             rg_wload<FILE, true>(a, wsrc, qq, lane, wr[BUF][qi]);                        \
         }                                                                                \
     } while (0)
-    /* branch-free: a quad past the range reads a valid x quad and has its scale zeroed */
+    /* branch-free: a quad past the range has its scale zeroed and its place in the chunk of x
+     * holds zeros (not a quad in range: 0 times its infinities would be NaN) */
 #define RGW_COMPUTE(BUF, N, XB)                                                          \
     do {                                                                                 \
         _Pragma("unroll") for (int qi = 0; qi < PDQ; ++qi) {                             \
             const unsigned int qq = RGW_QUAD((N) + (unsigned int)qi);                    \
-            const unsigned int qx = qq < q1 ? qq : q1 - 1u;                              \
-            const unsigned short *xq = (XB) + ((qx - q0) % KC) * 128u + 32u * g;         \
+            const unsigned short *xq = (XB) + ((qq - q0) % KC) * 128u + 32u * g;         \
             rg_h8 B[CB][4];                                                              \
             if (MT == 32)                                                                \
                 _Pragma("unroll") for (int t = 0; t < CB; ++t)                           \
@@ -642,7 +642,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ?
         }                                                                                \
     } while (0)
     /* x pieces of quad Q (a quad past the split repeats its last). TAIL: k ends inside the
-     * last quad; a piece past it reads the row's first and is stored as zeros */
+     * last quad; a piece past it reads the row's first, and that and a quad past the split are
+     * stored as zeros */
     rg_u4 xr[2][PPT];                             /* register buffer XB = Q & 1 holds quad Q */
 #define RGM_XLOAD(XB, Q)                                                                 \
     do {                                                                                 \
@@ -661,7 +662,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WIDE_REGS ?
         _Pragma("unroll") for (int i = 0; i < PPT; ++i)                                  \
             *(rg_u4 *)(xb_ + (unsigned int)i * RSTEP * XS) =                             \
                 xrow0 + (unsigned int)i * RSTEP < mrows                                  \
-                && (!TAIL || (Q) * 128u + xpc * 8u < a.k) ? xr[XB][i] : (rg_u4){0u, 0u, 0u, 0u}; \
+                && (!TAIL || ((Q) < qn && (Q) * 128u + xpc * 8u < a.k)) ? xr[XB][i] : (rg_u4){0u, 0u, 0u, 0u}; \
     } while (0)
 
     /* Quad q is computed from LDS x buffer q & 1 and weight buffer q & 1. Its step first

@@ -932,8 +932,8 @@ static __device__ __forceinline__ void rg_narrow(const aotx_rgemv_args &a, unsig
     } while (0)
 
     /* Branch-free: a quad past the wave's range reads the last quad's x and has its scale
-     * forced to zero (it adds nothing); a batch column past mrows reads row 0 of x (its
-     * results are never written). */
+     * forced to zero (it adds nothing; FILE: its x too, as 0 times an infinity would be NaN); a
+     * batch column past mrows reads row 0 of x (its results are never written). */
 #define RG_COMPUTE(BUF, QS)                                                              \
     do {                                                                                 \
         _Pragma("unroll") for (int qi = 0; qi < PD; ++qi) {                              \
@@ -944,8 +944,10 @@ static __device__ __forceinline__ void rg_narrow(const aotx_rgemv_args &a, unsig
             _Pragma("unroll") for (int t = 0; t < MT / 16; ++t) {                        \
                 const unsigned int mm = (unsigned int)t * 16u + r;                       \
                 const unsigned int mr = mm < mrows ? mm : 0u;                            \
-                _Pragma("unroll") for (int s = 0; s < 4; ++s)                            \
+                _Pragma("unroll") for (int s = 0; s < 4; ++s) {                          \
                     B[t][s] = *(const rg_h8 *)(xq + mr * xs + 8u * s);                   \
+                    if (FILE && qq >= wq1) B[t][s] = (rg_h8)(_Float16)0.0f;              \
+                }                                                                        \
             }                                                                            \
             _Pragma("unroll") for (int j = 0; j < RT; ++j) {                             \
                 unsigned int qd[8], sbits;                                               \

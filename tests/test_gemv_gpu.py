@@ -242,3 +242,25 @@ def test_product_of_more_rows_than_a_pass(torch, lib, orc, n, k, m):
         assert fn(p(at), n, k, p(dev(x, torch)), m, p(y), None) == 0
         torch.cuda.synchronize()
         assert np.abs(y.cpu().numpy() - want).max() < 1e-5 * max(rms, 1.0) * np.sqrt(k / 32.0)
+
+
+@pytest.mark.parametrize("n,k", [(48, 160), (300, 4128), (1000, 1056), (8200, 416), (4096, 4096)])
+@pytest.mark.parametrize("m", [1, 4, 8, 32, 64, 100])
+def test_file_product_of_infinities(torch, lib, n, k, m):
+    """An infinity in a row of x gives infinities of its weights' signs (NaN where the weight is
+    0, as in any sum of products), wherever it lies: at k that does not divide evenly among
+    waves, k splits or pairs of 128, by every kernel over the file's layout."""
+    w = make(torch, lib, n, k, n + k)
+    rows = w.cpu().numpy().reshape(n, k // 32, 34)
+    quant = rows[:, :, 2:].view(np.int8).reshape(n, k).astype(np.float32)
+    rng = np.random.default_rng(m + k)
+    for base in range(0, max(1, k // 32), max(1, m)):
+        x = rng.normal(0, 1, (m, k)).astype(np.float16)
+        at = np.array([((base + i) * 32 + rng.integers(32)) % k for i in range(m)])
+        x[np.arange(m), at] = np.where(rng.random(m) < 0.5, np.inf, -np.inf)
+        y = torch.zeros(m, n, dtype=torch.float32, device="cuda")
+        assert lib.aotx_q8_gemv(p(w), n, k, p(dev(x, torch)), m, p(y), None) == 0
+        torch.cuda.synchronize()
+        with np.errstate(invalid="ignore"):
+            want = quant[:, at].T * x[np.arange(m), at].astype(np.float32)[:, None]
+        assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
