@@ -414,10 +414,12 @@ static __device__ __forceinline__ float aotx_attn_max4(float v)
 /* One query row by one wave, the values of the positions it attends and no others: the rows
  * that the products left NaN. There a position that a row does not attend has weight 0, and 0
  * times a value of Inf or NaN (another sequence's, a later token's, or one past the sequence's
- * last position) is NaN. Rare and not fast: lanes over 64 positions for the scores, then over
- * the dimensions for the values, 32-bit weights. */
+ * last position) is NaN. Writes the dimensions [d0, d1), those that the wave wrote. Rare and not
+ * fast: lanes over 64 positions for the scores, then over the dimensions for the values, 32-bit
+ * weights. */
 template <int D>
-static __device__ void aotx_attend_row(const aotx_attn_args &a, unsigned int t, unsigned int kh, unsigned int h)
+static __device__ void aotx_attend_row(const aotx_attn_args &a, unsigned int t, unsigned int kh, unsigned int h,
+                                       unsigned int d0, unsigned int d1)
 {
     constexpr int E = D / 64;                        /* dimensions per lane */
     const unsigned int lane = threadIdx.x & 63u;
@@ -470,8 +472,292 @@ static __device__ void aotx_attend_row(const aotx_attn_args &a, unsigned int t, 
     }
     const float back = 1.0f / (l > 0.0f ? l : 1.0f);
 #pragma unroll
-    for (int e = 0; e < E; ++e)
-        a.out[aotx_attn_out_at(a, t, h, (unsigned int)e * 64u + lane, D)] = aotx_f2h(missing ? 0.0f : o[e] * back);
+    for (int e = 0; e < E; ++e) {
+        const unsigned int at = (unsigned int)e * 64u + lane;
+        if (at >= d0 && at < d1) a.out[aotx_attn_out_at(a, t, h, at, D)] = aotx_f2h(missing ? 0.0f : o[e] * back);
+    }
+}
+
+/* The addresses of a sequence's blocks, 64 at a time, one per lane. */
+struct aotx_attn_pages {
+    unsigned long long pages;
+    unsigned int base, agent, nblk;
+    bool held;
+};
+static __device__ __forceinline__ void aotx_attn_look(const aotx_attn_args &a, aotx_attn_pages &w, unsigned int pair)
+{
+    const unsigned int b0 = 2u * pair;
+    if (w.held && b0 + 1u - w.base < 64u) return;
+    w.held = true;
+    w.base = (unsigned int)__builtin_amdgcn_readfirstlane((int)b0);
+    /* (the first pair's divisions would be taken out of the loop over the sequences and kept) */
+    asm volatile("" : "+s"(w.base));
+    const unsigned int bl = w.base + (threadIdx.x & 63u);
+    w.pages = bl < w.nblk
+        ? (unsigned long long)aotx_kvl_block(a.shape, &a.state->kv, w.agent, a.layer, bl * 16u) : 0ull;
+}
+/* The scalar resource of block b (zero-size: loads return zeros) and whether it is missing. */
+static __device__ __forceinline__ __amdgpu_buffer_rsrc_t aotx_attn_block(const aotx_attn_args &a, const aotx_attn_pages &w,
+                                                                         unsigned int b, bool &gone)
+{
+    const unsigned int at = (b - w.base) & 63u;
+    const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)(w.pages >> 32), (int)at);
+    const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)w.pages, (int)at);
+    const unsigned long long pb = ((unsigned long long)hi << 32) | lo;
+    gone = pb == 0ull && b < w.nblk;
+    return __builtin_amdgcn_make_buffer_rsrc((void *)pb, (short)0, pb == 0ull ? 0 : (int)a.shape.block_bytes, 0x00020000);
+}
+
+/* A wave's NC tiles of 16 score columns and what it has added up for them. */
+template <int D, int NC>
+struct aotx_attn_cols {
+    aotx_h8a qb[NC][D / 32];
+    float mrun[NC];                                  /* column 16c + r */
+    aotx_f4a o[NC][D / 16], mass[NC];                /* columns 16c + 4g .. + 3 */
+    unsigned int plim[NC];                           /* column 16c + r: the positions it attends */
+    unsigned int *miss;                              /* [NC] in LDS: bit r, column 16c + r met a missing page */
+};
+template <int D, int NC>
+static __device__ __forceinline__ void aotx_attn_begin(aotx_attn_cols<D, NC> &s, unsigned int *miss)
+{
+    s.miss = miss;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        s.mrun[c] = -INFINITY;
+        miss[c] = 0u;                                /* the wave's own */
+        s.mass[c] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int cc = 0; cc < D / 16; ++cc) s.o[c][cc] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
+    }
+}
+
+/* Scores of pair p's blocks to weights, mass and the shifted accumulators; then the values at
+ * vw. EARLY: slices of the values read before the softmax, the others before the first products
+ * (with a wave's own loads in flight they cost registers that spill). masked: some column does
+ * not attend all of the pair's positions, or a block is missing. */
+template <int D, int NC, int EARLY>
+static __device__ __forceinline__ void aotx_attn_weigh(aotx_attn_cols<D, NC> &s, aotx_f4a (&scs)[NC][2], unsigned int p,
+                                                       bool gone0, bool gone1, bool masked, const unsigned short *vw,
+                                                       unsigned int lane)
+{
+    constexpr int NS = D / 16, VS = D + 8;
+    const unsigned int g = lane >> 4;
+    const float scale = 1.4426950408889634f / sqrtf((float)D);
+    /* the transposing read of a block's slice (see aotx_attend_body) */
+    const unsigned int vtr = (4u * g + (lane & 15u) / 4u) * VS + 4u * (lane & 3u);
+    const _Float16 one = (_Float16)1.0f;
+    const aotx_h8a ones = {one, one, one, one, one, one, one, one};
+    aotx_h8a vv[NS];
+    const auto values = [&](int cc) {
+        const aotx_s4a v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) aotx_s4a *)(vw + vtr + 16u * (unsigned int)cc));
+        const aotx_s4a v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) aotx_s4a *)(vw + 16u * VS + vtr + 16u * (unsigned int)cc));
+        vv[cc] = __builtin_bit_cast(aotx_h8a, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+#pragma unroll
+    for (int cc = 0; cc < EARLY; ++cc) values(cc);
+    if (EARLY != 0) __builtin_amdgcn_sched_barrier(0);
+    aotx_h8a pa[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        aotx_f4a *const sc = scs[c];
+        if (masked) {
+            if (gone0 || gone1)
+                s.miss[c] |= (unsigned int)__ballot((gone0 && 32u * p < s.plim[c]) || (gone1 && 32u * p + 16u < s.plim[c])) & 0xffffu;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const unsigned int at = 32u * p + 16u * (unsigned int)e + 4u * g + (unsigned int)i;
+                    if (at >= s.plim[c] || (e == 0 ? gone0 : gone1)) sc[e][i] = -INFINITY;
+                }
+        }
+        float mb = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])),
+                         fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
+        mb = aotx_attn_max4(mb) * scale;
+        const float mnew = fmaxf(s.mrun[c], mb);
+        /* a column with no position yet: weights and shift of 0 from -inf */
+        const float msafe = mnew == -INFINITY ? 0.0f : mnew;
+        const bool moved = mnew != s.mrun[c];
+        const float shift = moved ? aotx_exp2(s.mrun[c] - msafe) : 1.0f;
+        s.mrun[c] = mnew;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                pa[c][4 * e + i] = (_Float16)aotx_exp2(__builtin_fmaf(sc[e][i], scale, -msafe));
+        if (__any(moved)) {
+            float sh[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sh[i] = __shfl(shift, (int)(4u * g) + i, 64);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s.mass[c][i] *= sh[i];
+#pragma unroll
+                for (int cc = 0; cc < NS; ++cc) s.o[c][cc][i] *= sh[i];
+            }
+        }
+        s.mass[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[c], ones, s.mass[c], 0, 0, 0);
+    }
+#pragma unroll
+    for (int cc = EARLY; cc < NS; ++cc) values(cc);
+    if (EARLY != 0) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int cc = 0; cc < NS; ++cc)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            s.o[c][cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[c], vv[cc], s.o[c][cc], 0, 0, 0);
+}
+
+/* One sequence's blocks, the pairs part, part + PARTS, ... of them, by a wave that waits for no
+ * other: keys into registers and values through its own LDS slot vw. nmin: the positions that
+ * every column attends. */
+template <int D, int NC, int PARTS>
+static __device__ __forceinline__ void aotx_attn_walk(const aotx_attn_args &a, aotx_attn_cols<D, NC> &s, unsigned int agent,
+                                                      unsigned int n, unsigned int nmin, unsigned int kh,
+                                                      unsigned int part, unsigned short *vw, unsigned int lane)
+{
+    constexpr int KK = D / 32, VP = D / 32, VS = D + 8;
+    const unsigned int r = lane & 15u, g = lane >> 4;
+    const unsigned int kbyte = ((kh * AOTX_KVL_BLOCK + r) * D + 8u * g) * 2u;          /* A operand */
+    const unsigned int vbyte = ((a.kv_heads + kh) * AOTX_KVL_BLOCK * D + lane * 8u) * 2u;
+    aotx_attn_pages w = {0ull, 0u, agent, (n + 15u) / 16u, false};
+    const unsigned int pairs = (w.nblk + 1u) / 2u;
+    aotx_u4a kr[2][KK], vr[2][VP];
+    bool gone[2] = {false, false};
+    const auto load = [&](unsigned int p) {
+        aotx_attn_look(a, w, p);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const __amdgpu_buffer_rsrc_t rs = aotx_attn_block(a, w, 2u * p + (unsigned int)e, gone[e]);
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) kr[e][kk] = __builtin_amdgcn_raw_buffer_load_b128(rs, kbyte + kk * 64, 0, 0);
+#pragma unroll
+            for (int u = 0; u < VP; ++u) vr[e][u] = __builtin_amdgcn_raw_buffer_load_b128(rs, vbyte + u * 1024, 0, 0);
+        }
+    };
+    if (part < pairs) load(part);
+    for (unsigned int p = part; p < pairs; p += PARTS) {
+        aotx_f4a scs[NC][2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int u = 0; u < VP; ++u) {
+                const unsigned int piece = (unsigned int)u * 64u + lane;
+                *(aotx_u4a *)(vw + ((unsigned int)e * 16u + piece / (D / 8)) * VS + (piece % (D / 8)) * 8u) = vr[e][u];
+            }
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                scs[c][e] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk)
+                    scs[c][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(aotx_h8a, kr[e][kk]),
+                                                                       s.qb[c][kk], scs[c][e], 0, 0, 0);
+            }
+        const bool gone0 = gone[0], gone1 = gone[1];
+        /* the registers are used: the next pair's loads run under the rest of this step
+         * (unconditional: no copies where paths join) */
+        __builtin_amdgcn_sched_barrier(0);
+        load(p + PARTS);
+        __builtin_amdgcn_sched_barrier(0);
+        aotx_attn_weigh<D, NC, 0>(s, scs, p, gone0, gone1, 32u * p + 32u > nmin || gone0 || gone1, vw, lane);
+    }
+}
+
+/* The PARTS waves of one group of columns add their parts, in part order, and write the rows:
+ * column col is head kh G + col % G of token at(col), if that is below `tokens`. acc, pm, pl and
+ * pmiss are the group's LDS: [PARTS][16 NC][D] floats, [PARTS][16 NC] maxima and masses,
+ * [PARTS][NC] columns that met a missing page (acc may hold what the walks used: a barrier comes
+ * before its first write). Two barriers, which every wave of the workgroup meets. */
+template <int D, int G, int NC, int PARTS, class AT>
+static __device__ __forceinline__ void aotx_attn_finish(const aotx_attn_args &a, aotx_attn_cols<D, NC> &s, float *acc,
+                                                        float *pm, float *pl, unsigned int *pmiss, unsigned int part,
+                                                        unsigned int kh, unsigned int tokens, unsigned int lane, AT at)
+{
+    constexpr int NS = D / 16;
+    constexpr unsigned int COLS = 16u * NC, ACC = COLS * D;
+    constexpr int NP = NS >= PARTS ? NS / PARTS : 1;       /* d slices that a part adds up */
+    const unsigned int r = lane & 15u, g = lane >> 4;
+    /* maxima by column, masses by accumulator row (each lane group of a column saw all of its
+     * blocks) */
+    unsigned int missed = 0u;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        missed |= s.miss[c];
+        if (g == 0u) pm[part * COLS + 16u * (unsigned int)c + r] = s.mrun[c];
+        if (r == 0u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pl[part * COLS + 16u * (unsigned int)c + 4u * g + (unsigned int)i] = s.mass[c][i];
+    }
+    if (missed != 0u && lane == 0u) atomicAdd(&a.state->faults, 1u);
+    __syncthreads();
+    /* without branches: a part with no position has m = -inf, mass 0 and weight 2^-inf = 0 */
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned int col = 16u * (unsigned int)c + 4u * g + (unsigned int)i;
+            float m[PARTS], top = -INFINITY, sum = 0.0f;
+            unsigned int absent = 0u;
+#pragma unroll
+            for (unsigned int k = 0; k < (unsigned int)PARTS; ++k) {
+                m[k] = pm[k * COLS + col];
+                top = fmaxf(top, m[k]);
+                absent |= pmiss[k * NC + (unsigned int)c] >> (col & 15u);
+            }
+            top = top == -INFINITY ? 0.0f : top;
+#pragma unroll
+            for (unsigned int k = 0; k < (unsigned int)PARTS; ++k) sum += pl[k * COLS + col] * aotx_exp2(m[k] - top);
+            const float whole = 1.0f / (sum > 0.0f ? sum : 1.0f);
+            const float f = (absent & 1u) != 0u ? 0.0f : aotx_exp2(pm[part * COLS + col] - top) * whole;
+#pragma unroll
+            for (int cc = 0; cc < NS; ++cc)
+                acc[part * ACC + ((c * NS + cc) * 4 + i) * 64 + lane] = s.o[c][cc][i] * f;
+        }
+    __syncthreads();
+    /* part k adds the slices [k NP, (k + 1) NP) of all parts in part order */
+    if (part * (unsigned int)NP >= (unsigned int)NS) return;
+    unsigned int odd = 0u;                           /* bit 4c + i: NaN in this lane's column */
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const unsigned int col = 16u * (unsigned int)c + 4u * g + (unsigned int)i;
+            const unsigned int t = at(col);
+            float v[NP];
+            bool bad = false;
+#pragma unroll
+            for (int x = 0; x < NP; ++x) {
+                const unsigned int cc = part * (unsigned int)NP + (unsigned int)x;
+                v[x] = 0.0f;
+#pragma unroll
+                for (unsigned int k = 0; k < (unsigned int)PARTS; ++k)
+                    v[x] += acc[k * ACC + (((unsigned int)c * NS + cc) * 4u + (unsigned int)i) * 64u + lane];
+                bad = bad || v[x] != v[x];
+            }
+            if (t < tokens) {
+#pragma unroll
+                for (int x = 0; x < NP; ++x) {
+                    const unsigned int cc = part * (unsigned int)NP + (unsigned int)x;
+                    a.out[aotx_attn_out_at(a, t, kh * G + col % (unsigned int)G, 16u * cc + r, D)] = aotx_f2h(v[x]);
+                }
+                odd |= bad ? 1u << (4 * c + i) : 0u;
+            }
+        }
+    if (!__any(odd != 0u)) return;
+    const unsigned int d0 = part * (unsigned int)NP * 16u;
+#pragma unroll 1
+    for (unsigned int col = 0; col < COLS; ++col) {
+        /* column 16c + 4g + i: bit 4c + i of the 16 lanes of group g */
+        const bool mine = (odd >> (4u * (col / 16u) + col % 4u)) & 1u && g == col / 4u % 4u;
+        if (__any(mine)) {
+            const unsigned int t = (unsigned int)__builtin_amdgcn_readfirstlane((int)at(col));
+            aotx_attend_row<D>(a, t, kh, kh * G + col % (unsigned int)G, d0, d0 + (unsigned int)NP * 16u);
+        }
+    }
 }
 
 /* Batches with prompt pieces: a workgroup takes 16 NC H score columns of a KV head, the G
@@ -486,38 +772,48 @@ static __device__ void aotx_attend_row(const aotx_attn_args &a, unsigned int t, 
  *     (two transposing reads, shared by the tiles);
  *   - the mass is the product of the same fp16 weights with ones, on the matrix core, where it
  *     has the rows of the accumulators.
- * With one half (H = 1) a wave loads its pairs by itself, keys into registers and values
- * through its own LDS slot, and waits for no other wave. With two (H = 2) the halves of a part
- * load a block of the pair each into LDS for both, double-buffered, one barrier per pair: half
- * the reads from the L2s, which bound many columns otherwise. The next pair is on its way while
- * one is computed. The columns may be of several sequences: the workgroup goes over the blocks
- * of one after the other, and a column that does not take part keeps its state (but for values
- * that are not finite: aotx_attend_row).
+ * With one half (H = 1) a wave loads its pairs by itself (aotx_attn_walk). With two (H = 2) and
+ * one sequence the halves of a part load a block of the pair each into LDS for both,
+ * double-buffered, one barrier per pair: half the reads from the L2s, which bound many columns
+ * otherwise. The next pair is on its way while one is computed. Columns of several sequences:
+ * each half goes over the blocks of one sequence after the other by itself, and a column that
+ * does not take part keeps its state (but for values that are not finite: aotx_attend_row).
  * Bound by the softmax's vector work and the matrix work of a step, about 1600 cycles a wave.
  * Against a wave per 16 / G queries with one block per pass of softmax, at 32 / 8 heads x 128:
  * 512 tokens after 2000 cached ones 74.3 -> 42.8 us (H = 2; 55 with H = 1), a 512-token prompt
  * 21.7 -> 15.6, 256 tokens 14.6 -> 9.6, 128 tokens 10.8 -> 6.9, 200 tokens after 7800
- * 210 -> 78. Four tiles per wave at one wave per SIMD took 64 us in the first case. */
+ * 210 -> 78. Four tiles per wave at one wave per SIMD took 64 us in the first case.
+ *
+ * Tokens that are the only one of their run of a slot (decode rows beside a prompt piece, among
+ * the batch's first AOTX_RUN_SINGLES) are not columns of their place: walked there, their
+ * sequences would follow one another in the few workgroups of that range (63 rows at 2048
+ * positions beside a 449-token prompt 479 us, 366 by a wave per piece). Every workgroup takes its
+ * share of them at the end, a (token, KV head) at a time with the positions in 4 H parts: 108 us,
+ * where the keys and values alone (530 MB) take 88 at 6 TB/s. A launch without such tokens pays
+ * for the search 0.3 to 0.6 us (a 256-token prompt 10.0 -> 10.5, 512 tokens 16.5 -> 17.0). */
+#define AOTX_RUN_SINGLES 512u
 template <int D, int G, int NC, int H>
 static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a, unsigned int bx)
 {
     constexpr int KK = D / 32;                      /* score MFMA steps */
-    constexpr int NS = D / 16;                      /* d slices of the accumulators */
     constexpr int VP = D / 32;                      /* 16-byte pieces per lane and block */
     constexpr int VS = D + 8;                       /* LDS row stride (halves) */
     constexpr unsigned int TW = 16u * NC * H / G;   /* tokens */
-    constexpr unsigned int PARTS = 4u;
+    constexpr unsigned int PARTS = 4u, WAVES = PARTS * H;
     constexpr unsigned int COLS = 16u * NC;         /* columns of a half */
-    constexpr int NP = NS / (int)PARTS;             /* d slices that a part adds up */
-    static_assert(TW >= 1u && TW <= 64u && NS % (int)PARTS == 0, "a lane per token, a slice per part");
-    /* H = 1: the waves' value slots; H = 2: [buffer][part][keys, values] of a pair; after the
-     * loop the waves' accumulators */
+    static_assert(TW >= 1u && TW <= 64u && (TW & (TW - 1u)) == 0u && COLS % G == 0u,
+                  "a lane per token, whole tokens per half");
+    /* the waves' value slots; H = 2 with one sequence: [buffer][part][keys, values] of a pair;
+     * after the loop the waves' accumulators */
     constexpr unsigned int ROWS = 32u * VS * 2u, ACC = COLS * D * 4u;
     constexpr unsigned int STAGE = H == 1 ? PARTS * ROWS : 2u * PARTS * 2u * ROWS;
     __shared__ __attribute__((aligned(16))) unsigned char lds[STAGE > H * PARTS * ACC ? STAGE : H * PARTS * ACC];
-    __shared__ float pm[H][PARTS][COLS], pl[H][PARTS][COLS];
-    __shared__ unsigned int pmiss[H][PARTS][NC];
-    __shared__ unsigned int nan[H * NC];             /* each tile's columns that came out NaN */
+    __shared__ float pm[H * PARTS * COLS], pl[H * PARTS * COLS];
+    __shared__ unsigned int pmiss[H * PARTS * NC];
+    constexpr unsigned int WORDS = AOTX_RUN_SINGLES / 64u;
+    __shared__ unsigned long long same[WORDS];       /* bit t: token t + 1 is of the same slot */
+    __shared__ unsigned int lag[64], lps[64];        /* the tokens' slots and positions: the walks leave no
+                                                        registers for them (every wave writes the same) */
 
     const unsigned int lane = threadIdx.x & 63u;
     /* a scalar, so that the wave's blocks, loads and tests are scalar too */
@@ -525,224 +821,105 @@ static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a,
     const unsigned int part = wave % PARTS, half = H == 1 ? 0u : wave / PARTS;
     const unsigned int r = lane & 15u, g = lane >> 4;
     const unsigned int counted = aotx_attn_scalar(a.m_dev != nullptr ? a.m_dev : a.pos);
-    unsigned int tokens = a.m_dev != nullptr ? counted : a.tokens;
-    if (tokens > a.tokens) tokens = a.tokens;
     const unsigned int kh = bx % a.kv_heads;
     const unsigned int t0 = (bx / a.kv_heads) * TW;             /* the workgroup's first token */
+    /* lane i holds the slot and position of token t0 + i and its neighbours' slots; all words are
+     * read before the row count is known (below the launch's capacity every one exists), in one
+     * round trip with those of the batch's first tokens */
+    const auto slot_of = [&](unsigned int t) { return a.agent[t < a.tokens ? t : a.tokens - 1u]; };
+    const unsigned int tl = t0 + (lane < TW ? lane : 0u);
+    const unsigned int ag = slot_of(tl), ag0 = slot_of(tl != 0u ? tl - 1u : 0u), ag1 = slot_of(tl + 1u);
+    const unsigned int ps = a.pos[tl < a.tokens ? tl : a.tokens - 1u];
+    constexpr unsigned int ROUNDS = WORDS / WAVES;
+    unsigned int b0[ROUNDS], b1[ROUNDS];
+#pragma unroll
+    for (unsigned int i = 0u; i < ROUNDS; ++i) {
+        b0[i] = slot_of(i * 64u * WAVES + threadIdx.x);
+        b1[i] = slot_of(i * 64u * WAVES + threadIdx.x + 1u);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    unsigned int tokens = a.m_dev != nullptr ? counted : a.tokens;
+    if (tokens > a.tokens) tokens = a.tokens;
     if (t0 >= tokens) return;
-    /* lane i holds the slot and position of token t0 + i */
-    const bool live = lane < TW && t0 + lane < tokens;
-    const unsigned int tl = live ? t0 + lane : t0;
-    const unsigned int ag = a.agent[tl], ps = a.pos[tl];
-    const unsigned long long all = __ballot(live);
-    unsigned long long left = all;
-    if (threadIdx.x < (unsigned int)(H * NC)) nan[threadIdx.x] = 0u;
-
-    const unsigned int c0 = half * COLS;                        /* this half's first column */
-    aotx_h8a qb[NC][KK];
+    const bool live = lane < TW && tl < tokens;
+    const bool apart = tl < AOTX_RUN_SINGLES && (tl == 0u || ag0 != ag) && (tl + 1u == tokens || ag1 != ag);
+    const unsigned long long batch = __ballot(live), all = __ballot(live && !apart);
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        const unsigned int col = c0 + 16u * (unsigned int)c + r;
-        const unsigned int tc = col / (unsigned int)G, hh = col % (unsigned int)G;
-        /* a column past the batch reads its last token's query (its results are not written) */
-        const unsigned int tq = t0 + tc < tokens ? t0 + tc : tokens - 1u;
-        const unsigned short *q = a.q + ((unsigned long long)tq * a.heads + kh * G + hh) * D + 8u * g;
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk) qb[c][kk] = __builtin_bit_cast(aotx_h8a, co_load4(q + 32 * kk));
+    for (unsigned int i = 0u; i < ROUNDS; ++i) {
+        const unsigned long long e = __ballot(i * 64u * WAVES + threadIdx.x + 1u < tokens && b0[i] == b1[i]);
+        if (lane == 0u) same[i * WAVES + wave] = e;
     }
-    const aotx_kv_table *kv = &a.state->kv;
-    const float scale = 1.4426950408889634f / sqrtf((float)D);
-    const unsigned int kbyte = ((kh * AOTX_KVL_BLOCK + r) * D + 8u * g) * 2u;          /* A operand */
-    const unsigned int kbase = (kh * AOTX_KVL_BLOCK * D + lane * 8u) * 2u;             /* whole rows */
-    const unsigned int vbase = ((a.kv_heads + kh) * AOTX_KVL_BLOCK * D + lane * 8u) * 2u;
-    /* the transposing read of a block's slice (see aotx_attend_body) */
-    const unsigned int vtr = (4u * g + (lane & 15u) / 4u) * VS + 4u * (lane & 3u);
+    lag[lane] = ag;
+    lps[lane] = ps;
 
-    float mrun[NC];                                  /* column 16c + r */
-    aotx_f4a o[NC][NS], mass[NC];                    /* columns 16c + 4g .. + 3 */
-    unsigned int miss[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        mrun[c] = -INFINITY;
-        miss[c] = 0u;
-        mass[c] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int cc = 0; cc < NS; ++cc) o[c][cc] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    const _Float16 one = (_Float16)1.0f;
-    const aotx_h8a ones = {one, one, one, one, one, one, one, one};
-
-    while (left != 0ull) {
-        /* the tokens of one sequence, in any order of positions */
-        const unsigned int agent = (unsigned int)__builtin_amdgcn_readlane((int)ag, __builtin_ctzll(left));
-        const unsigned long long group = __ballot(ag == agent) & left;
-        const bool whole = group == all;                 /* the workgroup's only sequence */
-        left &= ~group;
-        /* the positions attended: by any token (n) and by every one (nmin) */
-        const bool in = (group >> lane) & 1ull;
-        unsigned int n = in ? ps + 1u : 0u, nmin = in ? ps + 1u : 0xFFFFFFFFu;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            const unsigned int on = (unsigned int)__shfl_xor((int)n, d, 64), om = (unsigned int)__shfl_xor((int)nmin, d, 64);
-            n = on > n ? on : n;
-            nmin = om < nmin ? om : nmin;
-        }
-        n = (unsigned int)__builtin_amdgcn_readfirstlane((int)n);
-        nmin = (unsigned int)__builtin_amdgcn_readfirstlane((int)nmin);
-        unsigned int plim[NC];
+    if (all != 0ull) {
+        const unsigned int c0 = half * COLS;                    /* this half's first column */
+        aotx_attn_cols<D, NC> s;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-            const unsigned int tc = (c0 + 16u * (unsigned int)c + r) / (unsigned int)G;
-            const unsigned int pt = (unsigned int)__shfl((int)ps, (int)tc, 64) + 1u;
-            plim[c] = (group >> tc) & 1ull ? pt : 0u;
-        }
-        const unsigned int nblk = (n + 15u) / 16u, pairs = (nblk + 1u) / 2u;
-        unsigned long long pages = 0ull;
-        unsigned int wbase = 0u;
-        bool window = false;
-        /* the scalar resource of block BI (zero-size: loads return zeros) and whether it is
-         * missing; the window holds the addresses of 64 blocks, one per lane */
-        const auto block = [&](unsigned int bi, bool &gone) {
-            const unsigned int at = (bi - wbase) & 63u;
-            const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)(pages >> 32), (int)at);
-            const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)pages, (int)at);
-            const unsigned long long pb = ((unsigned long long)hi << 32) | lo;
-            gone = pb == 0ull && bi < nblk;
-            return __builtin_amdgcn_make_buffer_rsrc((void *)pb, (short)0, pb == 0ull ? 0 : (int)a.shape.block_bytes,
-                                                     0x00020000);
-        };
-        const auto look = [&](unsigned int pair) {
-            const unsigned int b0 = 2u * pair;
-            if (window && b0 + 1u - wbase < 64u) return;
-            window = true;
-            wbase = (unsigned int)__builtin_amdgcn_readfirstlane((int)b0);
-            const unsigned int bl = wbase + lane;
-            pages = bl < nblk ? (unsigned long long)aotx_kvl_block(a.shape, kv, agent, a.layer, bl * 16u) : 0ull;
-        };
-        /* scores of a pair's blocks to weights, mass and the shifted accumulators; then the
-         * values at vw */
-        const auto weigh = [&](aotx_f4a (&scs)[NC][2], const unsigned int p, const bool gone0, const bool gone1,
-                               const unsigned short *vw) {
-            const bool masked = !whole || 32u * p + 32u > nmin || gone0 || gone1;
-            /* two halves: the first half of the values is read before the softmax, the second
-             * before the first products (with one half it costs registers that spill) */
-            constexpr int EARLY = H == 2 ? NS / 2 : 0;
-            aotx_h8a vv[NS];
-            const auto values = [&](int cc) {
-                const aotx_s4a v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (__attribute__((address_space(3))) aotx_s4a *)(vw + vtr + 16u * (unsigned int)cc));
-                const aotx_s4a v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (__attribute__((address_space(3))) aotx_s4a *)(vw + 16u * VS + vtr + 16u * (unsigned int)cc));
-                vv[cc] = __builtin_bit_cast(aotx_h8a, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-            };
+            const unsigned int col = c0 + 16u * (unsigned int)c + r;
+            const unsigned int tc = col / (unsigned int)G, hh = col % (unsigned int)G;
+            /* a column past the batch reads its last token's query (its results are not written) */
+            const unsigned int tq = t0 + tc < tokens ? t0 + tc : tokens - 1u;
+            const unsigned short *q = a.q + ((unsigned long long)tq * a.heads + kh * G + hh) * D + 8u * g;
 #pragma unroll
-            for (int cc = 0; cc < EARLY; ++cc) values(cc);
-            if (H == 2) __builtin_amdgcn_sched_barrier(0);
-            aotx_h8a pa[NC];
+            for (int kk = 0; kk < KK; ++kk) s.qb[c][kk] = __builtin_bit_cast(aotx_h8a, co_load4(q + 32 * kk));
+        }
+        aotx_attn_begin(s, pmiss + (half * PARTS + part) * NC);
+        /* the tokens `group` of slot `agent`, in any order of positions: the positions attended by
+         * any of them (n) and by every column (nmin, 0 if a column is another's) */
+        unsigned int agent = 0u, n = 0u, nmin = 0u;
+        const auto sequence = [&](unsigned long long group, unsigned long long columns, unsigned int ps) {
+            const bool in = (group >> lane) & 1ull;
+            n = in ? ps + 1u : 0u;
+            nmin = in ? ps + 1u : 0xFFFFFFFFu;
+#pragma unroll
+            for (int d = (int)TW / 2; d >= 1; d >>= 1) {              /* over the tokens' lanes */
+                const unsigned int on = (unsigned int)__shfl_xor((int)n, d, 64), om = (unsigned int)__shfl_xor((int)nmin, d, 64);
+                n = on > n ? on : n;
+                nmin = om < nmin ? om : nmin;
+            }
+            n = (unsigned int)__builtin_amdgcn_readfirstlane((int)n);
+            nmin = group == columns ? (unsigned int)__builtin_amdgcn_readfirstlane((int)nmin) : 0u;
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
-                aotx_f4a *const sc = scs[c];
-                if (masked) {
-                    if (gone0 && 32u * p < plim[c]) miss[c] = 1u;
-                    if (gone1 && 32u * p + 16u < plim[c]) miss[c] = 1u;
-#pragma unroll
-                    for (int e = 0; e < 2; ++e)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const unsigned int at = 32u * p + 16u * (unsigned int)e + 4u * g + (unsigned int)i;
-                            if (at >= plim[c] || (e == 0 ? gone0 : gone1)) sc[e][i] = -INFINITY;
-                        }
-                }
-                float mb = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])),
-                                 fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
-                mb = aotx_attn_max4(mb) * scale;
-                const float mnew = fmaxf(mrun[c], mb);
-                /* a column with no position yet: weights and shift of 0 from -inf */
-                const float msafe = mnew == -INFINITY ? 0.0f : mnew;
-                const bool moved = mnew != mrun[c];
-                const float shift = moved ? aotx_exp2(mrun[c] - msafe) : 1.0f;
-                mrun[c] = mnew;
-#pragma unroll
-                for (int e = 0; e < 2; ++e)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        pa[c][4 * e + i] = (_Float16)aotx_exp2(__builtin_fmaf(sc[e][i], scale, -msafe));
-                if (__any(moved)) {
-                    float sh[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) sh[i] = __shfl(shift, (int)(4u * g) + i, 64);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        mass[c][i] *= sh[i];
-#pragma unroll
-                        for (int cc = 0; cc < NS; ++cc) o[c][cc][i] *= sh[i];
-                    }
-                }
-                mass[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[c], ones, mass[c], 0, 0, 0);
+                const unsigned int tc = (c0 + 16u * (unsigned int)c + r) / (unsigned int)G;
+                const unsigned int pt = (unsigned int)__shfl((int)ps, (int)tc, 64) + 1u;
+                s.plim[c] = (group >> tc) & 1ull ? pt : 0u;
             }
-#pragma unroll
-            for (int cc = EARLY; cc < NS; ++cc) values(cc);
-            if (H == 2) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int cc = 0; cc < NS; ++cc)
-#pragma unroll
-                for (int c = 0; c < NC; ++c)
-                    o[c][cc] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[c], vv[cc], o[c][cc], 0, 0, 0);
         };
-        if constexpr (H == 1) {
-            unsigned short *const vw = (unsigned short *)(lds + part * ROWS);
-            aotx_u4a kr[2][KK], vr[2][VP];
-            bool gone[2] = {false, false};
-            const auto load = [&](unsigned int p) {
-                look(p);
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const __amdgpu_buffer_rsrc_t rs = block(2u * p + (unsigned int)e, gone[e]);
-#pragma unroll
-                    for (int kk = 0; kk < KK; ++kk) kr[e][kk] = __builtin_amdgcn_raw_buffer_load_b128(rs, kbyte + kk * 64, 0, 0);
-#pragma unroll
-                    for (int u = 0; u < VP; ++u) vr[e][u] = __builtin_amdgcn_raw_buffer_load_b128(rs, vbase + u * 1024, 0, 0);
-                }
-            };
-            if (part < pairs) load(part);
-            for (unsigned int p = part; p < pairs; p += PARTS) {
-                aotx_f4a scs[NC][2];
-#pragma unroll
-                for (int e = 0; e < 2; ++e)
-#pragma unroll
-                    for (int u = 0; u < VP; ++u) {
-                        const unsigned int piece = (unsigned int)u * 64u + lane;
-                        *(aotx_u4a *)(vw + ((unsigned int)e * 16u + piece / (D / 8)) * VS + (piece % (D / 8)) * 8u) = vr[e][u];
-                    }
-#pragma unroll
-                for (int e = 0; e < 2; ++e)
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) {
-                        scs[c][e] = (aotx_f4a){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                        for (int kk = 0; kk < KK; ++kk)
-                            scs[c][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(aotx_h8a, kr[e][kk]),
-                                                                               qb[c][kk], scs[c][e], 0, 0, 0);
-                    }
-                const bool gone0 = gone[0], gone1 = gone[1];
-                /* the registers are used: the next pair's loads run under the rest of this
-                 * step (unconditional: no copies where paths join) */
-                __builtin_amdgcn_sched_barrier(0);
-                load(p + PARTS);
-                __builtin_amdgcn_sched_barrier(0);
-                weigh(scs, p, gone0, gone1, vw);
+        agent = (unsigned int)__builtin_amdgcn_readlane((int)ag, __builtin_ctzll(all));
+        const unsigned long long first = __ballot(ag == agent) & all;
+        if (H == 1 || first != all) {
+            /* the tokens of this half's columns */
+            const unsigned long long here = COLS / G >= 64u ? ~0ull : ((1ull << (COLS / G)) - 1ull) << (c0 / G);
+            unsigned long long left = all & here;
+            while (left != 0ull) {
+                unsigned int li = lane;
+                asm volatile("" : "+v"(li));         /* read from LDS, not kept from where it was stored */
+                const unsigned int al = lag[li];
+                agent = (unsigned int)__builtin_amdgcn_readlane((int)al, __builtin_ctzll(left));
+                const unsigned long long group = __ballot(al == agent) & left;
+                left &= ~group;
+                sequence(group, batch & here, lps[li]);
+                aotx_attn_walk<D, NC, (int)PARTS>(a, s, agent, n, nmin, kh, part, (unsigned short *)(lds + wave * ROWS), lane);
             }
-        } else {
+        } else if constexpr (H == 2) {
             /* a wave brings block `half` of its part's pair; every wave meets every barrier */
+            sequence(first, batch, ps);
+            aotx_attn_pages w = {0ull, 0u, agent, (n + 15u) / 16u, false};
+            const unsigned int pairs = (w.nblk + 1u) / 2u;
+            const unsigned int kbase = (kh * AOTX_KVL_BLOCK * D + lane * 8u) * 2u;             /* whole rows */
+            const unsigned int vbase = ((a.kv_heads + kh) * AOTX_KVL_BLOCK * D + lane * 8u) * 2u;
             const auto slot = [&](unsigned int buf, unsigned int what) {
                 return (unsigned short *)(lds + ((buf * PARTS + part) * 2u + what) * ROWS);
             };
             aotx_u4a kl[VP], vr[VP];
             bool gone[2] = {false, false};
             const auto load = [&](unsigned int p) {
-                look(p);
+                aotx_attn_look(a, w, p);
                 bool g0, g1;
-                const __amdgpu_buffer_rsrc_t r0 = block(2u * p, g0), r1 = block(2u * p + 1u, g1);
+                const __amdgpu_buffer_rsrc_t r0 = aotx_attn_block(a, w, 2u * p, g0), r1 = aotx_attn_block(a, w, 2u * p + 1u, g1);
                 gone[0] = g0;
                 gone[1] = g1;
                 const __amdgpu_buffer_rsrc_t rs = half == 0u ? r0 : r1;
@@ -760,9 +937,8 @@ static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a,
                     *(aotx_u4a *)(slot(buf, 1u) + at) = vr[u];
                 }
             };
-            const bool mine = group >> (c0 / G) << (64u - (COLS + G - 1u) / G) != 0ull;   /* any column here */
+            const bool mine = first >> (c0 / G) << (64u - (COLS + G - 1u) / G) != 0ull;   /* any column here */
             load(part);
-            __syncthreads();          /* the sequence before is read */
             store(0u);
             __syncthreads();
             const unsigned int steps = (pairs + PARTS - 1u) / PARTS;
@@ -791,88 +967,66 @@ static __device__ __forceinline__ void aotx_attend_runs(const aotx_attn_args &a,
                         for (int e = 0; e < 2; ++e)
 #pragma unroll
                             for (int c = 0; c < NC; ++c)
-                                scs[c][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8[e][kk], qb[c][kk], scs[c][e], 0, 0, 0);
-                    weigh(scs, p, gone0, gone1, slot(st & 1u, 1u));
+                                scs[c][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8[e][kk], s.qb[c][kk], scs[c][e], 0, 0, 0);
+                    aotx_attn_weigh<D, NC, D / 32>(s, scs, p, gone0, gone1, 32u * p + 32u > nmin || gone0 || gone1, slot(st & 1u, 1u), lane);
                 }
                 store((st + 1u) & 1u);
                 __syncthreads();
             }
         }
+        const auto token = [&](unsigned int col) {
+            const unsigned int tc = (c0 + col) / (unsigned int)G;
+            return (all >> tc) & 1ull ? t0 + tc : 0xFFFFFFFFu;
+        };
+        aotx_attn_finish<D, G, NC, (int)PARTS>(a, s, (float *)lds + half * PARTS * (ACC / 4u), pm + half * PARTS * COLS,
+                                               pl + half * PARTS * COLS, pmiss + half * PARTS * NC, part, kh, tokens, lane, token);
+    } else {
+        __syncthreads();                             /* `same` is there */
     }
-    if (H == 2) __syncthreads();
-    /* the parts: maxima by column, masses by accumulator row, and which columns met a missing
-     * page (each lane group of a column saw all of its blocks) */
-    unsigned long long missed = 0ull;
+
+    /* a lane number of its own, so that no address made from it is kept in registers over the
+     * walks above, which have none to spare */
+    unsigned int ln = threadIdx.x & 63u;
+    asm volatile("" : "+v"(ln));
+    /* the tokens apart, lane i those of 64i .. 64i + 63 */
+    const unsigned int wi = ln < WORDS ? lane : 0u, past = 64u * wi < tokens ? tokens - 64u * wi : 0u;
+    const unsigned long long e = same[wi], e0 = wi != 0u ? same[wi - 1u] >> 63 : 0ull;
+    const unsigned long long alone = ln < WORDS ? ~e & ~(e << 1 | e0) & (past >= 64u ? ~0ull : (1ull << past) - 1ull) : 0ull;
+    if (!__any(alone != 0ull)) return;
+    /* (token, KV head) number u to workgroup u mod the workgroups with tokens */
+    const unsigned int groups = (tokens + TW - 1u) / TW * a.kv_heads;
+    const unsigned int mine = (unsigned int)__builtin_popcountll(alone);
+    unsigned int upto = mine;                        /* those of this lane's word and the ones before */
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        const unsigned long long mc = __ballot(miss[c] != 0u);
-        missed |= mc;
-        if (lane == 0u) pmiss[half][part][c] = (unsigned int)mc & 0xffffu;
-        if (g == 0u) pm[half][part][16u * (unsigned int)c + r] = mrun[c];
-        if (r == 0u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) pl[half][part][16u * (unsigned int)c + 4u * g + (unsigned int)i] = mass[c][i];
+    for (unsigned int d = 1u; d < WORDS; d <<= 1) {
+        const unsigned int o = (unsigned int)__shfl_up((int)upto, d, 64);
+        if (ln >= d) upto += o;
     }
-    if (missed != 0ull && lane == 0u) atomicAdd(&a.state->faults, 1u);
-    __syncthreads();
-    /* without branches: a part with no position has m = -inf, mass 0 and weight 2^-inf = 0 */
-    float *const acc = (float *)lds + (half * PARTS) * (ACC / 4u);
+    const unsigned int units = (unsigned int)__builtin_amdgcn_readlane((int)upto, (int)WORDS - 1) * a.kv_heads;
+    for (unsigned int u = bx; u < units; u += groups) {
+        /* the k-th of them: in the first word that reaches past k */
+        unsigned int k = u / a.kv_heads;
+        const unsigned int word = (unsigned int)__builtin_ctzll(__ballot(ln < WORDS && upto > k));
+        k -= (unsigned int)__builtin_amdgcn_readlane((int)(upto - mine), (int)word);
+        unsigned long long bits = (unsigned long long)(unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)(alone >> 32), (int)word) << 32
+                                | (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)alone, (int)word);
+        for (; k != 0u; --k) bits &= bits - 1ull;
+        const unsigned int t = word * 64u + (unsigned int)__builtin_ctzll(bits);
+        const unsigned int uh = u % a.kv_heads;
+        const unsigned int agent = (unsigned int)__builtin_amdgcn_readfirstlane((int)a.agent[t]);
+        const unsigned int n = (unsigned int)__builtin_amdgcn_readfirstlane((int)a.pos[t]) + 1u;
+        /* G columns; the others repeat them and are not written */
+        aotx_attn_cols<D, 1> s;
+        const unsigned short *q = a.q + ((unsigned long long)t * a.heads + uh * G + (ln & 15u) % (unsigned int)G) * D + 8u * (ln >> 4);
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const unsigned int col = 16u * (unsigned int)c + 4u * g + (unsigned int)i;
-            float m[PARTS], top = -INFINITY, sum = 0.0f;
-            unsigned int absent = 0u;
-#pragma unroll
-            for (unsigned int k = 0; k < PARTS; ++k) {
-                m[k] = pm[half][k][col];
-                top = fmaxf(top, m[k]);
-                absent |= pmiss[half][k][c] >> (col & 15u);
-            }
-            top = top == -INFINITY ? 0.0f : top;
-#pragma unroll
-            for (unsigned int k = 0; k < PARTS; ++k) sum += pl[half][k][col] * aotx_exp2(m[k] - top);
-            const float whole = 1.0f / (sum > 0.0f ? sum : 1.0f);
-            const float f = (absent & 1u) != 0u ? 0.0f : aotx_exp2(pm[half][part][col] - top) * whole;
-#pragma unroll
-            for (int cc = 0; cc < NS; ++cc)
-                acc[part * (ACC / 4u) + ((c * NS + cc) * 4 + i) * 64 + lane] = o[c][cc][i] * f;
-        }
-    __syncthreads();
-    /* part k adds the slices [k NP, (k + 1) NP) of all parts in part order */
-    bool odd = false;
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const unsigned int col = c0 + 16u * (unsigned int)c + 4u * g + (unsigned int)i;
-            const unsigned int tc = col / (unsigned int)G, hc = col % (unsigned int)G;
-            float v[NP];
-            bool bad = false;
-#pragma unroll
-            for (int s = 0; s < NP; ++s) {
-                const unsigned int cc = part * (unsigned int)NP + (unsigned int)s;
-                v[s] = 0.0f;
-#pragma unroll
-                for (unsigned int k = 0; k < PARTS; ++k)
-                    v[s] += acc[k * (ACC / 4u) + (((unsigned int)c * NS + cc) * 4u + (unsigned int)i) * 64u + lane];
-                bad = bad || v[s] != v[s];
-            }
-            if (t0 + tc < tokens) {
-#pragma unroll
-                for (int s = 0; s < NP; ++s) {
-                    const unsigned int cc = part * (unsigned int)NP + (unsigned int)s;
-                    a.out[aotx_attn_out_at(a, t0 + tc, kh * G + hc, 16u * cc + r, D)] = aotx_f2h(v[s]);
-                }
-                if (bad) atomicOr(nan + col / 16u, 1u << (col % 16u));
-                odd = odd || bad;
-            }
-        }
-    if (!__syncthreads_or(odd)) return;
-    for (unsigned int col = wave; col < 16u * NC * H; col += PARTS * H)
-        if ((nan[col / 16u] >> (col % 16u)) & 1u)
-            aotx_attend_row<D>(a, t0 + col / (unsigned int)G, kh, kh * G + col % (unsigned int)G);
+        for (int kk = 0; kk < KK; ++kk) s.qb[0][kk] = __builtin_bit_cast(aotx_h8a, co_load4(q + 32 * kk));
+        s.plim[0] = n;
+        __syncthreads();                             /* the accumulators before are read */
+        aotx_attn_begin(s, pmiss + wave);
+        aotx_attn_walk<D, 1, (int)WAVES>(a, s, agent, n, n, uh, wave, (unsigned short *)(lds + wave * ROWS), ln);
+        aotx_attn_finish<D, G, 1, (int)WAVES>(a, s, (float *)lds, pm, pl, pmiss, wave, uh, tokens, ln,
+                                              [&](unsigned int col) { return col < (unsigned int)G ? t : 0xFFFFFFFFu; });
+    }
 }
 
 #undef MMA_WINDOW

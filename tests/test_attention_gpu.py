@@ -186,22 +186,29 @@ def test_kv_release_and_reuse(torch, lib):
         lib.aotx_kv_close(ctypes.byref(m))
 
 
+# the three forms of a launch with prompt pieces (score columns of a workgroup), by its tokens x heads
+_FORMS = {"16": (0, 6144), "32": (6144, 12288), "64": (12288, 1 << 30)}
+
+
+def _is_form(form, tokens, heads):
+    return _FORMS[form][0] <= tokens * heads < _FORMS[form][1]
+
+
 # (slot, cached positions before the piece, piece length)
 _PIECES = [(3, 0, 57), (9, 13, 30), (21, 0, 1), (40, 301, 49), (5, 7, 3), (63, 1000, 1)]
-# 20 decode rows side by side (a 16-token range of the launch leads 16 pieces, so each
-# wave takes several), then a prompt
+# 20 decode rows side by side, then a prompt
 _SINGLES = [(10 + i, 5 * i + 2, 1) for i in range(20)] + [(50, 3, 117)]
 
 
 @pytest.mark.parametrize("layout", ["pieces", "singles"])
-@pytest.mark.parametrize("heads,kvh,d", [(32, 8, 128), (16, 2, 64), (8, 8, 64)])
-def test_attend_prompt_pieces_vs_oracle(torch, lib, orc, heads, kvh, d, layout):
+@pytest.mark.parametrize("form,heads,kvh,d", [("16", 32, 8, 128), ("16", 16, 2, 64), ("16", 8, 8, 64), ("32", 64, 16, 128),
+                                              ("32", 48, 48, 64), ("64", 96, 24, 128), ("64", 96, 96, 64), ("64", 96, 12, 64)])
+def test_attend_prompt_pieces_vs_oracle(torch, lib, orc, form, heads, kvh, d, layout):
     """A launch of 128 tokens or more (prompt pieces: more tokens than sequence slots) runs
-    the piece kernel, where one wave takes up to 16 / G consecutive queries of one sequence
-    on a single pass over their keys: pieces that start mid-cache at positions that are
-    not multiples of 16 / G, a run cut by the next sequence, single decode rows (many in
-    one workgroup's range), causal limits per query; every (token, head) vs the oracle's
-    online softmax at its own position."""
+    the piece kernel, a workgroup per 16, 32 or 64 score columns of a KV head: pieces that start
+    mid-cache, several sequences in a workgroup, single decode rows (many in one workgroup's
+    range), causal limits per query; every (token, head) vs the oracle's online softmax at its
+    own position."""
     layers, layer = 2, 0
     rng = np.random.default_rng(heads + kvh + d)
     pieces = _PIECES if layout == "pieces" else _SINGLES
@@ -216,7 +223,7 @@ def test_attend_prompt_pieces_vs_oracle(torch, lib, orc, heads, kvh, d, layout):
         pos = np.concatenate([np.arange(c, c + n) for _, c, n in pieces]).astype(np.uint32)
         ag = np.concatenate([np.full(n, s) for s, _, n in pieces]).astype(np.uint32)
         tokens = len(pos)
-        assert tokens >= 128
+        assert tokens >= 128 and _is_form(form, tokens, heads)
         q = rng.normal(0, 1, (tokens, heads, d)).astype(np.float16)
         out = torch.zeros(tokens * heads * d, dtype=torch.float16, device="cuda")
         lib.aotx_model_forget()
@@ -238,11 +245,13 @@ def test_attend_prompt_pieces_vs_oracle(torch, lib, orc, heads, kvh, d, layout):
         lib.aotx_kv_close(ctypes.byref(m))
 
 
-@pytest.mark.parametrize("heads,kvh,d", [(16, 8, 128), (8, 8, 128), (16, 2, 128), (8, 2, 64)])
-def test_attend_prompt_edges_vs_oracle(torch, lib, orc, heads, kvh, d):
+@pytest.mark.parametrize("form,heads,kvh,d", [("16", 16, 8, 128), ("16", 8, 8, 128), ("16", 16, 2, 128), ("16", 8, 2, 64),
+                                              ("32", 64, 16, 128), ("32", 48, 48, 64), ("32", 64, 8, 64), ("64", 96, 24, 128),
+                                              ("64", 96, 96, 64), ("64", 96, 48, 64), ("64", 96, 12, 128)])
+def test_attend_prompt_edges_vs_oracle(torch, lib, orc, form, heads, kvh, d):
     """The batch kernel's edges: contexts around the pairs of blocks that a wave takes in turn
     (1, 16, 17, 32, 33, 127..129 positions), past the 1024 positions of a window of page
-    addresses, positions of one sequence out of order, tokens that end inside a wave's 32
+    addresses, positions of one sequence out of order, tokens that end inside a workgroup's
     columns; and a slot without pages, whose rows are zero while its neighbours' are right and
     the fault count grows."""
     layers, layer = 2, 1
@@ -263,7 +272,7 @@ def test_attend_prompt_edges_vs_oracle(torch, lib, orc, heads, kvh, d):
         pos = np.insert(pos, 40, 100).astype(np.uint32)
         ag = np.insert(ag, 40, 33).astype(np.uint32)
         tokens = len(pos)
-        assert tokens >= 128 and tokens % 4 != 0
+        assert tokens >= 128 and tokens % 4 != 0 and _is_form(form, tokens, heads)
         q = rng.normal(0, 1, (tokens, heads, d)).astype(np.float16)
         out = torch.full((tokens * heads * d,), 7.0, dtype=torch.float16, device="cuda")
         lib.aotx_model_forget()
@@ -286,10 +295,6 @@ def test_attend_prompt_edges_vs_oracle(torch, lib, orc, heads, kvh, d):
         lib.aotx_kv_close(ctypes.byref(m))
 
 
-# the three forms of a launch with prompt pieces, by its score columns (tokens x heads)
-_FORMS = {"16": (0, 6144), "32": (6144, 12288), "64": (12288, 1 << 30)}
-
-
 @pytest.mark.parametrize("form,tokens,heads,kvh,d", [("16", 150, 32, 8, 128), ("32", 200, 32, 8, 128), ("64", 390, 32, 8, 128),
                                                      ("16", 300, 8, 8, 64), ("32", 400, 16, 16, 128), ("64", 400, 32, 16, 64),
                                                      ("64", 1000, 16, 2, 64)])
@@ -297,8 +302,7 @@ def test_attend_prompt_nonfinite_values(torch, lib, orc, form, tokens, heads, kv
     """Values of Inf and NaN reach the rows that attend their positions and no others: not the
     rows of sequences in the same workgroup (single rows, short pieces), not a sequence's own
     earlier rows; nor do the halves that lie past a sequence's last position."""
-    lo, hi = _FORMS[form]
-    assert lo <= tokens * heads < hi
+    assert _is_form(form, tokens, heads)
     layers, layer = 2, 1
     rng = np.random.default_rng(tokens + heads)
     pieces = [(1, 60, 1), (2, 0, 9), (3, 37, 1), (4, 90, 1), (5, 20, 7), (6, 45, 1), (7, 0, 33)]
@@ -344,5 +348,61 @@ def test_attend_prompt_nonfinite_values(torch, lib, orc, form, tokens, heads, kv
                 want = orc.attend_one(q[i, hh].astype(np.float32), keys[s][:, hh // g, :].astype(np.float32), v, last)
                 assert np.abs(got[i, hh] - want)[~hit].max() < 4e-3, (i, s, last, hh)
         assert lib.aotx_model_faulted() == 0
+    finally:
+        lib.aotx_kv_close(ctypes.byref(m))
+
+
+@pytest.mark.parametrize("form,tokens,heads,kvh,d", [("16", 190, 32, 8, 128), ("16", 600, 8, 8, 64), ("32", 270, 32, 4, 128),
+                                                     ("32", 600, 16, 8, 64), ("64", 600, 32, 8, 128), ("64", 700, 32, 32, 64)])
+def test_attend_prompt_single_rows(torch, lib, orc, form, tokens, heads, kvh, d):
+    """Tokens that are the only one of their run are shared out over the workgroups: at the
+    batch's start and end, between pieces, at the ends of the 64-token words they are listed in,
+    and past the 512 tokens that are; one without pages (zeros, its neighbours right)."""
+    assert _is_form(form, tokens, heads)
+    layers, layer = 2, 1
+    rng = np.random.default_rng(tokens + heads)
+    alone = [t for t in (0, 1, 2, 3, 7, 62, 63, 64, 65, 127, 128, 130, 191, 192, 255, 256, 511, 512, 513, 575, tokens - 2, tokens - 1)
+             if t < tokens]
+    pieces, t, slot = [], 0, 0
+    context = iter([1, 16, 17, 31, 32, 33, 129, 300, 1100, 64] * 8)
+    while t < tokens:
+        if t in alone:
+            n, cached = 1, next(context) - 1
+        else:
+            after = [x for x in alone if x > t]
+            n, cached = (min(after) if after else tokens) - t, int(rng.integers(0, 50))
+        pieces.append((slot, cached, n))
+        slot, t = slot + 1, t + n
+    assert slot <= 64
+    gone = pieces[5][0]                                # its rows find no pages
+    m = _open_pool(lib, 400)
+    try:
+        for s, c, n in pieces:
+            if s != gone:
+                assert lib.aotx_kv_request(s, layout_pages(c + n, layers, kvh, d)) == 1
+        lib.aotx_kv_serve(ctypes.byref(m), None)
+        have = [(s, c + n) for s, c, n in pieces if s != gone]
+        keys, vals = _fill(torch, lib, [s for s, _ in have], [n for _, n in have], layers, layer, kvh, d, rng)
+        pos = np.concatenate([np.arange(c, c + n) for _, c, n in pieces]).astype(np.uint32)
+        ag = np.concatenate([np.full(n, s) for s, _, n in pieces]).astype(np.uint32)
+        assert len(pos) == tokens
+        q = rng.normal(0, 1, (tokens, heads, d)).astype(np.float16)
+        out = torch.full((tokens * heads * d,), 7.0, dtype=torch.float16, device="cuda")
+        lib.aotx_model_forget()
+        assert lib.aotx_attend_paged(p(dev(q, torch)), p(dev(pos, torch)), p(dev(ag, torch)),
+                                     tokens, heads, kvh, d, layer, layers, p(out), None) == 0
+        torch.cuda.synchronize()
+        assert lib.aotx_model_faulted() > 0
+        got = out.cpu().numpy().reshape(tokens, heads, d).astype(np.float32)
+        g = heads // kvh
+        for i in range(tokens):
+            s, last = int(ag[i]), int(pos[i])
+            if s == gone:
+                assert (got[i] == 0).all()
+                continue
+            for hh in range(i % 3, heads, 3 if i in alone else 7):
+                want = orc.attend_one(q[i, hh].astype(np.float32), keys[s][:, hh // g, :].astype(np.float32),
+                                      vals[s][:, hh // g, :].astype(np.float32), last)
+                assert np.abs(got[i, hh] - want).max() < 4e-3, (i, s, last, hh)
     finally:
         lib.aotx_kv_close(ctypes.byref(m))
