@@ -178,3 +178,25 @@ def test_pick_edges_vs_oracle(torch, lib, orc, vocab):
         for r in range(rows):
             want = orc.pick(logits[r], top_k, top_p, 0.0, temp, 77, int(agent[r]), 0)[0]
             assert got[r] == want, (r, top_k, temp, got[r], want)
+
+
+@pytest.mark.parametrize("vocab", [4096, 6001])
+def test_pick_flat_rows(torch, lib, orc, vocab):
+    """Rows of near-equal logits (the second pass of the cut, then more candidates than places or
+    fewer), among others, in more rows than a row has slices."""
+    rng = np.random.default_rng(vocab)
+    rows = 40
+    logits = rng.normal(0, 2.0, (rows, vocab)).astype(np.float32)
+    logits[::3] = rng.normal(0, 0.01, logits[::3].shape).astype(np.float32)
+    logits[1::6] = np.float32(1.5)
+    logits[1::12, vocab // 3] = np.float32(1.5000001)
+    agent = np.arange(rows, dtype=np.uint32)
+    tok = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    for top_k, top_p, temp in ((40, 0.9, 0.8), (0, 1.0, 1.0)):
+        lib.aotx_model_restream()
+        assert lib.aotx_pick(p(dev(logits, torch)), rows, vocab, p(dev(agent, torch)), None, top_k, top_p, temp,
+                             5, p(tok), None, None) == 0
+        torch.cuda.synchronize()
+        got = tok.cpu().numpy()
+        for r in range(rows):
+            assert got[r] == orc.pick(logits[r], top_k, top_p, 0.0, temp, 5, int(agent[r]), 0)[0], (r, top_k)
