@@ -144,6 +144,13 @@ static __device__ __forceinline__ const unsigned short *rg_scales(const aotx_rge
          + (unsigned long long)tile * a.qn * 64ull;
 }
 
+/* Lane 0's value, for all lanes. */
+static __device__ __forceinline__ unsigned long long rg_first(unsigned long long v)
+{
+    return (unsigned long long)(unsigned int)__builtin_amdgcn_readfirstlane((int)(unsigned int)(v >> 32)) << 32
+         | (unsigned int)__builtin_amdgcn_readfirstlane((int)(unsigned int)v);
+}
+
 /* Where a lane (r, g) reads the weights of a 16-row tile: block 4q + g of row r for quad q.
  * Q8R: 16 + 16 bytes of the tile's quant plane and a word of its scale plane, the wave's
  * loads contiguous. FILE: the 34-byte block where the model file has it; a wave's load covers
@@ -208,11 +215,16 @@ static __device__ __forceinline__ unsigned int rg_wend(const aotx_rgemv_args &a,
 /* Quad q's quants and scale bits (FILE: of the row's last block past its end). */
 template <bool FILE, bool STREAM>
 static __device__ __forceinline__ void rg_wload(const aotx_rgemv_args &a, const rg_wsrc<FILE> &w,
-                                                unsigned int q, unsigned int lane, rg_wreg &o)
+                                                unsigned int q, unsigned int lane, rg_wreg &o, bool unused = false)
 {
     if constexpr (FILE) {
         const unsigned int last = a.k / 32u - 1u, at = 4u * q + (lane >> 4);
         const unsigned char *b = w.q + (at < last ? at : last) * 34u;
+        /* a quad that is not computed: one address for all lanes, so that the load costs the
+         * address unit one line instead of 16 rows (256 square at 1 row, where 7 of a wave's 8 loads
+         * are such, 5.75 -> 4.9 us; 1024 x 4096 10.3 -> 8.4; in launches of many workgroups, of 4
+         * waves, the selection cost more: 14336 x 4096 19.4 -> 21.5) */
+        if (unused) b = (const unsigned char *)rg_first((unsigned long long)b);
         const unsigned int odd = (unsigned int)(unsigned long long)b & 2u;     /* the quants are aligned */
         typedef unsigned int u4d __attribute__((ext_vector_type(4), aligned(4)));
         o.w0 = *(const u4d *)(b + odd);
@@ -924,9 +936,10 @@ static __device__ __forceinline__ void rg_narrow(const aotx_rgemv_args &a, unsig
     do {                                                                                 \
         _Pragma("unroll") for (int qi = 0; qi < PD; ++qi) {                              \
             unsigned int qq = (QS) + (unsigned int)qi;                                   \
+            const bool unused = NW == 8 && qq >= wq1;                                    \
             if (qq > qlast) qq = qlast;                                                  \
             _Pragma("unroll") for (int j = 0; j < RT; ++j) {                             \
-                rg_wload<FILE, true>(a, wsrc[j], qq, lane, wr[BUF][qi][j]);             \
+                rg_wload<FILE, true>(a, wsrc[j], qq, lane, wr[BUF][qi][j], unused);     \
             }                                                                            \
         }                                                                                \
     } while (0)
