@@ -382,50 +382,52 @@ static __device__ bool char_starts(const unsigned char *b, unsigned int from, un
  * per text. */
 __global__ __launch_bounds__(1024) void aotx_text_clean_kernel(const unsigned char *bytes,
                                                                const unsigned long long *at,
-                                                               unsigned char *out, unsigned char *mark,
-                                                               unsigned int *clean_len, unsigned int *longs)
+                                                               unsigned int texts, unsigned char *out,
+                                                               unsigned char *mark, unsigned int *clean_len,
+                                                               unsigned int *longs)
 {
     __shared__ unsigned int part[16];
-    const unsigned int t = blockIdx.x;
-    const unsigned char *b = bytes + at[t];
-    const unsigned int end = (unsigned int)(at[t + 1u] - at[t]);
-    unsigned char *o = out + 3ull * at[t], *m = mark + 3ull * at[t];
-    if (t == 0u && threadIdx.x == 0u) *longs = 0u;
-    unsigned int done = 0u;
-    for (unsigned int tile = 0u; tile < end; tile += 4096u) {
-        const unsigned int i0 = tile + 4u * threadIdx.x;
-        unsigned int bad = 0u, n = 0u;
+    for (unsigned int t = blockIdx.x; t < texts; t += gridDim.x) {
+        const unsigned char *b = bytes + at[t];
+        const unsigned int end = (unsigned int)(at[t + 1u] - at[t]);
+        unsigned char *o = out + 3ull * at[t], *m = mark + 3ull * at[t];
+        if (t == 0u && threadIdx.x == 0u) *longs = 0u;
+        unsigned int done = 0u;
+        for (unsigned int tile = 0u; tile < end; tile += 4096u) {
+            const unsigned int i0 = tile + 4u * threadIdx.x;
+            unsigned int bad = 0u, n = 0u;
 #pragma unroll
-        for (unsigned int j = 0u; j < 4u; ++j) {
-            const unsigned int i = i0 + j;
-            if (i >= end) continue;
-            bool replace = false;
-            if (b[i] >= 0x80u && char_starts(b, 0u, end, i)) {
-                unsigned int p;
-                replace = utf8_at(b, end, i, &p) == 1u;
+            for (unsigned int j = 0u; j < 4u; ++j) {
+                const unsigned int i = i0 + j;
+                if (i >= end) continue;
+                bool replace = false;
+                if (b[i] >= 0x80u && char_starts(b, 0u, end, i)) {
+                    unsigned int p;
+                    replace = utf8_at(b, end, i, &p) == 1u;
+                }
+                bad |= replace ? 1u << j : 0u;
+                n += replace ? 3u : 1u;
             }
-            bad |= replace ? 1u << j : 0u;
-            n += replace ? 3u : 1u;
-        }
-        unsigned int total;
-        unsigned int w = done + block_before(n, part, &total);
+            unsigned int total;
+            unsigned int w = done + block_before(n, part, &total);
 #pragma unroll
-        for (unsigned int j = 0u; j < 4u; ++j) {
-            const unsigned int i = i0 + j;
-            if (i >= end) continue;
-            if ((bad >> j) & 1u) {
-                o[w] = 0xEFu; o[w + 1u] = 0xBFu; o[w + 2u] = 0xBDu;
-                m[w] = 0u; m[w + 1u] = 0u; m[w + 2u] = 0u;
-                w += 3u;
-            } else {
-                o[w] = b[i];
-                m[w] = 0u;
-                w += 1u;
+            for (unsigned int j = 0u; j < 4u; ++j) {
+                const unsigned int i = i0 + j;
+                if (i >= end) continue;
+                if ((bad >> j) & 1u) {
+                    o[w] = 0xEFu; o[w + 1u] = 0xBFu; o[w + 2u] = 0xBDu;
+                    m[w] = 0u; m[w + 1u] = 0u; m[w + 2u] = 0u;
+                    w += 3u;
+                } else {
+                    o[w] = b[i];
+                    m[w] = 0u;
+                    w += 1u;
+                }
             }
+            done += total;
         }
-        done += total;
+        if (threadIdx.x == 0u) clean_len[t] = done;
     }
-    if (threadIdx.x == 0u) clean_len[t] = done;
 }
 
 /* The longest special token whose bytes start at `at` (cuda/text/pretok.cu:339-372): its
@@ -456,46 +458,48 @@ static __device__ unsigned int special_at(const aotx_text_vocab &v, const unsign
  * at send[3 at[t] + i]; scount[t] counts them. */
 __global__ __launch_bounds__(64) void aotx_text_special_kernel(aotx_text_vocab v, const unsigned char *bytes,
                                                                const unsigned long long *at,
-                                                               const unsigned int *clean_len, unsigned char *mark,
-                                                               unsigned int *sat, unsigned int *send,
-                                                               unsigned int *scount)
+                                                               const unsigned int *clean_len, unsigned int texts,
+                                                               unsigned char *mark, unsigned int *sat,
+                                                               unsigned int *send, unsigned int *scount)
 {
-    const unsigned int t = blockIdx.x, lane = threadIdx.x;
-    const unsigned long long base = 3ull * at[t];
-    const unsigned char *b = bytes + base;
-    const unsigned int end = clean_len[t];
-    unsigned int pos = 0u, n = 0u;
-    for (unsigned int tile = 0u; tile < end; tile += 512u) {
-        unsigned int c[8];
+    const unsigned int lane = threadIdx.x;
+    for (unsigned int t = blockIdx.x; t < texts; t += gridDim.x) {
+        const unsigned long long base = 3ull * at[t];
+        const unsigned char *b = bytes + base;
+        const unsigned int end = clean_len[t];
+        unsigned int pos = 0u, n = 0u;
+        for (unsigned int tile = 0u; tile < end; tile += 512u) {
+            unsigned int c[8];
 #pragma unroll
-        for (unsigned int j = 0u; j < 8u; ++j) {
-            const unsigned int i = tile + 64u * j + lane;
-            c[j] = b[i < end ? i : tile];
-        }
+            for (unsigned int j = 0u; j < 8u; ++j) {
+                const unsigned int i = tile + 64u * j + lane;
+                c[j] = b[i < end ? i : tile];
+            }
 #pragma unroll
-        for (unsigned int j = 0u; j < 8u; ++j) {
-            const unsigned int i = tile + 64u * j + lane;
-            const bool maybe = i < end && ((v.first[c[j] >> 6] >> (c[j] & 63u)) & 1ull) != 0ull;
-            if (!__any(maybe)) continue;
-            unsigned int id = 0u;
-            const unsigned int span = maybe ? special_at(v, b, i, end, &id) : 0u;
-            unsigned long long found = __ballot(span != 0u);
-            while (found != 0ull) {
-                const unsigned int l = (unsigned int)__builtin_ctzll(found);
-                found &= found - 1ull;
-                const unsigned int p = tile + 64u * j + l, k = (unsigned int)__shfl((int)span, (int)l, 64);
-                if (p < pos) continue;                   /* inside the one before */
-                if (lane == 0u) {
-                    mark[base + p] = TX_MARK_SPECIAL;
-                    sat[base + n] = p;
-                    send[base + n] = p + k;
+            for (unsigned int j = 0u; j < 8u; ++j) {
+                const unsigned int i = tile + 64u * j + lane;
+                const bool maybe = i < end && ((v.first[c[j] >> 6] >> (c[j] & 63u)) & 1ull) != 0ull;
+                if (!__any(maybe)) continue;
+                unsigned int id = 0u;
+                const unsigned int span = maybe ? special_at(v, b, i, end, &id) : 0u;
+                unsigned long long found = __ballot(span != 0u);
+                while (found != 0ull) {
+                    const unsigned int l = (unsigned int)__builtin_ctzll(found);
+                    found &= found - 1ull;
+                    const unsigned int p = tile + 64u * j + l, k = (unsigned int)__shfl((int)span, (int)l, 64);
+                    if (p < pos) continue;                   /* inside the one before */
+                    if (lane == 0u) {
+                        mark[base + p] = TX_MARK_SPECIAL;
+                        sat[base + n] = p;
+                        send[base + n] = p + k;
+                    }
+                    n += 1u;
+                    pos = p + k;
                 }
-                n += 1u;
-                pos = p + k;
             }
         }
+        if (lane == 0u) scount[t] = n;
     }
-    if (lane == 0u) scount[t] = n;
 }
 
 /* Whether every way of cutting the text up to `at` has a cut at `at`, a place where a
@@ -526,46 +530,48 @@ static __device__ bool is_sync(unsigned int pattern, const unsigned char *b, uns
  * word: 64 texts of 4000 bytes 6812 -> 45 us. */
 __global__ __launch_bounds__(256) void aotx_text_pretok_kernel(aotx_text_vocab v, const unsigned char *bytes,
                                                                const unsigned long long *at,
-                                                               const unsigned int *clean_len, unsigned int chunks,
-                                                               const unsigned int *sat, const unsigned int *send,
-                                                               const unsigned int *scount, unsigned char *mark)
+                                                               const unsigned int *clean_len, unsigned int texts,
+                                                               unsigned int chunks, const unsigned int *sat,
+                                                               const unsigned int *send, const unsigned int *scount,
+                                                               unsigned char *mark)
 {
-    const unsigned int t = blockIdx.x / chunks;
-    const unsigned long long base = 3ull * at[t];
-    const unsigned char *b = bytes + base;
-    const unsigned int text_end = clean_len[t];
-    for (unsigned int tile = (blockIdx.x % chunks) * 256u; tile < text_end; tile += chunks * 256u) {
-        unsigned int pos = tile + threadIdx.x;
-        if (pos >= text_end) return;
-        unsigned int from = 0u, end = text_end;
-        if (v.specials != 0u) {
-            /* the run between special tokens that holds pos: after the last one at or before it */
-            unsigned int lo = 0u, hi = scount[t];
-            while (lo < hi) {
-                const unsigned int mid = (lo + hi) >> 1;
-                if (sat[base + mid] <= pos) lo = mid + 1u; else hi = mid;
-            }
-            if (lo > 0u) from = send[base + lo - 1u];
-            if (lo < scount[t]) end = sat[base + lo];
-            if (pos < from) continue;                    /* inside a special token */
-        }
-        if (!char_starts(b, from, end, pos) || !is_sync(v.pattern, b, from, end, pos)) continue;
-        do {
-            unsigned int m = match(v.pattern, b, pos, end);
-            if (m == 0u) m = 1u;
-            if (m > AOTX_TEXT_CHUNK_BYTES) {          /* cut at a character boundary */
-                unsigned int cut = 0u;
-                while (cut < end - pos) {
-                    unsigned int p;
-                    const unsigned int k = utf8_at(b, end, pos + cut, &p);
-                    if (cut + k > AOTX_TEXT_CHUNK_BYTES) break;
-                    cut += k;
+    for (unsigned int t = blockIdx.x / chunks; t < texts; t += gridDim.x / chunks) {
+        const unsigned long long base = 3ull * at[t];
+        const unsigned char *b = bytes + base;
+        const unsigned int text_end = clean_len[t];
+        for (unsigned int tile = (blockIdx.x % chunks) * 256u; tile < text_end; tile += chunks * 256u) {
+            unsigned int pos = tile + threadIdx.x;
+            if (pos >= text_end) break;
+            unsigned int from = 0u, end = text_end;
+            if (v.specials != 0u) {
+                /* the run between special tokens that holds pos: after the last one at or before it */
+                unsigned int lo = 0u, hi = scount[t];
+                while (lo < hi) {
+                    const unsigned int mid = (lo + hi) >> 1;
+                    if (sat[base + mid] <= pos) lo = mid + 1u; else hi = mid;
                 }
-                m = cut;
+                if (lo > 0u) from = send[base + lo - 1u];
+                if (lo < scount[t]) end = sat[base + lo];
+                if (pos < from) continue;                    /* inside a special token */
             }
-            mark[base + pos] = TX_MARK_START;
-            pos += m;
-        } while (pos < end && !is_sync(v.pattern, b, from, end, pos));
+            if (!char_starts(b, from, end, pos) || !is_sync(v.pattern, b, from, end, pos)) continue;
+            do {
+                unsigned int m = match(v.pattern, b, pos, end);
+                if (m == 0u) m = 1u;
+                if (m > AOTX_TEXT_CHUNK_BYTES) {          /* cut at a character boundary */
+                    unsigned int cut = 0u;
+                    while (cut < end - pos) {
+                        unsigned int p;
+                        const unsigned int k = utf8_at(b, end, pos + cut, &p);
+                        if (cut + k > AOTX_TEXT_CHUNK_BYTES) break;
+                        cut += k;
+                    }
+                    m = cut;
+                }
+                mark[base + pos] = TX_MARK_START;
+                pos += m;
+            } while (pos < end && !is_sync(v.pattern, b, from, end, pos));
+        }
     }
 }
 
@@ -586,8 +592,9 @@ __global__ __launch_bounds__(256) void aotx_text_pretok_kernel(aotx_text_vocab v
 __global__ __launch_bounds__(64 * TX_WAVES) void aotx_text_merge_kernel(aotx_text_vocab v, const unsigned char *bytes,
                                                                         const unsigned long long *at,
                                                                         const unsigned int *clean_len,
-                                                                        const unsigned char *mark, unsigned int chunks,
-                                                                        unsigned int *out, unsigned short *count,
+                                                                        const unsigned char *mark, unsigned int texts,
+                                                                        unsigned int chunks, unsigned int *out,
+                                                                        unsigned short *count,
                                                                         unsigned int *long_list, unsigned int *longs)
 {
     __shared__ unsigned int tokl[TX_WAVES][64 + TX_SHORT], rankl[TX_WAVES][64 + TX_SHORT], resl[TX_WAVES][64 + TX_SHORT];
@@ -595,106 +602,107 @@ __global__ __launch_bounds__(64 * TX_WAVES) void aotx_text_merge_kernel(aotx_tex
     const unsigned int lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     unsigned int *tok = tokl[wave], *rank = rankl[wave], *res = resl[wave];
     unsigned char *nxt = nxtl[wave], *prv = prvl[wave];
-    const unsigned int t = blockIdx.x / chunks;
-    const unsigned long long base = 3ull * at[t];
-    const unsigned char *b = bytes + base;
-    const unsigned int end = clean_len[t];
-    for (unsigned int w = ((blockIdx.x % chunks) * TX_WAVES + wave) * 64u; w < end; w += chunks * TX_WAVES * 64u) {
-        const unsigned int p = w + lane;
-        const unsigned int kind = p < end ? mark[base + p] : 0u;
-        const unsigned long long starts = __ballot(kind != 0u);
-        if (p < end) count[base + p] = 0u;
-        if (starts == 0ull) continue;                    /* inside a longer one */
-        /* the end of the last pre-token that starts here */
-        unsigned int after = w + 64u;
-        for (; after < end; after += 64u) {
-            const unsigned int q = after + lane;
-            const unsigned long long more = __ballot(q < end && mark[base + (q < end ? q : after)] != 0u);
-            if (more != 0ull) {
-                after += (unsigned int)__builtin_ctzll(more);
-                break;
+    for (unsigned int t = blockIdx.x / chunks; t < texts; t += gridDim.x / chunks) {
+        const unsigned long long base = 3ull * at[t];
+        const unsigned char *b = bytes + base;
+        const unsigned int end = clean_len[t];
+        for (unsigned int w = ((blockIdx.x % chunks) * TX_WAVES + wave) * 64u; w < end; w += chunks * TX_WAVES * 64u) {
+            const unsigned int p = w + lane;
+            const unsigned int kind = p < end ? mark[base + p] : 0u;
+            const unsigned long long starts = __ballot(kind != 0u);
+            if (p < end) count[base + p] = 0u;
+            if (starts == 0ull) continue;                    /* inside a longer one */
+            /* the end of the last pre-token that starts here */
+            unsigned int after = w + 64u;
+            for (; after < end; after += 64u) {
+                const unsigned int q = after + lane;
+                const unsigned long long more = __ballot(q < end && mark[base + (q < end ? q : after)] != 0u);
+                if (more != 0ull) {
+                    after += (unsigned int)__builtin_ctzll(more);
+                    break;
+                }
             }
-        }
-        if (after > end) after = end;
-        const unsigned long long later = lane == 63u ? 0ull : starts >> (lane + 1u);
-        const unsigned int n = later != 0ull ? 1u + (unsigned int)__builtin_ctzll(later) : after - p;
-        unsigned int *dst = out + base + p;
-        bool open = kind != 0u;
-        if (kind == TX_MARK_SPECIAL) {
-            unsigned int id = AOTX_TEXT_NONE;
-            special_at(v, b, p, end, &id);
-            dst[0] = id;
-            count[base + p] = 1u;
-            open = false;
-        } else if (open && v.whole) {
-            const unsigned int whole = find_bytes(v, b + p, n);
-            if (whole != AOTX_TEXT_NONE) {
-                dst[0] = whole;
+            if (after > end) after = end;
+            const unsigned long long later = lane == 63u ? 0ull : starts >> (lane + 1u);
+            const unsigned int n = later != 0ull ? 1u + (unsigned int)__builtin_ctzll(later) : after - p;
+            unsigned int *dst = out + base + p;
+            bool open = kind != 0u;
+            if (kind == TX_MARK_SPECIAL) {
+                unsigned int id = AOTX_TEXT_NONE;
+                special_at(v, b, p, end, &id);
+                dst[0] = id;
                 count[base + p] = 1u;
                 open = false;
+            } else if (open && v.whole) {
+                const unsigned int whole = find_bytes(v, b + p, n);
+                if (whole != AOTX_TEXT_NONE) {
+                    dst[0] = whole;
+                    count[base + p] = 1u;
+                    open = false;
+                }
             }
-        }
-        if (open && n > TX_SHORT) {
-            unsigned int *item = long_list + 3ull * atomicAdd(longs, 1u);
-            item[0] = t;
-            item[1] = p;
-            item[2] = n;
-            open = false;
-        }
-        const unsigned long long mine = __ballot(open);
-        if (mine == 0ull) continue;
-        /* every byte's token and its pair with the next, the last pre-token's bytes past the
-         * window in a second round */
+            if (open && n > TX_SHORT) {
+                unsigned int *item = long_list + 3ull * atomicAdd(longs, 1u);
+                item[0] = t;
+                item[1] = p;
+                item[2] = n;
+                open = false;
+            }
+            const unsigned long long mine = __ballot(open);
+            if (mine == 0ull) continue;
+            /* every byte's token and its pair with the next, the last pre-token's bytes past the
+             * window in a second round */
 #pragma unroll
-        for (unsigned int round = 0u; round < 2u; ++round) {
-            const unsigned int i = round * 64u + lane;
-            const unsigned long long upto = round != 0u ? starts : starts & (~0ull >> (63u - lane));
-            const unsigned int own = upto != 0ull ? 63u - (unsigned int)__builtin_clzll(upto) : 64u;
-            const unsigned int size = (unsigned int)__shfl((int)n, (int)(own & 63u), 64);
-            if (i < 64u + TX_SHORT && own < 64u && ((mine >> own) & 1ull) != 0ull && i < own + size) {
-                const unsigned int x = v.byte_token[b[w + i]];
-                unsigned int r = 0u, k = AOTX_TEXT_NONE;
-                if (i + 1u < own + size) k = find_pair(v, x, v.byte_token[b[w + i + 1u]], &r);
-                tok[i] = x;
-                rank[i] = k;
-                res[i] = r;
-                nxt[i] = (unsigned char)(i + 1u);
-                prv[i] = i == own ? 0xFFu : (unsigned char)(i - 1u);
-            }
-        }
-        /* the wave's writes before its lanes' reads of one another's places */
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (open) {
-            const unsigned int last = lane + n;
-            for (;;) {
-                unsigned int best = AOTX_TEXT_NONE, i = lane;
-                for (unsigned int q = lane; q < last; ++q) {
-                    const unsigned int k = rank[q];
-                    if (k < best) { best = k; i = q; }
-                }
-                if (best == AOTX_TEXT_NONE) break;
-                const unsigned int j = nxt[i], k = nxt[j], f = prv[i], x = res[i];
-                unsigned int ranks[2], made[2];
-                find_pairs(v, x, k < last ? tok[k] : AOTX_TEXT_NONE, f != 0xFFu ? tok[f] : AOTX_TEXT_NONE, x, ranks,
-                           made);
-                tok[i] = x;
-                nxt[i] = (unsigned char)k;
-                if (k < last) prv[k] = (unsigned char)i;
-                rank[j] = AOTX_TEXT_NONE;
-                rank[i] = ranks[0];
-                res[i] = made[0];
-                if (f != 0xFFu) {
-                    rank[f] = ranks[1];
-                    res[f] = made[1];
+            for (unsigned int round = 0u; round < 2u; ++round) {
+                const unsigned int i = round * 64u + lane;
+                const unsigned long long upto = round != 0u ? starts : starts & (~0ull >> (63u - lane));
+                const unsigned int own = upto != 0ull ? 63u - (unsigned int)__builtin_clzll(upto) : 64u;
+                const unsigned int size = (unsigned int)__shfl((int)n, (int)(own & 63u), 64);
+                if (i < 64u + TX_SHORT && own < 64u && ((mine >> own) & 1ull) != 0ull && i < own + size) {
+                    const unsigned int x = v.byte_token[b[w + i]];
+                    unsigned int r = 0u, k = AOTX_TEXT_NONE;
+                    if (i + 1u < own + size) k = find_pair(v, x, v.byte_token[b[w + i + 1u]], &r);
+                    tok[i] = x;
+                    rank[i] = k;
+                    res[i] = r;
+                    nxt[i] = (unsigned char)(i + 1u);
+                    prv[i] = i == own ? 0xFFu : (unsigned char)(i - 1u);
                 }
             }
-            unsigned int c = 0u;
-            for (unsigned int i = lane; i < last; i = nxt[i]) dst[c++] = tok[i];
-            count[base + p] = (unsigned short)c;
+            /* the wave's writes before its lanes' reads of one another's places */
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (open) {
+                const unsigned int last = lane + n;
+                for (;;) {
+                    unsigned int best = AOTX_TEXT_NONE, i = lane;
+                    for (unsigned int q = lane; q < last; ++q) {
+                        const unsigned int k = rank[q];
+                        if (k < best) { best = k; i = q; }
+                    }
+                    if (best == AOTX_TEXT_NONE) break;
+                    const unsigned int j = nxt[i], k = nxt[j], f = prv[i], x = res[i];
+                    unsigned int ranks[2], made[2];
+                    find_pairs(v, x, k < last ? tok[k] : AOTX_TEXT_NONE, f != 0xFFu ? tok[f] : AOTX_TEXT_NONE, x, ranks,
+                               made);
+                    tok[i] = x;
+                    nxt[i] = (unsigned char)k;
+                    if (k < last) prv[k] = (unsigned char)i;
+                    rank[j] = AOTX_TEXT_NONE;
+                    rank[i] = ranks[0];
+                    res[i] = made[0];
+                    if (f != 0xFFu) {
+                        rank[f] = ranks[1];
+                        res[f] = made[1];
+                    }
+                }
+                unsigned int c = 0u;
+                for (unsigned int i = lane; i < last; i = nxt[i]) dst[c++] = tok[i];
+                count[base + p] = (unsigned short)c;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -769,35 +777,36 @@ __global__ __launch_bounds__(64) void aotx_text_long_kernel(aotx_text_vocab v, c
  * ids + 3 at[t] (64 texts of 4000 bytes 277 -> 6.4 us against a wave that went from pre-token
  * to pre-token). */
 __global__ __launch_bounds__(1024) void aotx_text_gather_kernel(const unsigned long long *at,
-                                                                const unsigned int *clean_len,
+                                                                const unsigned int *clean_len, unsigned int texts,
                                                                 const unsigned int *tokens,
                                                                 const unsigned short *place_count,
                                                                 unsigned int *ids, unsigned int *count)
 {
     __shared__ unsigned int part[16];
-    const unsigned int t = blockIdx.x;
-    const unsigned long long base = 3ull * at[t];
-    const unsigned int end = clean_len[t];
-    unsigned int done = 0u;
-    for (unsigned int tile = 0u; tile < end; tile += 4096u) {
-        unsigned int c[4], mine = 0u;
+    for (unsigned int t = blockIdx.x; t < texts; t += gridDim.x) {
+        const unsigned long long base = 3ull * at[t];
+        const unsigned int end = clean_len[t];
+        unsigned int done = 0u;
+        for (unsigned int tile = 0u; tile < end; tile += 4096u) {
+            unsigned int c[4], mine = 0u;
 #pragma unroll
-        for (unsigned int j = 0u; j < 4u; ++j) {
-            const unsigned int i = tile + 4u * threadIdx.x + j;
-            c[j] = i < end ? place_count[base + i] : 0u;
-            mine += c[j];
-        }
-        unsigned int total;
-        unsigned int w = done + block_before(mine, part, &total);
+            for (unsigned int j = 0u; j < 4u; ++j) {
+                const unsigned int i = tile + 4u * threadIdx.x + j;
+                c[j] = i < end ? place_count[base + i] : 0u;
+                mine += c[j];
+            }
+            unsigned int total;
+            unsigned int w = done + block_before(mine, part, &total);
 #pragma unroll
-        for (unsigned int j = 0u; j < 4u; ++j) {
-            const unsigned long long src = base + tile + 4u * threadIdx.x + j;
-            for (unsigned int i = 0u; i < c[j]; ++i) ids[base + w + i] = tokens[src + i];
-            w += c[j];
+            for (unsigned int j = 0u; j < 4u; ++j) {
+                const unsigned long long src = base + tile + 4u * threadIdx.x + j;
+                for (unsigned int i = 0u; i < c[j]; ++i) ids[base + w + i] = tokens[src + i];
+                w += c[j];
+            }
+            done += total;
         }
-        done += total;
+        if (threadIdx.x == 0u) count[t] = done;
     }
-    if (threadIdx.x == 0u) count[t] = done;
 }
 
 /* ---- detokenize ------------------------------------------------------------------------ */
@@ -1080,24 +1089,28 @@ extern "C" int aotx_text_encode(const unsigned char *bytes, const unsigned long 
     const unsigned long long tiles = (total / texts + 255ull) / 256ull;
     const unsigned long long most = 65536ull / texts > 0ull ? 65536ull / texts : 1ull;
     const unsigned int chunks = (unsigned int)(tiles < 1ull ? 1ull : (tiles < most ? tiles : most));
-    hipLaunchKernelGGL(aotx_text_clean_kernel, dim3(texts), dim3(1024), 0, s, bytes, at, clean, mark, clean_len,
+    /* workgroups for so many texts, each going on with later ones: a launch holds 2^32 threads, and
+     * a text takes up to 1024 */
+    const unsigned int most_texts = 1u << 20, here = texts < most_texts ? texts : most_texts;
+    hipLaunchKernelGGL(aotx_text_clean_kernel, dim3(here), dim3(1024), 0, s, bytes, at, texts, clean, mark, clean_len,
                        longs);
     AOTX_LAUNCH_CHECK();
     if (g_vocab.specials != 0u) {
-        hipLaunchKernelGGL(aotx_text_special_kernel, dim3(texts), dim3(64), 0, s, g_vocab, clean, at, clean_len, mark,
-                           sat, send, scount);
+        hipLaunchKernelGGL(aotx_text_special_kernel, dim3(here), dim3(64), 0, s, g_vocab, clean, at, clean_len, texts,
+                           mark, sat, send, scount);
         AOTX_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(aotx_text_pretok_kernel, dim3(texts * chunks), dim3(256), 0, s, g_vocab, clean, at, clean_len,
-                       chunks, sat, send, scount, mark);
+    hipLaunchKernelGGL(aotx_text_pretok_kernel, dim3(here * chunks), dim3(256), 0, s, g_vocab, clean, at, clean_len,
+                       texts, chunks, sat, send, scount, mark);
     AOTX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(aotx_text_merge_kernel, dim3(texts * chunks), dim3(64 * TX_WAVES), 0, s, g_vocab, clean, at,
-                       clean_len, mark, chunks, tok, pcount, long_list, longs);
+    hipLaunchKernelGGL(aotx_text_merge_kernel, dim3(here * chunks), dim3(64 * TX_WAVES), 0, s, g_vocab, clean, at,
+                       clean_len, mark, texts, chunks, tok, pcount, long_list, longs);
     AOTX_LAUNCH_CHECK();
     hipLaunchKernelGGL(aotx_text_long_kernel, dim3(512), dim3(64), 0, s, g_vocab, clean, at, long_list, longs, tok,
                        pcount);
     AOTX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(aotx_text_gather_kernel, dim3(texts), dim3(1024), 0, s, at, clean_len, tok, pcount, ids, count);
+    hipLaunchKernelGGL(aotx_text_gather_kernel, dim3(here), dim3(1024), 0, s, at, clean_len, texts, tok, pcount, ids,
+                       count);
     AOTX_LAUNCH_CHECK();
     AOTX_CHECK(hipFreeAsync(buf, s));
     AOTX_CHECK(hipStreamSynchronize(s));

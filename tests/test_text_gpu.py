@@ -272,3 +272,23 @@ def test_encode_edges_vs_oracle(torch, lib, bpe, family, special):
             assert g == v.encode(s), (family, repr(s[:80]), len(s))
     finally:
         built.close()
+
+
+def test_encode_many_texts(torch, lib, bpe):
+    """More texts than a launch has room for at a workgroup of 1024 threads each (2^22)."""
+    tokens, merges, _ = bpe
+    built = Built(lib, tokens, merges, [1] * len(tokens), "gpt-2")
+    try:
+        texts = (1 << 22) + 77
+        letters = np.frombuffer(b"abcdefghijklmnop", dtype=np.uint8)
+        data = letters[np.arange(texts) % 16]
+        want = np.array([_encode(torch, lib, [bytes([c])])[0] for c in letters]).reshape(16)
+        d = torch.from_numpy(data.copy()).cuda()
+        at = torch.arange(texts + 1, dtype=torch.int64, device="cuda")
+        ids = torch.zeros(3 * texts, dtype=torch.int32, device="cuda")
+        cnt = torch.zeros(texts, dtype=torch.int32, device="cuda")
+        assert lib.aotx_text_encode(d.data_ptr(), at.data_ptr(), texts, ids.data_ptr(), cnt.data_ptr(), None) == 0
+        assert int(cnt.min()) == 1 and int(cnt.max()) == 1
+        assert np.array_equal(ids[::3].cpu().numpy(), want[np.arange(texts) % 16])
+    finally:
+        built.close()
