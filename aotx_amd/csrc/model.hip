@@ -37,7 +37,6 @@
 unsigned long long aotx_mem_weights_bytes(void);
 
 #define AOTX_BUCKETS 10u   /* 1, 2, 4, ..., 512 */
-#define AOTX_WIDE_PASSES 4u        /* 32-row passes of a wide product in one launch */
 #define AOTX_GEMV_COUNTS 65536u   /* split arrival counters: experts x product groups */
 #define AOTX_PIECES 48u            /* device buffers of one role */
 
@@ -245,8 +244,8 @@ extern "C" int aotx_model_set_desc(unsigned int role, const aotx_model_desc *des
 
 static void aotx_roperands(aotx_rgemv_args *p, const aotx_rgemv_args &tmpl);
 
-/* One product of a step over repacked weights, in passes of at most 32 batch rows; a
- * batch of at most 16 rows may stage x from the residual stream (norm fused). */
+/* One product of a step over repacked weights; a batch of at most 16 rows may stage x from the
+ * residual stream (norm fused). */
 static void aotx_rproduct(aotx_hold *h, const void *const *w, const unsigned int *rows,
                           unsigned int nseg, unsigned int k, int epi, unsigned int cap,
                           const unsigned int *m_dev, const aotx_rgemv_args &tmpl)
@@ -273,15 +272,6 @@ static void aotx_rproduct(aotx_hold *h, const void *const *w, const unsigned int
         aotx_roperands(&a, tmpl);
         a.m_dev = m_dev;
         a.m0 = m0;
-        /* whole 32-row passes of a wide product over direct rows run as one launch (grid.y
-         * is the pass): one launch's ramp and tail instead of one per pass */
-        if (!gemm && a.wide && mt == 32u && cap - m0 >= 64u && tmpl.expert_stride == 0ull
-            && tmpl.list == nullptr && tmpl.xrow == nullptr) {
-            a.passes = (cap - m0) / 32u;
-            if (a.passes > AOTX_WIDE_PASSES) a.passes = AOTX_WIDE_PASSES;
-            mt = 32u * a.passes;
-            a.m = mt;
-        }
         if (a.splits > 1u) {
             size_t need = aotx_rgemv_partial_bytes(a);
             if (need > h->gemv_partial_bytes) {
@@ -802,9 +792,8 @@ extern "C" int aotx_model_open(unsigned int role, unsigned int max_tokens)
             if (aotx_rgemv_plan_frag(&a, w1, rv, 1u, d->hidden, AOTX_EPI_F32, mt) == 0)
                 gp = gp > aotx_rgemv_partial_bytes(a) ? gp : aotx_rgemv_partial_bytes(a);
         }
-        gp *= AOTX_WIDE_PASSES;                              /* passes in one launch */
         /* the passes of 64 rows and more of the dense products */
-        for (unsigned int mt = 64u; mt <= AOTX_RGEMM_ROWS && mt <= cap; mt += 64u) {
+        for (unsigned int mt = 64u; mt <= AOTX_RGEMM_ROWS && mt <= h->max_rows; mt += 64u) {
             aotx_rgemv_args a;
             unsigned int r3[3] = {(unsigned int)wide, (unsigned int)narrow, (unsigned int)narrow};
             unsigned int r1[1] = {d->hidden};

@@ -237,8 +237,7 @@ def test_8b_width_wide_batch_vs_oracle(torch, orc, rows):
     take the fragment-layout product, with x written in that layout by the norm, the down
     epilogue and the attention; gate/up and down take the wide kernel. A prompt pass of 4
     tokens per slot, then a decode step of one token per slot, logits vs the oracle.
-    40 and 48 rows fall in the 64-token bucket: two 32-row passes in one launch, the second
-    one partly filled (8 and 16 rows)."""
+    40 and 48 rows fall in the 64-token bucket: one pass of 64 rows, partly filled."""
     shape = Shape(layers=1, hidden=4096, ffn=14336, heads=32, kv_heads=8, head_dim=128,
                   vocab=1024)
     region_dev, region, lay = _device_model(torch, shape, 5)
@@ -295,7 +294,7 @@ def test_wide_qkv_fragment_four_tiles_vs_oracle(torch, orc, rows):
 def test_8b_width_experts_wide_batch_vs_oracle(torch, orc, rows):
     """Routed experts at d_model 4096 with 24 and 40 rows: the expert down product (k = 4096)
     takes the wide kernel through the expert row lists; at 40 rows the dense products run
-    two 32-row passes in one launch, the second with 8 rows. At 40 rows the first step's 80
+    one pass of 64 rows. At 40 rows the first step's 80
     tokens give some expert more than 32 rows, so the routed products' second 32-row pass
     computes rows too."""
     shape = Shape(layers=1, hidden=4096, ffn=4096, heads=32, kv_heads=8, head_dim=128,
