@@ -178,7 +178,8 @@ def test_product_ends_and_alignment(torch, lib, orc, n, k, shift, m):
     number of blocks a row, a tensor at any even address), and of both layouts where k ends
     inside 128 and rows inside 16, by every kernel (1-4, 5-32, 33 rows and more). What lies
     after x and the weights is never used: it holds NaN and scales of infinity here. The fp32
-    sums agree with the fp64 product to 1e-5 of the result's rms."""
+    sums agree with the fp64 product to 1e-5 of the result's rms (of 1 where that is smaller) times
+    the square root of the 32-value blocks added up."""
     w = make(torch, lib, n, k, 3 + n + k)
     buf = torch.full((shift + w.numel() + 512,), 0x7C, dtype=torch.uint8, device="cuda")
     buf[shift:shift + w.numel()] = w
@@ -222,6 +223,14 @@ def test_product_rows_past_32_bit_offsets(torch, lib, orc):
     torch.cuda.empty_cache()
 
 
+def _product64(w, n, k, x):
+    """The fp64 product over the fp16 weights the kernels multiply with, on many rows at once."""
+    rows = w.cpu().numpy().reshape(n, k // 32, 34)
+    scale = rows[:, :, :2].copy().view(np.float16).astype(np.float32)
+    wide = (scale * rows[:, :, 2:].view(np.int8)).astype(np.float16).astype(np.float64).reshape(n, k)
+    return x.astype(np.float64) @ wide.T
+
+
 @pytest.mark.parametrize("n,k", [(544, 4128), (2064, 512), (100, 96)])
 @pytest.mark.parametrize("m", [512, 513, 580, 1024, 1100])
 def test_product_of_more_rows_than_a_pass(torch, lib, orc, n, k, m):
@@ -231,10 +240,7 @@ def test_product_of_more_rows_than_a_pass(torch, lib, orc, n, k, m):
     wr = repack(torch, lib, w, n, k)
     rng = np.random.default_rng(n + m)
     x = rng.normal(0, 1, (m, k)).astype(np.float16)
-    rows = w.cpu().numpy().reshape(n, k // 32, 34)
-    scale = rows[:, :, :2].copy().view(np.float16).astype(np.float32)
-    wide = (scale * rows[:, :, 2:].view(np.int8)).astype(np.float16).astype(np.float64).reshape(n, k)
-    want = x.astype(np.float64) @ wide.T                 # the oracle's product, on many rows at once
+    want = _product64(w, n, k, x)
     assert np.abs(want[-2:] - orc.q8_gemv_f64(w.cpu().numpy(), n, k, x[-2:].view(np.uint16))).max() < 1e-9
     rms = np.sqrt((want ** 2).mean())
     for fn, at in ((lib.aotx_q8_gemv, w), (lib.aotx_q8r_gemv, wr)):
@@ -264,3 +270,21 @@ def test_file_product_of_infinities(torch, lib, n, k, m):
         with np.errstate(invalid="ignore"):
             want = quant[:, at].T * x[np.arange(m), at].astype(np.float32)[:, None]
         assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
+
+
+@pytest.mark.parametrize("n,k,m", [(6144, 4128, 64), (6144, 4096, 40), (20000, 416, 300), (2064, 14336, 512)])
+def test_product_large_forms(torch, lib, orc, n, k, m):
+    """Both layouts through the 64-row form with k in two splits (96 groups of 4 tiles), the GEMM of
+    more workgroups than CUs where k ends inside 128 (79 groups of 16 tiles x 5 row blocks), and
+    its split merge (9 groups x 8 row blocks x 2 splits)."""
+    w = make(torch, lib, n, k, n + m)
+    wr = repack(torch, lib, w, n, k)
+    x = np.random.default_rng(n + m).normal(0, 1, (m, k)).astype(np.float16)
+    want = _product64(w, n, k, x)
+    assert np.abs(want[-1:] - orc.q8_gemv_f64(w.cpu().numpy(), n, k, x[-1:].view(np.uint16))).max() < 1e-9
+    rms = np.sqrt((want ** 2).mean())
+    for fn, at in ((lib.aotx_q8_gemv, w), (lib.aotx_q8r_gemv, wr)):
+        y = torch.full((m, n), 7.0, dtype=torch.float32, device="cuda")
+        assert fn(p(at), n, k, p(dev(x, torch)), m, p(y), None) == 0
+        torch.cuda.synchronize()
+        assert np.abs(y.cpu().numpy() - want).max() < 1e-5 * max(rms, 1.0) * np.sqrt(k / 32.0)
