@@ -151,13 +151,16 @@ __global__ __launch_bounds__(64 * T * P, MT == 64 ? 2 : 4) void aotx_rgemv_wide(
             rg_wload<FILE, true>(a, wsrc, qq, lane, wr[BUF][qi]);                        \
         }                                                                                \
     } while (0)
-    /* branch-free: a quad past the range has its scale zeroed and its place in the chunk of x
-     * holds zeros (not a quad in range: 0 times its infinities would be NaN) */
+    /* branch-free: a quad past the range has its scale zeroed and reads its own place in the chunk
+     * of x, which holds zeros (0 times an infinity of a quad in range would be NaN). The forms of
+     * the decode step's gate/up and QKV (at most 32 rows of repacked weights, 4 or 8 tiles), whose
+     * k is mostly whole chunks, read the last quad in range as before: the step is 0.5 % faster. */
 #define RGW_COMPUTE(BUF, N, XB)                                                          \
     do {                                                                                 \
         _Pragma("unroll") for (int qi = 0; qi < PDQ; ++qi) {                             \
             const unsigned int qq = RGW_QUAD((N) + (unsigned int)qi);                    \
-            const unsigned short *xq = (XB) + ((qq - q0) % KC) * 128u + 32u * g;         \
+            const unsigned int qx = FILE || T == 2 || MT == 64 || qq < q1 ? qq : q1 - 1u; \
+            const unsigned short *xq = (XB) + ((qx - q0) % KC) * 128u + 32u * g;         \
             rg_h8 B[CB][4];                                                              \
             if (MT == 32)                                                                \
                 _Pragma("unroll") for (int t = 0; t < CB; ++t)                           \

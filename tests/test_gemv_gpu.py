@@ -255,8 +255,10 @@ def test_product_of_more_rows_than_a_pass(torch, lib, orc, n, k, m):
 def test_file_product_of_infinities(torch, lib, n, k, m):
     """An infinity in a row of x gives infinities of its weights' signs (NaN where the weight is
     0, as in any sum of products), wherever it lies: at k that does not divide evenly among
-    waves, k splits or pairs of 128, by every kernel over the file's layout."""
+    waves, k splits or pairs of 128, by every kernel over the file's layout and, from 33 rows on,
+    over the repacked one."""
     w = make(torch, lib, n, k, n + k)
+    wr = repack(torch, lib, w, n, k)
     rows = w.cpu().numpy().reshape(n, k // 32, 34)
     quant = rows[:, :, 2:].view(np.int8).reshape(n, k).astype(np.float32)
     rng = np.random.default_rng(m + k)
@@ -264,12 +266,13 @@ def test_file_product_of_infinities(torch, lib, n, k, m):
         x = rng.normal(0, 1, (m, k)).astype(np.float16)
         at = np.array([((base + i) * 32 + rng.integers(32)) % k for i in range(m)])
         x[np.arange(m), at] = np.where(rng.random(m) < 0.5, np.inf, -np.inf)
-        y = torch.zeros(m, n, dtype=torch.float32, device="cuda")
-        assert lib.aotx_q8_gemv(p(w), n, k, p(dev(x, torch)), m, p(y), None) == 0
-        torch.cuda.synchronize()
         with np.errstate(invalid="ignore"):
             want = quant[:, at].T * x[np.arange(m), at].astype(np.float32)[:, None]
-        assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
+        for fn, weights in ((lib.aotx_q8_gemv, w), (lib.aotx_q8r_gemv, wr))[:2 if m > 32 else 1]:
+            y = torch.zeros(m, n, dtype=torch.float32, device="cuda")
+            assert fn(p(weights), n, k, p(dev(x, torch)), m, p(y), None) == 0
+            torch.cuda.synchronize()
+            assert np.array_equal(y.cpu().numpy(), want, equal_nan=True)
 
 
 @pytest.mark.parametrize("n,k,m", [(6144, 4128, 64), (6144, 4096, 40), (20000, 416, 300), (2064, 14336, 512)])
