@@ -78,7 +78,7 @@ def _ffn_oracle(orc, gate, up, down, E, H, F, x, prob, ids):
 
 
 # (16, 16, 300): 4800 routed slots, grouped in two chunks
-@pytest.mark.parametrize("E,used,tokens", [(8, 2, 64), (4, 2, 5), (8, 2, 1), (16, 16, 300)])
+@pytest.mark.parametrize("E,used,tokens", [(8, 2, 64), (4, 2, 5), (8, 2, 1), (16, 4, 3), (16, 16, 300)])
 def test_expert_ffn_vs_oracle(torch, lib, orc, E, used, tokens):
     rng = np.random.default_rng(E + tokens)
     H, F = 256, 512
